@@ -26,15 +26,8 @@ namespace vkgv {
 uint32_t hiz_tile_levels(const PyramidDesc& pd);
 }
 
-// Scratch of vkgv_view_aa_image_noalloc: the per-pixel material indices of
-// the image pass, for views of at most kNoAllocPixels pixels (4K UHD, 33 MB).
-// Each GPU the library runs on holds its own copy until the process ends.
-// The pass's first kernel writes all W*H entries it later reads, so nothing
-// needs clearing between calls.  Host code never uses the array's name as an
-// address: vkgv_create resolves the device address with hipGetSymbolAddress
-// (per context, with the context's device current).
+// Largest view of vkgv_view_aa_image_noalloc (4K UHD).
 constexpr size_t kNoAllocPixels = 3840u * 2160u;
-static __device__ __align__(256) uint32_t scratch[kNoAllocPixels];
 
 namespace {
 
@@ -87,8 +80,6 @@ struct vkgv_ctx {
     // is set at vkgv_create, the context's first n device allocations succeed and
     // every later one fails with VKGV_ERROR_OUT_OF_MEMORY (-1: off).
     int64_t fault_alloc_after = -1;
-    // device address of `scratch` on this context's device
-    uint32_t* noalloc_scratch = nullptr;
 };
 
 struct vkgv_view {
@@ -98,7 +89,6 @@ struct vkgv_view {
     DevBuf keys_b, counters_b;       // the second key buffer and counters (frames alternate between them)
     DevBuf setups, tri_cache, slot_albedo, slot_mat, draw_slot, big_chunk, chunk_tri, redo;
     DevBuf frag_stage, frag_jobs;    // deferred fragment runs of heavy meshlets
-    DevBuf aa_mat;                   // per-pixel material indices of the differentiable frame (allocated on first use)
     DevBuf mvp_tab;                  // per-frame VP M table, kMvpStride floats per transform
     DevBuf pmvp_tab, motion;         // prevVP * previous M table and W*H motion vectors (allocated on first use)
     uint32_t list_capacity = 0;
@@ -532,15 +522,6 @@ int vkgv_create(const vkgv_create_info* info, vkgv_ctx** out)
     if (hipGetDeviceProperties(&prop, c->device) == hipSuccess && prop.multiProcessorCount > 0)
         c->cus = prop.multiProcessorCount;
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) { delete c; return VKGV_ERROR_HIP; }
-    {
-        // this device's copy of the no-alloc scratch (the device is current)
-        void* sp = nullptr;
-        if (hipGetSymbolAddress(&sp, HIP_SYMBOL(scratch)) != hipSuccess || !sp) {
-            vkgv_destroy(c);
-            return VKGV_ERROR_HIP;
-        }
-        c->noalloc_scratch = static_cast<uint32_t*>(sp);
-    }
     SrgbTables tab;
     std::memset(&tab, 0, sizeof tab);
     srgb_thresholds(tab.thr);
@@ -1278,7 +1259,7 @@ void vkgv_view_destroy(vkgv_view* v)
                        &v->history, &v->counters, &v->big,
                        &v->clipq, &v->bin_count, &v->bins, &v->setups, &v->tri_cache,
                        &v->slot_albedo, &v->slot_mat, &v->draw_slot, &v->big_chunk, &v->chunk_tri, &v->maps,
-                       &v->aa_mat, &v->mvp_tab, &v->pmvp_tab, &v->motion, &v->redo, &v->frag_stage, &v->frag_jobs })
+                       &v->mvp_tab, &v->pmvp_tab, &v->motion, &v->redo, &v->frag_stage, &v->frag_jobs })
         dfree(*b);
     for (auto& set : v->ev)
         for (auto& e : set)
@@ -1397,13 +1378,6 @@ int vkgv_view_read_ids_depth(vkgv_ctx* c, vkgv_view* v, uint32_t* ids, float* de
     return VKGV_OK;
 }
 
-static int ensure_aa_mat(vkgv_ctx* c, vkgv_view* v)
-{
-    if (v->aa_mat.p) return VKGV_OK;
-    HIP_TRY(c, hipDeviceSynchronize());   // the allocation must not race work of other streams on the buffer list
-    return dalloc(c, v->aa_mat, 4ull * v->dev.width * v->dev.height);
-}
-
 static int check_grad(vkgv_ctx* c, vkgv_view* v, const vkgv_camera* cam, const void* a, const void* b)
 {
     int rc = check_view(c, v);
@@ -1419,9 +1393,7 @@ int vkgv_view_aa_image(vkgv_ctx* c, vkgv_view* v, const vkgv_camera* cam, float*
     if (rc) return rc;
     hipStream_t st = stream ? static_cast<hipStream_t>(stream) : c->stream;
     if (v->last_stream && v->last_stream != st) HIP_TRY(c, hipStreamSynchronize(v->last_stream));
-    if ((rc = ensure_aa_mat(c, v))) return rc;
-    launch_aa_image(scene_dev(c), v->dev.keys, static_cast<uint32_t*>(v->aa_mat.p), v->dev.width, v->dev.height,
-                    cam->view_projection, image, st);
+    launch_aa_image(scene_dev(c), v->dev.keys, v->dev.width, v->dev.height, cam->view_projection, image, st);
     HIP_TRY(c, hipGetLastError());
     return VKGV_OK;
 }
@@ -1433,13 +1405,11 @@ int vkgv_view_aa_image_noalloc(vkgv_ctx* c, vkgv_view* v, const vkgv_camera* cam
     const uint64_t npx = (uint64_t)v->dev.width * v->dev.height;
     if (npx > kNoAllocPixels)
         return fail(c, VKGV_ERROR_LIMIT, "aa_image_noalloc: the view has " + std::to_string(npx)
-                                             + " pixels, the scratch holds at most " + std::to_string(kNoAllocPixels));
-    if (!c->noalloc_scratch) return fail(c, VKGV_ERROR_STATE, "aa_image_noalloc: no scratch address");
+                                             + " pixels, more than the limit of " + std::to_string(kNoAllocPixels));
     HIP_TRY(c, hipSetDevice(c->device));
     hipStream_t st = stream ? static_cast<hipStream_t>(stream) : c->stream;
     if (v->last_stream && v->last_stream != st) HIP_TRY(c, hipStreamSynchronize(v->last_stream));
-    launch_aa_image(scene_dev(c), v->dev.keys, c->noalloc_scratch, v->dev.width, v->dev.height, cam->view_projection,
-                    image, st);
+    launch_aa_image(scene_dev(c), v->dev.keys, v->dev.width, v->dev.height, cam->view_projection, image, st);
     HIP_TRY(c, hipGetLastError());
     return VKGV_OK;
 }
@@ -1453,9 +1423,7 @@ int vkgv_view_aa_backward(vkgv_ctx* c, vkgv_view* v, const vkgv_camera* cam, con
         return fail(c, VKGV_ERROR_INVALID_ARGUMENT, "aa_backward: g_transforms holds fewer transforms than the scene");
     hipStream_t st = stream ? static_cast<hipStream_t>(stream) : c->stream;
     if (v->last_stream && v->last_stream != st) HIP_TRY(c, hipStreamSynchronize(v->last_stream));
-    if ((rc = ensure_aa_mat(c, v))) return rc;
-    launch_aa_backward(scene_dev(c), v->dev.keys, static_cast<uint32_t*>(v->aa_mat.p), v->dev.width, v->dev.height,
-                       cam->view_projection, g_image, g_transforms, st);
+    launch_aa_backward(scene_dev(c), v->dev.keys, v->dev.width, v->dev.height, cam->view_projection, g_image, g_transforms, st);
     HIP_TRY(c, hipGetLastError());
     return VKGV_OK;
 }

@@ -328,7 +328,7 @@ class View:
 
     def aa_image_noalloc(self, camera: N.Camera, out):
         """aa_image through vkgv_view_aa_image_noalloc: the library allocates
-        nothing (its scratch is a fixed per-GPU array); `out` is required."""
+        nothing; `out` is required."""
         import torch
         self._tensor(out, (self.height, self.width, 3), torch.float32, "out")
         self._torch_call(lambda st: self.r._check(
