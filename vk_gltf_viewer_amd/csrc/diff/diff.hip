@@ -32,6 +32,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "diff.hpp"
 
 namespace vkgv_diff {
@@ -152,6 +154,10 @@ template <typename T> struct V2 {
 };
 template <typename T> struct V4 {
     T x, y, z, w;
+};
+// A pair moved by one load or store.
+template <typename T> struct alignas(2 * sizeof(T)) R2 {
+    T x, y;
 };
 
 template <typename T> __device__ __forceinline__ V4<T> load_clip4(const T* clip, const Dims& d, int c, int i, int v)
@@ -312,14 +318,16 @@ __device__ __forceinline__ bool gather_box(const V4<C> P[3], const int vi[3], co
 
 // One thread per (camera, instance, triangle).
 // Also clears vis, the per-triangle flags that the forward's pixel pass sets
-// for the triangles with a gathered pixel.
+// for the triangles with a gathered pixel, and the nflags stray flags.
 template <typename C>
 __global__ __launch_bounds__(kBlock) void tri_boxes_kernel(const C* __restrict__ clip, const int* __restrict__ tris,
                                                             Dims d, unsigned long long* __restrict__ boxes,
-                                                            uint8_t* __restrict__ vis)
+                                                            uint8_t* __restrict__ vis, unsigned* __restrict__ flags,
+                                                            size_t nflags)
 {
     const size_t g = (size_t)blockIdx.x * kBlock + threadIdx.x;
     const size_t n = (size_t)d.C * d.I * d.T;
+    if (g < nflags) flags[g] = 0u;
     if (g >= n) return;
     const int t = (int)(g % d.T);
     const size_t ci = g / d.T;
@@ -344,12 +352,14 @@ __device__ __forceinline__ bool pixel_stray(const unsigned long long* boxes, con
     return !(px >= b.x0 && px <= b.x1 && py >= b.y0 && py <= b.y1);
 }
 
-// One flag per block of kBlock pixels: whether the block holds a stray.
-// Every thread of the block must call it.
-__device__ __forceinline__ void flag_block(bool stray, unsigned* __restrict__ flags)
+// Marks pixel p of an in-range triangle `id` for the backward: its triangle as
+// one with a gathered pixel, or its run of kBlock pixels as one with a stray.
+// Every writer of a flag stores the same value.
+__device__ __forceinline__ void mark_pixel(const unsigned long long* boxes, const Dims& d, int c, int id, int px, int py,
+                                           size_t p, unsigned* __restrict__ flags, uint8_t* __restrict__ vis)
 {
-    const int any = __syncthreads_or(stray ? 1 : 0);
-    if (threadIdx.x == 0) flags[blockIdx.x] = any ? 1u : 0u;
+    if (pixel_stray(boxes, d, c, id, px, py)) flags[p / kBlock] = 1u;
+    else vis[tri_index(d, c, id)] = 1;
 }
 
 // (camera-instance pair, vertex) of a vertex-pass thread; false past the end.
@@ -359,6 +369,12 @@ __device__ __forceinline__ bool gather_thread(const Dims& d, int& ci, int& v)
     ci = (int)(blockIdx.x / nvb);
     v = (int)((blockIdx.x % nvb) * kBlock + threadIdx.x);
     return v < d.V;
+}
+
+// Channel a of the interpolated attributes.
+template <typename R> __device__ __forceinline__ R interp_value(const Bary<R>& b, const R* attr, int A, int a)
+{
+    return (b.lam[0] * attr[b.v[0] * A + a] + b.lam[1] * attr[b.v[1] * A + a]) + b.lam[2] * attr[b.v[2] * A + a];
 }
 
 template <typename C, typename R>
@@ -371,23 +387,17 @@ __global__ __launch_bounds__(kBlock) void interp_fwd_kernel(const C* __restrict_
 {
     const size_t p = (size_t)blockIdx.x * kBlock + threadIdx.x;
     const size_t npx = (size_t)d.C * d.H * d.W;
-    bool stray = false;
-    if (p < npx) {
-        const int id = ids[p];
-        R* o = out + p * A;
-        const int c = (int)(p / ((size_t)d.H * d.W)), py = (int)((p / d.W) % d.H), px = (int)(p % d.W);
-        Bary<R> b;
-        if (!bary_at(clip, tris, d, c, id, px, py, b)) {
-            for (int a = 0; a < A; ++a) o[a] = R(0);
-        } else {
-            for (int a = 0; a < A; ++a)
-                o[a] = (b.lam[0] * attr[b.v[0] * A + a] + b.lam[1] * attr[b.v[1] * A + a])
-                       + b.lam[2] * attr[b.v[2] * A + a];
-            stray = pixel_stray(boxes, d, c, id, px, py);
-            if (!stray) vis[tri_index(d, c, id)] = 1;   // every writer stores the same value
-        }
+    if (p >= npx) return;
+    const int id = ids[p];
+    R* o = out + p * A;
+    const int c = (int)(p / ((size_t)d.H * d.W)), py = (int)((p / d.W) % d.H), px = (int)(p % d.W);
+    Bary<R> b;
+    if (!bary_at(clip, tris, d, c, id, px, py, b)) {
+        for (int a = 0; a < A; ++a) o[a] = R(0);
+        return;
     }
-    flag_block(stray, stray_blocks);
+    for (int a = 0; a < A; ++a) o[a] = interp_value(b, attr, A, a);
+    mark_pixel(boxes, d, c, id, px, py, p, stray_blocks, vis);
 }
 
 // d colour / d attr_k = lambda_k; d colour / d lambda_k = attr_k;
@@ -417,34 +427,37 @@ template <typename C, typename R> struct InterpTerms {
     R gw[3];
 };
 
+// o.b set: the rest, from dL/dlambda.
 template <typename C, typename R>
-__device__ __forceinline__ bool interp_terms(const C* clip, const R* attr, const int* tris, const Dims& d, int A,
-                                             int c, int id, int px, int py, const R* go, InterpTerms<C, R>& o)
+__device__ __forceinline__ void interp_terms_of(const R glam[3], R xn, R yn, InterpTerms<C, R>& o)
 {
-    if (!bary_at(clip, tris, d, c, id, px, py, o.b)) return false;
-    const R xn = ndc_x<R>(px, d), yn = ndc_y<R>(py, d);
-    R glam[3] = { R(0), R(0), R(0) };
-    for (int a = 0; a < A; ++a)
-        for (int k = 0; k < 3; ++k) glam[k] += go[a] * attr[o.b.v[k] * A + a];
     R gl[3];
     lambda_grad(o.b, glam, gl);
     for (int k = 0; k < 3; ++k) {
         o.gu[k] = corner_grad(o.b, gl, k);
         o.gw[k] = -(xn * o.gu[k].x + yn * o.gu[k].y);
     }
+}
+
+template <typename C, typename R>
+__device__ __forceinline__ bool interp_terms(const C* clip, const R* attr, const int* tris, const Dims& d, int A,
+                                             int c, int id, int px, int py, const R* go, InterpTerms<C, R>& o)
+{
+    if (!bary_at(clip, tris, d, c, id, px, py, o.b)) return false;
+    R glam[3] = { R(0), R(0), R(0) };
+    for (int a = 0; a < A; ++a)
+        for (int k = 0; k < 3; ++k) glam[k] += go[a] * attr[o.b.v[k] * A + a];
+    interp_terms_of(glam, ndc_x<R>(px, d), ndc_y<R>(py, d), o);
     return true;
 }
 
-// Pixel pass: contrib[p][k] = (dL/dx, dL/dy, dL/dw, lambda_k g_out[p][0..A-1]),
-// with the antialiasing pass's terms contrib_a[p][k] added to the first three
-// when given (one load per pixel in the vertex pass of the combined backward).
+// Pixel pass: contrib[p][k] = (dL/dx, dL/dy, dL/dw, lambda_k g_out[p][0..A-1]).
 template <typename C, typename R>
 __global__ __launch_bounds__(kBlock) void interp_bwd_pixel_kernel(const C* __restrict__ clip,
                                                                    const R* __restrict__ attr,
                                                                    const int* __restrict__ tris,
                                                                    const int* __restrict__ ids, Dims d, int A,
                                                                    const R* __restrict__ g_out,
-                                                                   const R* __restrict__ contrib_a,
                                                                    R* __restrict__ contrib)
 {
     const size_t p = (size_t)blockIdx.x * kBlock + threadIdx.x;
@@ -454,14 +467,12 @@ __global__ __launch_bounds__(kBlock) void interp_bwd_pixel_kernel(const C* __res
     const R* go = g_out + p * A;
     InterpTerms<C, R> it;
     if (!interp_terms(clip, attr, tris, d, A, c, ids[p], px, py, go, it)) return;
-    R ca[9];
-    for (int k = 0; k < 9; ++k) ca[k] = contrib_a ? contrib_a[p * 9 + k] : R(0);
     R* o = contrib + p * 3 * (3 + A);
     for (int k = 0; k < 3; ++k) {
         R* ok = o + k * (3 + A);
-        ok[0] = it.gu[k].x + ca[3 * k];
-        ok[1] = it.gu[k].y + ca[3 * k + 1];
-        ok[2] = it.gw[k] + ca[3 * k + 2];
+        ok[0] = it.gu[k].x;
+        ok[1] = it.gu[k].y;
+        ok[2] = it.gw[k];
         for (int a = 0; a < A; ++a) ok[3 + a] = it.b.lam[k] * go[a];
     }
 }
@@ -630,51 +641,86 @@ template <typename R> __device__ __forceinline__ R edge_fn(V2<R> a, V2<R> b, V2<
     return (b.x - a.x) * (p.y - a.y) - (b.y - a.y) * (p.x - a.x);
 }
 
-// The blend of a pair whose front pixel (centre at NDC (xc, yc)) holds the
-// triangle with vertices vi and clip positions P of instance i, the back
-// centre at cb from the front one: the first edge of the triangle that the
-// segment from the front centre to the back one leaves through.  Fills every
-// field but f and bpx.
-template <typename C, typename R>
-__device__ __forceinline__ bool front_eval(const V4<C> P[3], const int vi[3], int i, C xc, C yc, V2<R> cb,
-                                           const Dims& d, PairEval<R>& e)
-{
+// The triangle of a front pixel, seen from its centre: screen offsets of the
+// vertices, orientation (interior on the positive side of every edge k, k+1)
+// and the edge functions at the centre.  False for a triangle that blends no
+// pair.  It depends on the pixel alone: the pixel's pairs share it.
+template <typename R> struct FrontTri {
     V2<R> S[3];
+    R sgn, ef[3];
+};
+
+template <typename C, typename R>
+__device__ __forceinline__ bool front_tri(const V4<C> P[3], C xc, C yc, const Dims& d, FrontTri<R>& f)
+{
     for (int k = 0; k < 3; ++k) {
         if (!(P[k].w > C(0))) return false;
-        S[k] = screen_rel<C, R>(P[k], xc, yc, d);
+        f.S[k] = screen_rel<C, R>(P[k], xc, yc, d);
     }
-    // orientation: interior on the positive side of every edge (k, k+1)
-    const R area = edge_fn(S[0], S[1], S[2]);
+    const R area = edge_fn(f.S[0], f.S[1], f.S[2]);
     if (area == R(0)) return false;
-    const R sgn = area > R(0) ? R(1) : R(-1);
+    f.sgn = area > R(0) ? R(1) : R(-1);
     const V2<R> zero{ R(0), R(0) };
-    R best = R(2);
+    for (int k = 0; k < 3; ++k) f.ef[k] = f.sgn * edge_fn(f.S[k], f.S[(k + 1) % 3], zero);
+    return true;
+}
+
+// The first edge of the front triangle that the segment from the front centre
+// to the back one (cb from it) leaves through: its first corner (-1: none),
+// the parameter and the edge function at the back centre.
+template <typename R> __device__ __forceinline__ int front_cross(const FrontTri<R>& f, V2<R> cb, R& t, R& eb)
+{
+    t = R(2);
+    eb = R(0);
     int kb = -1;
-    R bef = R(0), beb = R(0);
     for (int k = 0; k < 3; ++k) {
-        const R ef = sgn * edge_fn(S[k], S[(k + 1) % 3], zero);
-        const R eb = sgn * edge_fn(S[k], S[(k + 1) % 3], cb);
-        if (!(ef >= R(0) && eb <= R(0) && ef > eb)) continue;
-        const R tt = ef / (ef - eb);
-        if (tt < best) { best = tt; kb = k; bef = ef; beb = eb; }
+        const R ebk = f.sgn * edge_fn(f.S[k], f.S[(k + 1) % 3], cb);
+        if (!(f.ef[k] >= R(0) && ebk <= R(0) && f.ef[k] > ebk)) continue;
+        const R tt = f.ef[k] / (f.ef[k] - ebk);
+        if (tt < t) { t = tt; kb = k; eb = ebk; }
     }
+    return kb;
+}
+
+// The k-th of three values, k known only at run time.  Scalars by value: a
+// record picked through its address is placed in scratch memory.
+template <typename T> __device__ __forceinline__ T pick3(T a, T b, T c, int k) { return k == 0 ? a : k == 1 ? b : c; }
+template <typename T> __device__ __forceinline__ T pick3(const T (&x)[3], int k) { return pick3(x[0], x[1], x[2], k); }
+template <typename R> __device__ __forceinline__ V2<R> pick3(const V2<R> (&v)[3], int k)
+{
+    return V2<R>{ pick3(v[0].x, v[1].x, v[2].x, k), pick3(v[0].y, v[1].y, v[2].y, k) };
+}
+// The k-th clip position rounded to R.
+template <typename C, typename R> __device__ __forceinline__ V4<R> pick_clip(const V4<C> (&P)[3], int k)
+{
+    return V4<R>{ pick3(R(P[0].x), R(P[1].x), R(P[2].x), k), pick3(R(P[0].y), R(P[1].y), R(P[2].y), k),
+                  pick3(R(P[0].z), R(P[1].z), R(P[2].z), k), pick3(R(P[0].w), R(P[1].w), R(P[2].w), k) };
+}
+
+// The blend of a pair whose front pixel holds the triangle with vertices vi
+// and clip positions P of instance i: every field of e but f and bpx.
+template <typename C, typename R>
+__device__ __forceinline__ bool front_eval(const V4<C> (&P)[3], const int (&vi)[3], int i, const FrontTri<R>& f, V2<R> cb,
+                                           PairEval<R>& e)
+{
+    R best, beb;
+    const int kb = front_cross(f, cb, best, beb);
     if (kb < 0) return false;
+    const int kn = kb == 2 ? 0 : kb + 1;
     e.cb = cb;
     e.i = i;
     e.t = best;
     e.to_front = best < R(0.5);
     e.alpha = e.to_front ? R(0.5) - best : best - R(0.5);
     e.ka = kb;
-    e.va = vi[kb];
-    e.vb = vi[(kb + 1) % 3];
-    const V4<C> pa = P[kb], pb = P[(kb + 1) % 3];
-    e.pa = V4<R>{ R(pa.x), R(pa.y), R(pa.z), R(pa.w) };
-    e.pb = V4<R>{ R(pb.x), R(pb.y), R(pb.z), R(pb.w) };
-    e.sa = S[kb];
-    e.sb = S[(kb + 1) % 3];
-    e.ef = sgn * bef;      // unsigned-orientation values, re-signed in the backward
-    e.eb = sgn * beb;
+    e.va = pick3(vi, kb);
+    e.vb = pick3(vi, kn);
+    e.pa = pick_clip<C, R>(P, kb);
+    e.pb = pick_clip<C, R>(P, kn);
+    e.sa = pick3(f.S, kb);
+    e.sb = pick3(f.S, kn);
+    e.ef = f.sgn * pick3(f.ef, kb);      // unsigned-orientation values, re-signed in the backward
+    e.eb = f.sgn * beb;
     return true;
 }
 
@@ -713,7 +759,8 @@ __device__ bool pair_eval(const C* clip, const int* tris, const int* ids, const 
     }
     V4<C> P[3];
     for (int k = 0; k < 3; ++k) P[k] = load_clip4(clip, d, c, i, vi[k]);
-    return front_eval<C, R>(P, vi, i, ndc_x<C>(fx, d), ndc_y<C>(fy, d), cb, d, e);
+    FrontTri<R> f;
+    return front_tri<C, R>(P, ndc_x<C>(fx, d), ndc_y<C>(fy, d), d, f) && front_eval<C, R>(P, vi, i, f, cb, e);
 }
 
 // The four pairs of pixel (px, py), as (a, dir) with b the right (dir 0) or
@@ -726,40 +773,153 @@ __device__ __forceinline__ bool pair_of(int q, int px, int py, int& ax, int& ay,
     return ax >= 0 && ay >= 0;
 }
 
-// stray_blocks may be null (the flags and vis come from elsewhere).
-template <typename C, typename R>
-__global__ __launch_bounds__(kBlock) void aa_fwd_kernel(const R* __restrict__ color, const C* __restrict__ clip,
-                                                         const int* __restrict__ tris, const int* __restrict__ ids,
-                                                         const float* __restrict__ depth, Dims d, int A,
-                                                         R* __restrict__ out,
-                                                         const unsigned long long* __restrict__ boxes,
-                                                         unsigned* __restrict__ stray_blocks, uint8_t* __restrict__ vis)
+// ---------------------------------------------------------------------------
+// The pixel passes of the antialiasing.  A block of 32x16 threads takes as
+// many pixels, the outer ring of which only serves its 30x14 inner ones: each
+// thread evaluates the triangle of its pixel once (three vertices, six
+// divisions, in the clip type) and crosses it with the up to four pairs it is
+// the front of; the blends go to LDS, and an inner pixel takes those of its own
+// pairs and of its neighbours'.  (One thread per pixel evaluating all four of
+// its pairs did the triangle work up to four times a pixel, and again for the
+// neighbours that are in front.)  shade's forward also interpolates here and
+// its backward goes on through the interpolation, so that the colour gradient
+// and the edge terms stay in registers.  18 % of the threads are ring.  Bound
+// by the gathers of clip positions and the divisions: 8 views of 512x512 of a
+// 100k-triangle mesh as 8 instances, float64 clip: forward 53 us (interpolation and
+// antialiasing apart: 44 + 118), backward 106 us (107 + 242).
+constexpr int kTileW = 32, kTileH = 16, kTileThreads = kTileW * kTileH;
+constexpr int kInnerW = kTileW - 2, kInnerH = kTileH - 2;
+constexpr int kMaxAttr = 8;
+
+struct TilePixel {
+    int c, x, y;
+    bool in, inner;     // in the image; one of the block's inner pixels
+    size_t p;           // index (0 outside the image)
+};
+
+__device__ __forceinline__ TilePixel tile_pixel(const Dims& d)
 {
-    // gather: pixel p sums the blends of its four pairs that target it
-    const size_t p = (size_t)blockIdx.x * kBlock + threadIdx.x;
-    const size_t npx = (size_t)d.C * d.H * d.W;
-    bool stray = false;
-    if (p < npx) {
-        const int c = (int)(p / ((size_t)d.H * d.W)), py = (int)((p / d.W) % d.H), px = (int)(p % d.W);
-        R acc[8];
-        for (int a = 0; a < A; ++a) acc[a] = color[p * A + a];
-        for (int q = 0; q < 4; ++q) {
-            int ax, ay, dir;
-            if (!pair_of(q, px, py, ax, ay, dir)) continue;
-            PairEval<R> e;
-            if (!pair_eval(clip, tris, ids, depth, d, c, ax, ay, dir, e)) continue;
-            const size_t tgt = e.to_front ? e.f : e.bpx, src = e.to_front ? e.bpx : e.f;
-            if (tgt != p) continue;
-            for (int a = 0; a < A; ++a) acc[a] += e.alpha * (color[src * A + a] - color[tgt * A + a]);
+    const unsigned tw = (unsigned)((d.W + kInnerW - 1) / kInnerW), th = (unsigned)((d.H + kInnerH - 1) / kInnerH);
+    const unsigned col = blockIdx.x % tw, rest = blockIdx.x / tw, row = rest % th;
+    const int tx = (int)threadIdx.x % kTileW, ty = (int)threadIdx.x / kTileW;
+    TilePixel t;
+    t.c = (int)(rest / th);
+    t.x = (int)col * kInnerW + tx - 1;
+    t.y = (int)row * kInnerH + ty - 1;
+    t.in = t.x >= 0 && t.y >= 0 && t.x < d.W && t.y < d.H;
+    t.inner = t.in && tx > 0 && ty > 0 && tx < kTileW - 1 && ty < kTileH - 1;
+    t.p = t.in ? ((size_t)t.c * d.H + t.y) * d.W + t.x : 0;
+    return t;
+}
+
+inline unsigned tile_blocks(const Dims& d)
+{
+    return (unsigned)(((d.W + kInnerW - 1) / kInnerW) * ((d.H + kInnerH - 1) / kInnerH)) * (unsigned)d.C;
+}
+
+// Directions: right, left, down, up (the order a pixel's blends are summed
+// in); q ^ 1 is the opposite one.
+__device__ __forceinline__ int dir_x(int q) { return q == 0 ? 1 : q == 1 ? -1 : 0; }
+__device__ __forceinline__ int dir_y(int q) { return q == 2 ? 1 : q == 3 ? -1 : 0; }
+__device__ __forceinline__ int dir_thread(int q) { return dir_x(q) + kTileW * dir_y(q); }
+
+// A blend in LDS: alpha, the sign telling the target (0 the front pixel, 1
+// the back one), NaN for none.
+__device__ __forceinline__ bool blend_to_back(float v) { return __float_as_uint(v) >> 31; }
+__device__ __forceinline__ bool blend_to_back(double v) { return __double_as_longlong(v) < 0; }
+template <typename R> __device__ __forceinline__ R blend_none() { return R(__builtin_nanf("")); }
+
+// What the pixel passes share: ids (-1 outside the image, 0 background or out
+// of range) and depths of the block's pixels, and the blends of each pixel as
+// the front of its pairs.
+template <typename R> struct TileState {
+    int id[kTileThreads];
+    float depth[kTileThreads];
+    R blend[4][kTileThreads];
+
+    // Whether the pixel of thread t, with id idp > 0, is the front of its
+    // differing pair in direction q.
+    __device__ __forceinline__ bool front(int t, int q, int idp) const
+    {
+        const int n = t + dir_thread(q), idn = id[n];
+        if (idn < 0 || idn == idp) return false;
+        return q & 1 ? !a_is_front(idn, idp, depth[n], depth[t]) : a_is_front(idp, idn, depth[t], depth[n]);
+    }
+};
+
+// NA: the attribute count, 0 for a count only known at run time (at most kMaxAttr).
+#define VKGV_CHANNELS(a) _Pragma("unroll") for (int a = 0; a < (NA ? NA : kMaxAttr); ++a) if (NA || a < A)
+
+// Forward: SHADE interpolates the colour (written to `color`) and marks the
+// pixels for the backward as interp_fwd_kernel does; without it `color` is
+// given.  out = the antialiased colour.
+template <typename C, typename R, bool SHADE, int NA>
+__global__ __launch_bounds__(kTileThreads) void aa_fwd_kernel(R* __restrict__ color, const C* __restrict__ clip,
+                                                               const R* __restrict__ attr,
+                                                               const int* __restrict__ tris, const int* __restrict__ ids,
+                                                               const float* __restrict__ depth, Dims d, int A,
+                                                               R* __restrict__ out,
+                                                               const unsigned long long* __restrict__ boxes,
+                                                               unsigned* __restrict__ stray_blocks,
+                                                               uint8_t* __restrict__ vis)
+{
+    __shared__ TileState<R> s;
+    __shared__ R s_col[NA ? NA : kMaxAttr][kTileThreads];
+    const int t = (int)threadIdx.x;
+    const TilePixel px = tile_pixel(d);
+    const int raw = px.in ? ids[px.p] : 0;
+    const int id = id_in_range(raw, d) ? raw : 0;
+    s.id[t] = px.in ? id : -1;
+    s.depth[t] = px.in ? depth[px.p] : 0.0f;
+    if (!SHADE) {
+        VKGV_CHANNELS(a) s_col[a][t] = px.in ? color[px.p * A + a] : R(0);
+    }
+    int i, tri, vi[3];
+    V4<C> P[3];
+    const bool ok = id > 0 && tri_of(clip, tris, d, px.c, id, i, tri, vi, P);
+    const C xn = ndc_x<C>(px.x, d), yn = ndc_y<C>(px.y, d);
+    if (SHADE) {
+        Bary<R> b;
+        if (ok) {
+            bary_from(P, xn, yn, b);
+            for (int k = 0; k < 3; ++k) b.v[k] = vi[k];
         }
-        for (int a = 0; a < A; ++a) out[p * A + a] = acc[a];
-        if (stray_blocks) {
-            const int id = ids[p];
-            stray = pixel_stray(boxes, d, c, id, px, py);
-            if (id_in_range(id, d) && !stray) vis[tri_index(d, c, id)] = 1;
+        VKGV_CHANNELS(a) {
+            const R v = ok ? interp_value(b, attr, A, a) : R(0);
+            s_col[a][t] = v;
+            if (px.inner) color[px.p * A + a] = v;
         }
     }
-    if (stray_blocks) flag_block(stray, stray_blocks);   // uniform over the grid
+    if (ok && px.inner) mark_pixel(boxes, d, px.c, id, px.x, px.y, px.p, stray_blocks, vis);
+    __syncthreads();
+    FrontTri<R> f;
+    const bool fr = ok && front_tri<C, R>(P, xn, yn, d, f);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        R v = blend_none<R>();
+        // the ring's pairs towards the block's outside have no thread and no use
+        const int nx = t % kTileW + dir_x(q), ny = t / kTileW + dir_y(q);
+        if (fr && nx >= 0 && ny >= 0 && nx < kTileW && ny < kTileH && s.front(t, q, id)) {
+            R tt, eb;
+            if (front_cross(f, V2<R>{ R(dir_x(q)), R(dir_y(q)) }, tt, eb) >= 0)
+                v = tt < R(0.5) ? R(0.5) - tt : -(tt - R(0.5));
+        }
+        s.blend[q][t] = v;
+    }
+    __syncthreads();
+    if (!px.inner) return;
+    R acc[NA ? NA : kMaxAttr];
+    VKGV_CHANNELS(a) acc[a] = s_col[a][t];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int n = t + dir_thread(q);
+        const R own = s.blend[q][t], nb = s.blend[q ^ 1][n];
+        const bool take = (own == own && !blend_to_back(own)) || (nb == nb && blend_to_back(nb));
+        if (!take) continue;
+        const R alpha = own == own ? own : -nb;
+        VKGV_CHANNELS(a) acc[a] += alpha * (s_col[a][n] - s_col[a][t]);
+    }
+    VKGV_CHANNELS(a) out[px.p * A + a] = acc[a];
 }
 
 // One blend's backward.  out_tgt = c_tgt + alpha (c_src - c_tgt):
@@ -819,50 +979,144 @@ __device__ __forceinline__ void add_clip_grad(C* g_clip, const Dims& d, int c, i
     atomicAdd(&g[3], C(gw));
 }
 
-// Pixel pass.  g_color (written): g_out (the identity part) plus the pixel's
-// share of the blends of its four pairs, -alpha g_out[p] where it is the
-// target and alpha g_out[tgt] where it is the source.  contrib[p][k] (for
-// every pixel with an id): dL/d(x, y, w) of corner k of the pixel's triangle
-// from the blends whose front pixel it is, summed over its pairs.
-template <typename C, typename R>
-__global__ __launch_bounds__(kBlock) void aa_bwd_pixel_kernel(const R* __restrict__ color, const C* __restrict__ clip,
-                                                               const int* __restrict__ tris,
-                                                               const int* __restrict__ ids,
-                                                               const float* __restrict__ depth, Dims d, int A,
-                                                               const R* __restrict__ g_out, R* __restrict__ g_color,
-                                                               R* __restrict__ contrib)
+// Pixel pass.  The colour gradient of a pixel is g_out (the identity part)
+// plus its share of the blends of its four pairs, -alpha g_out[p] where it is
+// the target and alpha g_out[tgt] where it is the source.  cg[k] is dL/d(x, y,
+// w) of corner k of the pixel's triangle from the blends whose front pixel it
+// is.  SHADE: the colour gradient goes on through the interpolation, and
+// contrib[p][k] = (its corner terms + cg[k], lambda_k g_color[0..A-1]); g_color
+// is written only where the stray pass reads it.  Without SHADE g_color is
+// written and contrib[p][k] = cg[k], for every pixel with an id.
+template <typename C, typename R, bool SHADE, int NA>
+__global__ __launch_bounds__(kTileThreads) void aa_bwd_pixel_kernel(const R* __restrict__ color,
+                                                                     const C* __restrict__ clip,
+                                                                     const R* __restrict__ attr,
+                                                                     const int* __restrict__ tris,
+                                                                     const int* __restrict__ ids,
+                                                                     const float* __restrict__ depth, Dims d, int A,
+                                                                     const R* __restrict__ g_out,
+                                                                     const unsigned* __restrict__ stray_blocks,
+                                                                     R* __restrict__ g_color, R* __restrict__ contrib)
 {
-    const size_t p = (size_t)blockIdx.x * kBlock + threadIdx.x;
-    const size_t npx = (size_t)d.C * d.H * d.W;
-    if (p >= npx) return;
-    const int c = (int)(p / ((size_t)d.H * d.W)), py = (int)((p / d.W) % d.H), px = (int)(p % d.W);
-    R acc[8];
-    for (int a = 0; a < A; ++a) acc[a] = g_out[p * A + a];
+    __shared__ TileState<R> s;
+    constexpr int kStaged = NA ? NA : 1;   // a run-time channel count reads the neighbours from memory
+    __shared__ R s_col[kStaged][kTileThreads], s_g[kStaged][kTileThreads];
+    const int t = (int)threadIdx.x;
+    const TilePixel px = tile_pixel(d);
+    const int raw = px.in ? ids[px.p] : 0;
+    const int id = id_in_range(raw, d) ? raw : 0;
+    s.id[t] = px.in ? id : -1;
+    s.depth[t] = px.in ? depth[px.p] : 0.0f;
+    if (NA) {
+        VKGV_CHANNELS(a) {
+            s_col[a % kStaged][t] = px.in ? color[px.p * A + a] : R(0);
+            s_g[a % kStaged][t] = px.in ? g_out[px.p * A + a] : R(0);
+        }
+    }
+    int i, tri, vi[3];
+    V4<C> P[3];
+    const bool ok = id > 0 && tri_of(clip, tris, d, px.c, id, i, tri, vi, P);
+    const C xn = ndc_x<C>(px.x, d), yn = ndc_y<C>(px.y, d);
+    __syncthreads();
+    // pixel of direction q's neighbour (in the image wherever a pair exists)
+    auto pixel_at = [&](int q) { return (size_t)((long long)px.p + dir_x(q) + (long long)dir_y(q) * d.W); };
+    auto col_of = [&](int th, size_t p, int a) { return NA ? s_col[a % kStaged][th] : color[p * A + a]; };
+    auto g_of = [&](int th, size_t p, int a) { return NA ? s_g[a % kStaged][th] : g_out[p * A + a]; };
+    FrontTri<R> f;
+    const bool fr = ok && front_tri<C, R>(P, xn, yn, d, f);
     R cg[9];
     for (int k = 0; k < 9; ++k) cg[k] = R(0);
+#pragma unroll
     for (int q = 0; q < 4; ++q) {
-        int ax, ay, dir;
-        if (!pair_of(q, px, py, ax, ay, dir)) continue;
-        PairEval<R> e;
-        if (!pair_eval(clip, tris, ids, depth, d, c, ax, ay, dir, e)) continue;
-        const size_t tgt = e.to_front ? e.f : e.bpx;
-        if (tgt == p)
-            for (int a = 0; a < A; ++a) acc[a] += -e.alpha * g_out[tgt * A + a];
-        else
-            for (int a = 0; a < A; ++a) acc[a] += e.alpha * g_out[tgt * A + a];
-        if (e.f != p) continue;
-        const EdgeGrad<R> g = edge_grad(e, blend_galpha(e, color, g_out, A), d);
-        const int ka = 3 * e.ka, kb = 3 * ((e.ka + 1) % 3);
-        cg[ka] += g.ax;
-        cg[ka + 1] += g.ay;
-        cg[ka + 2] += g.aw;
-        cg[kb] += g.bx;
-        cg[kb + 1] += g.by;
-        cg[kb + 2] += g.bw;
+        R v = blend_none<R>();
+        const int nx = t % kTileW + dir_x(q), ny = t / kTileW + dir_y(q);
+        if (fr && nx >= 0 && ny >= 0 && nx < kTileW && ny < kTileH && s.front(t, q, id)) {
+            PairEval<R> e;
+            if (front_eval<C, R>(P, vi, i, f, V2<R>{ R(dir_x(q)), R(dir_y(q)) }, e)) {
+                v = e.to_front ? e.alpha : -e.alpha;
+                if (px.inner) {
+                    const int n = t + dir_thread(q);
+                    const size_t pn = pixel_at(q);
+                    R galpha = R(0);
+                    VKGV_CHANNELS(a) {
+                        const R ct = e.to_front ? col_of(t, px.p, a) : col_of(n, pn, a);
+                        const R cs = e.to_front ? col_of(n, pn, a) : col_of(t, px.p, a);
+                        galpha += (e.to_front ? g_of(t, px.p, a) : g_of(n, pn, a)) * (cs - ct);
+                    }
+                    const EdgeGrad<R> g = edge_grad(e, galpha, d);
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) {   // corner k is vertex a of the edge, or b, or neither
+                        const bool isa = e.ka == k, isb = (e.ka == 2 ? 0 : e.ka + 1) == k;
+                        if (isa || isb) {
+                            cg[3 * k] += isa ? g.ax : g.bx;
+                            cg[3 * k + 1] += isa ? g.ay : g.by;
+                            cg[3 * k + 2] += isa ? g.aw : g.bw;
+                        }
+                    }
+                }
+            }
+        }
+        s.blend[q][t] = v;
     }
-    for (int a = 0; a < A; ++a) g_color[p * A + a] = acc[a];
-    if (id_in_range(ids[p], d))
-        for (int k = 0; k < 9; ++k) contrib[p * 9 + k] = cg[k];
+    __syncthreads();
+    if (!px.inner) return;
+    R acc[NA ? NA : kMaxAttr];
+    VKGV_CHANNELS(a) acc[a] = g_of(t, px.p, a);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int n = t + dir_thread(q);
+        const R own = s.blend[q][t], nb = s.blend[q ^ 1][n];
+        const bool mine = own == own;
+        if (!mine && !(nb == nb)) continue;
+        const R v = mine ? own : nb, alpha = blend_to_back(v) ? -v : v;
+        const bool target = mine != blend_to_back(v);   // the front pixel of a blend into the front, or the back one's
+        const size_t pn = pixel_at(q);
+        VKGV_CHANNELS(a) acc[a] += target ? -alpha * g_of(t, px.p, a) : alpha * g_of(n, pn, a);
+    }
+    if (!SHADE) {
+        VKGV_CHANNELS(a) g_color[px.p * A + a] = acc[a];
+        if (id > 0)
+            for (int k = 0; k < 9; ++k) contrib[px.p * 9 + k] = cg[k];
+        return;
+    }
+    if (stray_blocks[px.p / kBlock] != 0u) {
+        VKGV_CHANNELS(a) g_color[px.p * A + a] = acc[a];
+    }
+    if (!ok) return;
+    InterpTerms<C, R> it;
+    bary_from(P, xn, yn, it.b);
+    for (int k = 0; k < 3; ++k) it.b.v[k] = vi[k];
+    {
+        const R xr = ndc_x<R>(px.x, d), yr = ndc_y<R>(px.y, d);
+        R glam[3] = { R(0), R(0), R(0) };
+        VKGV_CHANNELS(a) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) glam[k] += acc[a] * attr[vi[k] * A + a];
+        }
+        interp_terms_of(glam, xr, yr, it);
+    }
+    R* o = contrib + px.p * 3 * (3 + A);
+    if (NA == 3) {   // 18 values as pairs (the record is a whole number of them)
+        R v[18];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            v[6 * k] = it.gu[k].x + cg[3 * k];
+            v[6 * k + 1] = it.gu[k].y + cg[3 * k + 1];
+            v[6 * k + 2] = it.gw[k] + cg[3 * k + 2];
+            VKGV_CHANNELS(a) v[6 * k + 3 + a % 3] = it.b.lam[k] * acc[a];
+        }
+#pragma unroll
+        for (int k = 0; k < 9; ++k) reinterpret_cast<R2<R>*>(o)[k] = R2<R>{ v[2 * k], v[2 * k + 1] };
+        return;
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        R* ok3 = o + k * (3 + A);
+        ok3[0] = it.gu[k].x + cg[3 * k];
+        ok3[1] = it.gu[k].y + cg[3 * k + 1];
+        ok3[2] = it.gw[k] + cg[3 * k + 2];
+        VKGV_CHANNELS(a) ok3[3 + a] = it.b.lam[k] * acc[a];
+    }
 }
 
 // The stray pass: the edge terms of the blends whose front pixel is a stray,
@@ -1098,22 +1352,24 @@ static const uint8_t* vis_of(const unsigned long long* boxes, int nc, int I, int
 
 template <typename C>
 static void tri_boxes_t(const C* clip, const int* tris, int nc, int I, int V, int T, int H, int W,
-                        unsigned long long* boxes, hipStream_t st)
+                        unsigned long long* boxes, unsigned* stray_blocks, hipStream_t st)
 {
     const Dims d{ nc, I, V, T, H, W };
-    const size_t n = (size_t)nc * I * T;
-    if (n) tri_boxes_kernel<C><<<blocks(n), kBlock, 0, st>>>(clip, tris, d, boxes, vis_of(boxes, nc, I, T));
+    const size_t nflags = stray_flag_count(nc, H, W), n = std::max((size_t)nc * I * T, nflags);
+    if (n)
+        tri_boxes_kernel<C><<<blocks(n), kBlock, 0, st>>>(clip, tris, d, boxes, vis_of(boxes, nc, I, T), stray_blocks,
+                                                          nflags);
 }
 
 void tri_boxes(const float* clip, const int* tris, int nc, int I, int V, int T, int H, int W,
-               unsigned long long* boxes, hipStream_t st)
+               unsigned long long* boxes, unsigned* stray_blocks, hipStream_t st)
 {
-    tri_boxes_t<float>(clip, tris, nc, I, V, T, H, W, boxes, st);
+    tri_boxes_t<float>(clip, tris, nc, I, V, T, H, W, boxes, stray_blocks, st);
 }
 void tri_boxes(const double* clip, const int* tris, int nc, int I, int V, int T, int H, int W,
-               unsigned long long* boxes, hipStream_t st)
+               unsigned long long* boxes, unsigned* stray_blocks, hipStream_t st)
 {
-    tri_boxes_t<double>(clip, tris, nc, I, V, T, H, W, boxes, st);
+    tri_boxes_t<double>(clip, tris, nc, I, V, T, H, W, boxes, stray_blocks, st);
 }
 
 // Blocks of a vertex pass over (camera-instance pair, vertex).
@@ -1140,7 +1396,7 @@ static void interp_bwd_t(const C* clip, const R* attr, const int* tris, const in
     const size_t npx = (size_t)nc * H * W;
     if (V == 0) return;
     if (npx)
-        interp_bwd_pixel_kernel<C, R><<<blocks(npx), kBlock, 0, st>>>(clip, attr, tris, ids, d, A, g_out, nullptr,
+        interp_bwd_pixel_kernel<C, R><<<blocks(npx), kBlock, 0, st>>>(clip, attr, tris, ids, d, A, g_out,
                                                                       contrib);
     if (nc * I)
         vertex_gather_kernel<C, R, 1><<<gather_blocks(nc, I, V), kBlock, 0, st>>>(
@@ -1151,15 +1407,34 @@ static void interp_bwd_t(const C* clip, const R* attr, const int* tris, const in
                                                                       stray_blocks, g_clip, g_attr);
 }
 
-template <typename C, typename R>
-static void aa_fwd_t(const R* color, const C* clip, const int* tris, const int* ids, const float* depth, int nc, int I,
-                     int V, int T, int H, int W, int A, R* out, unsigned long long* boxes, unsigned* stray_blocks,
-                     hipStream_t st)
+template <typename C, typename R, bool SHADE>
+static void aa_fwd_t(R* color, const C* clip, const R* attr, const int* tris, const int* ids, const float* depth, int nc,
+                     int I, int V, int T, int H, int W, int A, R* out, unsigned long long* boxes,
+                     unsigned* stray_blocks, hipStream_t st)
 {
     const Dims d{ nc, I, V, T, H, W };
     if ((size_t)nc * H * W == 0) return;
-    aa_fwd_kernel<C, R><<<blocks((size_t)nc * H * W), kBlock, 0, st>>>(color, clip, tris, ids, depth, d, A, out, boxes,
-                                                                       stray_blocks, vis_of(boxes, nc, I, T));
+    uint8_t* vis = vis_of(boxes, nc, I, T);
+    if (A == 3)
+        aa_fwd_kernel<C, R, SHADE, 3><<<tile_blocks(d), kTileThreads, 0, st>>>(color, clip, attr, tris, ids, depth, d, A,
+                                                                               out, boxes, stray_blocks, vis);
+    else
+        aa_fwd_kernel<C, R, SHADE, 0><<<tile_blocks(d), kTileThreads, 0, st>>>(color, clip, attr, tris, ids, depth, d, A,
+                                                                               out, boxes, stray_blocks, vis);
+}
+
+template <typename C, typename R, bool SHADE>
+static void aa_bwd_pixel(const R* color, const C* clip, const R* attr, const int* tris, const int* ids,
+                         const float* depth, const Dims& d, int A, const R* g_out, const unsigned* stray_blocks,
+                         R* g_color, R* contrib, hipStream_t st)
+{
+    if ((size_t)d.C * d.H * d.W == 0) return;
+    if (A == 3)
+        aa_bwd_pixel_kernel<C, R, SHADE, 3><<<tile_blocks(d), kTileThreads, 0, st>>>(
+            color, clip, attr, tris, ids, depth, d, A, g_out, stray_blocks, g_color, contrib);
+    else
+        aa_bwd_pixel_kernel<C, R, SHADE, 0><<<tile_blocks(d), kTileThreads, 0, st>>>(
+            color, clip, attr, tris, ids, depth, d, A, g_out, stray_blocks, g_color, contrib);
 }
 
 template <typename C, typename R>
@@ -1170,9 +1445,7 @@ static void aa_bwd_t(const R* color, const C* clip, const int* tris, const int* 
 {
     const Dims d{ nc, I, V, T, H, W };
     const size_t npx = (size_t)nc * H * W;
-    if (npx)
-        aa_bwd_pixel_kernel<C, R><<<blocks(npx), kBlock, 0, st>>>(color, clip, tris, ids, depth, d, A, g_out, g_color,
-                                                                  contrib);
+    aa_bwd_pixel<C, R, false>(color, clip, nullptr, tris, ids, depth, d, A, g_out, stray_blocks, g_color, contrib, st);
     if (V && nc * I)
         vertex_gather_kernel<C, R, 2><<<gather_blocks(nc, I, V), kBlock, 0, st>>>(
             ids, d, A, adj_off, adj, boxes, vis_of(boxes, nc, I, T), nullptr, contrib, g_clip, nullptr);
@@ -1181,29 +1454,22 @@ static void aa_bwd_t(const R* color, const C* clip, const int* tris, const int* 
                                                                   stray_blocks, g_clip);
 }
 
-// antialias(interpolate(...)) as one backward: the antialiasing pixel pass
-// gives the colour gradient and its edge terms, the interpolation pixel pass
-// takes both (adding the edge terms to its own), and one vertex pass sums
-// them into a single g_clip.
+// antialias(interpolate(...)) as one backward: one pixel pass and one vertex
+// pass for both.
 template <typename C, typename R>
 static void shade_bwd_t(const R* color, const C* clip, const R* attr, const int* tris, const int* ids,
                         const float* depth, int nc, int I, int V, int T, int H, int W, int A,
                         const unsigned long long* boxes, const unsigned* stray_blocks, const int* adj_off,
-                        const int* adj, const R* g_out, R* g_color, R* contrib_a, R* contrib_i, R* part, C* g_clip,
-                        R* g_attr, hipStream_t st)
+                        const int* adj, const R* g_out, R* g_color, R* contrib, R* part, C* g_clip, R* g_attr,
+                        hipStream_t st)
 {
     const Dims d{ nc, I, V, T, H, W };
     const size_t npx = (size_t)nc * H * W;
     if (V == 0) return;
-    if (npx) {
-        aa_bwd_pixel_kernel<C, R><<<blocks(npx), kBlock, 0, st>>>(color, clip, tris, ids, depth, d, A, g_out, g_color,
-                                                                  contrib_a);
-        interp_bwd_pixel_kernel<C, R><<<blocks(npx), kBlock, 0, st>>>(clip, attr, tris, ids, d, A, g_color, contrib_a,
-                                                                      contrib_i);
-    }
+    aa_bwd_pixel<C, R, true>(color, clip, attr, tris, ids, depth, d, A, g_out, stray_blocks, g_color, contrib, st);
     if (nc * I)
         vertex_gather_kernel<C, R, 1><<<gather_blocks(nc, I, V), kBlock, 0, st>>>(
-            ids, d, A, adj_off, adj, boxes, vis_of(boxes, nc, I, T), contrib_i, nullptr, g_clip, part);
+            ids, d, A, adj_off, adj, boxes, vis_of(boxes, nc, I, T), contrib, nullptr, g_clip, part);
     attr_reduce_kernel<R><<<blocks((size_t)V * A), kBlock, 0, st>>>(part, nc * I, (size_t)V * A, g_attr);
     if (npx) {
         interp_bwd_stray_kernel<C, R><<<blocks(npx), kBlock, 0, st>>>(clip, attr, tris, ids, d, A, g_color, boxes,
@@ -1264,7 +1530,14 @@ void transform_bwd(const double* g_clip, const double* pos, const double* A, int
                 int V, int T, int H, int W, int A, R* out, unsigned long long* boxes, unsigned* stray_blocks,          \
                 hipStream_t st)                                                                                        \
     {                                                                                                                  \
-        aa_fwd_t<C, R>(color, clip, tris, ids, depth, nc, I, V, T, H, W, A, out, boxes, stray_blocks, st);             \
+        aa_fwd_t<C, R, false>(const_cast<R*>(color), clip, nullptr, tris, ids, depth, nc, I, V, T, H, W, A, out,       \
+                              boxes, stray_blocks, st);                                                                \
+    }                                                                                                                  \
+    void shade_fwd(const C* clip, const R* attr, const int* tris, const int* ids, const float* depth, int nc, int I,   \
+                   int V, int T, int H, int W, int A, R* color, R* out, unsigned long long* boxes,                     \
+                   unsigned* stray_blocks, hipStream_t st)                                                             \
+    {                                                                                                                  \
+        aa_fwd_t<C, R, true>(color, clip, attr, tris, ids, depth, nc, I, V, T, H, W, A, out, boxes, stray_blocks, st); \
     }                                                                                                                  \
     void aa_bwd(const R* color, const C* clip, const int* tris, const int* ids, const float* depth, int nc, int I,     \
                 int V, int T, int H, int W, int A, const unsigned long long* boxes, const unsigned* stray_blocks,      \
@@ -1277,10 +1550,10 @@ void transform_bwd(const double* g_clip, const double* pos, const double* A, int
     void shade_bwd(const R* color, const C* clip, const R* attr, const int* tris, const int* ids, const float* depth,  \
                    int nc, int I, int V, int T, int H, int W, int A, const unsigned long long* boxes,                  \
                    const unsigned* stray_blocks, const int* adj_off, const int* adj, const R* g_out, R* g_color,       \
-                   R* contrib_a, R* contrib_i, R* part, C* g_clip, R* g_attr, hipStream_t st)                          \
+                   R* contrib, R* part, C* g_clip, R* g_attr, hipStream_t st)                                          \
     {                                                                                                                  \
         shade_bwd_t<C, R>(color, clip, attr, tris, ids, depth, nc, I, V, T, H, W, A, boxes, stray_blocks, adj_off,     \
-                          adj, g_out, g_color, contrib_a, contrib_i, part, g_clip, g_attr, st);                        \
+                          adj, g_out, g_color, contrib, part, g_clip, g_attr, st);                                     \
     }
 
 VKGV_DIFF_LAUNCHERS(float, float)

@@ -26,27 +26,28 @@ void mesh_adjacency(const int* tris, int T, int V, int* off, int* adj, hipStream
 // Screen boxes of every (camera, instance, triangle), for the stray flags of
 // the forwards and the gathers of the backwards: tri_boxes_words(nc, I, T)
 // u64 entries (nc * I * T box words, then one flag byte per triangle that the
-// forwards set for the triangles with a gathered pixel).
+// forwards set for the triangles with a gathered pixel).  Also clears the
+// stray flags.
 size_t tri_boxes_words(int nc, int I, int T);
 void tri_boxes(const float* clip, const int* tris, int nc, int I, int V, int T, int H, int W,
-               unsigned long long* boxes, hipStream_t st);
+               unsigned long long* boxes, unsigned* stray_blocks, hipStream_t st);
 void tri_boxes(const double* clip, const int* tris, int nc, int I, int V, int T, int H, int W,
-               unsigned long long* boxes, hipStream_t st);
+               unsigned long long* boxes, unsigned* stray_blocks, hipStream_t st);
 
-// Entries of the per-block stray flags that the forwards write and the
-// backwards read (one per 256 pixels).
+// Entries of the stray flags that the forwards set and the backwards read (one
+// per 256 pixels).
 size_t stray_flag_count(int nc, int H, int W);
 
 // Interpolation and antialiasing.  C is the type of the clip positions and
 // their gradient, R that of attributes, images, their gradients and the
 // arithmetic: (float, float), (double, double) or (double, float).  Depth
 // stays float.  The forwards take the boxes of the same clip positions and
-// write stray_blocks (aa_fwd: unless null); the backwards take them with the
-// adjacency of tris and write every output (g_clip with z = 0).
-// shade_bwd is the backward of aa(interp(...)) in one: g_color is scratch.
-// Scratch: contrib (contrib_i), nc * H * W * 3 * (3 + A) entries for the
-// interpolation and contrib (contrib_a), nc * H * W * 9 for the
-// antialiasing; part, nc * I * V * A entries.
+// the cleared stray flags; the backwards take them with the adjacency of tris
+// and write every output (g_clip with z = 0).  shade_fwd writes both the
+// interpolated colour and the antialiased one.
+// Scratch: contrib, nc * H * W * 3 * (3 + A) entries for interp_bwd and
+// shade_bwd and nc * H * W * 9 for aa_bwd; part, nc * I * V * A entries; the
+// g_color of shade_bwd.
 #define VKGV_DIFF_DECLARE(C, R)                                                                                       \
     void interp_fwd(const C* clip, const R* attr, const int* tris, const int* ids, int nc, int I, int V, int T, int H, \
                     int W, int A, R* out, unsigned long long* boxes, unsigned* stray_blocks, hipStream_t st);          \
@@ -56,6 +57,9 @@ size_t stray_flag_count(int nc, int H, int W);
     void aa_fwd(const R* color, const C* clip, const int* tris, const int* ids, const float* depth, int nc, int I,     \
                 int V, int T, int H, int W, int A, R* out, unsigned long long* boxes, unsigned* stray_blocks,          \
                 hipStream_t st);                                                                                       \
+    void shade_fwd(const C* clip, const R* attr, const int* tris, const int* ids, const float* depth, int nc, int I,   \
+                   int V, int T, int H, int W, int A, R* color, R* out, unsigned long long* boxes,                     \
+                   unsigned* stray_blocks, hipStream_t st);                                                            \
     void aa_bwd(const R* color, const C* clip, const int* tris, const int* ids, const float* depth, int nc, int I,     \
                 int V, int T, int H, int W, int A, const unsigned long long* boxes, const unsigned* stray_blocks,      \
                 const int* adj_off, const int* adj, const R* g_out, R* contrib, R* g_color, C* g_clip,                 \
@@ -63,7 +67,7 @@ size_t stray_flag_count(int nc, int H, int W);
     void shade_bwd(const R* color, const C* clip, const R* attr, const int* tris, const int* ids, const float* depth,  \
                    int nc, int I, int V, int T, int H, int W, int A, const unsigned long long* boxes,                  \
                    const unsigned* stray_blocks, const int* adj_off, const int* adj, const R* g_out, R* g_color,       \
-                   R* contrib_a, R* contrib_i, R* part, C* g_clip, R* g_attr, hipStream_t st);
+                   R* contrib, R* part, C* g_clip, R* g_attr, hipStream_t st);
 
 VKGV_DIFF_DECLARE(float, float)
 VKGV_DIFF_DECLARE(double, double)

@@ -123,15 +123,16 @@ Tensor stray_flags(const Shape& s, const Tensor& like)
     return torch::empty({ (int64_t)vkgv_diff::stray_flag_count(s.C, s.H, s.W) }, like.options().dtype(torch::kInt32));
 }
 
-Tensor tri_boxes(const Tensor& clip, const Tensor& tris, const Shape& s)
+Tensor tri_boxes(const Tensor& clip, const Tensor& tris, const Shape& s, Tensor& flags)
 {
+    auto* f = reinterpret_cast<unsigned*>(flags.data_ptr<int>());
     Tensor boxes = torch::empty({ std::max<int64_t>((int64_t)vkgv_diff::tri_boxes_words(s.C, s.I, s.T), 1) },
                                 clip.options().dtype(torch::kInt64));
     auto* b = reinterpret_cast<unsigned long long*>(boxes.data_ptr<int64_t>());
     if (clip.scalar_type() == torch::kFloat64)
-        vkgv_diff::tri_boxes(clip.data_ptr<double>(), tris.data_ptr<int>(), s.C, s.I, s.V, s.T, s.H, s.W, b, stream());
+        vkgv_diff::tri_boxes(clip.data_ptr<double>(), tris.data_ptr<int>(), s.C, s.I, s.V, s.T, s.H, s.W, b, f, stream());
     else
-        vkgv_diff::tri_boxes(clip.data_ptr<float>(), tris.data_ptr<int>(), s.C, s.I, s.V, s.T, s.H, s.W, b, stream());
+        vkgv_diff::tri_boxes(clip.data_ptr<float>(), tris.data_ptr<int>(), s.C, s.I, s.V, s.T, s.H, s.W, b, f, stream());
     return boxes;
 }
 
@@ -154,7 +155,7 @@ struct InterpolateFn : public torch::autograd::Function<InterpolateFn> {
         check_real(attr, "attr", clip);
         TORCH_CHECK(attr.dim() == 2 && attr.size(0) == clip.size(2), "attr must be [V, A]");
         Tensor out = torch::empty({ s.C, s.H, s.W, s.A }, attr.options());
-        Tensor flags = stray_flags(s, ids), boxes = tri_boxes(clip, tris, s);
+        Tensor flags = stray_flags(s, ids), boxes = tri_boxes(clip, tris, s, flags);
         dispatch_real(clip, attr, [&](auto cc, auto r) {
             using C = decltype(cc);
             using R = decltype(r);
@@ -200,7 +201,7 @@ struct AntialiasFn : public torch::autograd::Function<AntialiasFn> {
                     "color must be [C, H, W, A]");
         TORCH_CHECK(depth.sizes() == ids.sizes(), "depth must match ids");
         Tensor out = torch::empty_like(color);
-        Tensor flags = stray_flags(s, ids), boxes = tri_boxes(clip, tris, s);
+        Tensor flags = stray_flags(s, ids), boxes = tri_boxes(clip, tris, s, flags);
         dispatch_real(clip, color, [&](auto cc, auto r) {
             using C = decltype(cc);
             using R = decltype(r);
@@ -248,16 +249,14 @@ struct ShadeFn : public torch::autograd::Function<ShadeFn> {
         TORCH_CHECK(depth.sizes() == ids.sizes(), "depth must match ids");
         Tensor color = torch::empty({ s.C, s.H, s.W, s.A }, attr.options());
         Tensor out = torch::empty_like(color);
-        Tensor flags = stray_flags(s, ids), boxes = tri_boxes(clip, tris, s);
+        Tensor flags = stray_flags(s, ids), boxes = tri_boxes(clip, tris, s, flags);
         dispatch_real(clip, attr, [&](auto cc, auto r) {
             using C = decltype(cc);
             using R = decltype(r);
-            vkgv_diff::interp_fwd(clip.data_ptr<C>(), attr.data_ptr<R>(), tris.data_ptr<int>(), ids.data_ptr<int>(), s.C,
-                                  s.I, s.V, s.T, s.H, s.W, s.A, color.data_ptr<R>(), box_ptr(boxes),
-                                  reinterpret_cast<unsigned*>(flags.data_ptr<int>()), stream());
-            vkgv_diff::aa_fwd(color.data_ptr<R>(), clip.data_ptr<C>(), tris.data_ptr<int>(), ids.data_ptr<int>(),
-                              depth.data_ptr<float>(), s.C, s.I, s.V, s.T, s.H, s.W, s.A, out.data_ptr<R>(),
-                              box_ptr(boxes), nullptr, stream());
+            vkgv_diff::shade_fwd(clip.data_ptr<C>(), attr.data_ptr<R>(), tris.data_ptr<int>(), ids.data_ptr<int>(),
+                                 depth.data_ptr<float>(), s.C, s.I, s.V, s.T, s.H, s.W, s.A, color.data_ptr<R>(),
+                                 out.data_ptr<R>(), box_ptr(boxes), reinterpret_cast<unsigned*>(flags.data_ptr<int>()),
+                                 stream());
         });
         ctx->save_for_backward({ clip, attr, tris, ids, depth, color, flags, boxes });
         return out;
@@ -273,8 +272,7 @@ struct ShadeFn : public torch::autograd::Function<ShadeFn> {
         Tensor g_clip = torch::empty_like(clip), g_attr = torch::empty_like(attr), g_color = torch::empty_like(color);
         const int64_t npx = (int64_t)s.C * s.H * s.W;
         Tensor part = torch::empty({ std::max<int64_t>((int64_t)s.C * s.I * s.V * s.A, 1) }, attr.options());
-        Tensor contrib_i = torch::empty({ std::max<int64_t>(npx * 3 * (3 + s.A), 1) }, attr.options());
-        Tensor contrib_a = torch::empty({ std::max<int64_t>(npx * 9, 1) }, attr.options());
+        Tensor contrib = torch::empty({ std::max<int64_t>(npx * 3 * (3 + s.A), 1) }, attr.options());
         const auto adj = adjacency(tris, s.V);
         dispatch_real(clip, attr, [&](auto cc, auto r) {
             using C = decltype(cc);
@@ -282,9 +280,8 @@ struct ShadeFn : public torch::autograd::Function<ShadeFn> {
             vkgv_diff::shade_bwd(color.data_ptr<R>(), clip.data_ptr<C>(), attr.data_ptr<R>(), tris.data_ptr<int>(),
                                  ids.data_ptr<int>(), depth.data_ptr<float>(), s.C, s.I, s.V, s.T, s.H, s.W, s.A,
                                  box_ptr(boxes), flag_ptr(flags), adj.first.data_ptr<int>(), adj.second.data_ptr<int>(),
-                                 g_out.data_ptr<R>(), g_color.data_ptr<R>(), contrib_a.data_ptr<R>(),
-                                 contrib_i.data_ptr<R>(), part.data_ptr<R>(), g_clip.data_ptr<C>(),
-                                 g_attr.data_ptr<R>(), stream());
+                                 g_out.data_ptr<R>(), g_color.data_ptr<R>(), contrib.data_ptr<R>(),
+                                 part.data_ptr<R>(), g_clip.data_ptr<C>(), g_attr.data_ptr<R>(), stream());
         });
         return { g_clip, g_attr, Tensor(), Tensor(), Tensor() };
     }
