@@ -40,6 +40,7 @@ namespace vkgv_diff {
 namespace {
 
 constexpr uint32_t kBlock = 256;
+constexpr int kMaxAttr = 8;
 
 __device__ __forceinline__ uint32_t float_bits(float f) { return __float_as_uint(f); }
 
@@ -48,13 +49,49 @@ __device__ __forceinline__ unsigned long long make_key(float z, uint32_t id)
     return ((unsigned long long)(~float_bits(z + 0.0f)) << 32) | (unsigned long long)(0xFFFFFFFEu - id);
 }
 
+template <typename T> struct V2 {
+    T x, y;
+};
+template <typename T> struct alignas(4 * sizeof(T) > 16 ? 16 : 4 * sizeof(T)) V4 {
+    T x, y, z, w;
+};
+// A pair moved by one load or store.
+template <typename T> struct alignas(2 * sizeof(T)) R2 {
+    T x, y;
+};
+
+// clip = m (p, 1), m row-major.
+template <typename C> __device__ __forceinline__ void transform_vertex(const C* m, const C* p, V4<C>& o)
+{
+    const C x = p[0], y = p[1], z = p[2];
+    o.x = fma(m[0], x, fma(m[1], y, fma(m[2], z, m[3])));
+    o.y = fma(m[4], x, fma(m[5], y, fma(m[6], z, m[7])));
+    o.z = fma(m[8], x, fma(m[9], y, fma(m[10], z, m[11])));
+    o.w = fma(m[12], x, fma(m[13], y, fma(m[14], z, m[15])));
+}
+
 struct Dims {
     int C, I, V, T, H, W;
 };
 
-__device__ __forceinline__ float4 load_clip(const float* clip, const Dims& d, int c, int i, int v)
+struct Box {
+    int x0, x1, y0, y1;
+};
+
+// boxes[(c * I + i) * T + t]: x0 | x1 << 16 | y0 << 32 | y1 << 48, or kNoBox
+// for a triangle that is not gathered (or has a vertex out of range); an
+// empty box (x0 > x1) for one on no pixel.
+constexpr unsigned long long kNoBox = ~0ull;
+
+__device__ __forceinline__ unsigned long long pack_box(const Box& b)
 {
-    return reinterpret_cast<const float4*>(clip)[((size_t)c * d.I + i) * d.V + v];
+    return (unsigned long long)(uint16_t)b.x0 | ((unsigned long long)(uint16_t)b.x1 << 16)
+           | ((unsigned long long)(uint16_t)b.y0 << 32) | ((unsigned long long)(uint16_t)b.y1 << 48);
+}
+
+__device__ __forceinline__ Box unpack_box(unsigned long long v)
+{
+    return Box{ (int)(v & 0xFFFFu), (int)((v >> 16) & 0xFFFFu), (int)((v >> 32) & 0xFFFFu), (int)(v >> 48) };
 }
 
 // ---------------------------------------------------------------------------
@@ -62,72 +99,195 @@ __device__ __forceinline__ float4 load_clip(const float* clip, const Dims& d, in
 // exact integer edge functions with a top-left rule, depth plane evaluated at
 // pixel centres, 64-bit atomicMin of (depth, id).  Triangles with a vertex at
 // w <= 0 are skipped (the cameras of this form see the mesh from outside).
-__global__ __launch_bounds__(kBlock) void raster_tris_kernel(const float* __restrict__ clip,
-                                                              const int* __restrict__ tris, Dims d,
-                                                              unsigned long long* __restrict__ keys, int cull_back)
+//
+// The vertices are projected and snapped once each (Snap, 16 bytes), not once
+// for each of the about six triangles that share one: the triangle pass then
+// has no division until a triangle's box holds a pixel centre, and its
+// coordinates are 32-bit (below 2^28), its edge functions 64-bit.  A box of more than kWaveBox pixels is walked by
+// the whole wave.  Bound by the vector ALU (36.9M instructions) and the
+// atomics of every front and back fragment: 6.5M triangles of about half a
+// pixel in 8 views of 512x512 take 130 us; with a projection per triangle
+// corner 147 us, besides the pass that rounded the clip positions to float.
+// (Reading the key first and skipping the atomic of a hidden fragment puts a
+// load's latency in the pixel loop: 223 us.)
+struct alignas(16) Snap {
+    int x, y;       // 1/256 pixel
+    float z;        // z / w
+    int ok;         // 0: w <= 0 or beyond the guard band, no triangle of this vertex is drawn
+};
+constexpr int kWaveBox = 64;
+
+__device__ __forceinline__ Snap snap_vertex(float4 p, const Dims& d)
 {
-    const long long g = (long long)blockIdx.x * kBlock + threadIdx.x;
-    const long long per_cam = (long long)d.I * d.T;
-    if (g >= per_cam * d.C) return;
-    const int c = (int)(g / per_cam);
-    const int i = (int)((g % per_cam) / d.T);
-    const int t = (int)(g % d.T);
     const float hw = (float)d.W * 0.5f, hh = (float)d.H * 0.5f;
-    long long X[3], Y[3];
-    float Z[3];
-    for (int k = 0; k < 3; ++k) {
-        const float4 p = load_clip(clip, d, c, i, tris[3 * t + k]);
-        if (!(p.w > 0.0f)) return;
-        const float xf = hw * (p.x / p.w) + hw, yf = hh * (p.y / p.w) + hh;
-        if (!(fabsf(xf) < 1048576.0f && fabsf(yf) < 1048576.0f)) return;
-        X[k] = (long long)rintf(xf * 256.0f);
-        Y[k] = (long long)rintf(yf * 256.0f);
-        Z[k] = p.z / p.w;
+    Snap s{ 0, 0, 0.0f, 0 };
+    if (!(p.w > 0.0f)) return s;
+    const float xf = hw * (p.x / p.w) + hw, yf = hh * (p.y / p.w) + hh;
+    if (!(fabsf(xf) < 1048576.0f && fabsf(yf) < 1048576.0f)) return s;
+    s.x = (int)rintf(xf * 256.0f);
+    s.y = (int)rintf(yf * 256.0f);
+    s.z = p.z / p.w;
+    s.ok = 1;
+    return s;
+}
+
+// The start of render: clip[ci, v] = M[ci] (p_v, 1), its snapped vertex (of the
+// position rounded to float), and the buffers of the passes that follow
+// cleared: npx keys and nvis words of flags, spread over the grid.
+template <typename C>
+__global__ __launch_bounds__(kBlock) void project_kernel(const C* __restrict__ pos, const C* __restrict__ M, Dims d,
+                                                          C* __restrict__ clip, Snap* __restrict__ snap,
+                                                          unsigned long long* __restrict__ keys, size_t npx,
+                                                          uint32_t* __restrict__ vis, size_t nvis)
+{
+    const size_t g = ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * kBlock + threadIdx.x;
+    const size_t n = (size_t)gridDim.x * gridDim.y * kBlock;
+    for (size_t k = g; k < npx; k += n) keys[k] = ~0ull;
+    for (size_t k = g; k < nvis; k += n) vis[k] = 0u;
+    const int v = (int)(blockIdx.x * kBlock + threadIdx.x);
+    const size_t ci = blockIdx.y;
+    if (v >= d.V || ci >= (size_t)d.C * d.I) return;
+    V4<C> o;
+    transform_vertex(M + ci * 16, pos + 3 * (size_t)v, o);
+    reinterpret_cast<V4<C>*>(clip)[ci * d.V + v] = o;
+    snap[ci * d.V + v] = snap_vertex(make_float4((float)o.x, (float)o.y, (float)o.z, (float)o.w), d);
+}
+
+// Snapped vertices of given clip positions.
+__global__ __launch_bounds__(kBlock) void snap_kernel(const float* __restrict__ clip, Dims d, size_t n,
+                                                       Snap* __restrict__ snap)
+{
+    const size_t g = (size_t)blockIdx.x * kBlock + threadIdx.x;
+    if (g < n) snap[g] = snap_vertex(reinterpret_cast<const float4*>(clip)[g], d);
+}
+
+// A triangle ready to be walked over its box of pixels: edge functions at the
+// first centre minus the top-left bias (a centre is covered iff all are >= 0),
+// the depth plane from vertex 0.
+struct TriWalk {
+    long long e[3];
+    int ex[3], ey[3];   // a pixel to the right adds -256 ey, a row down 256 ex
+    float z0, za, zb;
+    int ox, oy;         // first centre from vertex 0, 1/256 pixel
+    int px0, px1, py0, py1;
+    uint32_t id;
+
+    // Visibility-buffer key of pixel (i, j) of the box; all ones where the
+    // centre is not covered.
+    __device__ __forceinline__ unsigned long long key_at(int i, int j) const
+    {
+        long long c = 0;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) c |= e[k] + (((long long)j * ex[k] - (long long)i * ey[k]) << 8);
+        const float z = z0 + (za * ((float)(ox + 256 * i) * 0.00390625f) + zb * ((float)(oy + 256 * j) * 0.00390625f));
+        return c >= 0 && z >= 0.0f && z <= 1.0f ? make_key(z, id) : ~0ull;
     }
-    long long area = (X[1] - X[0]) * (Y[2] - Y[0]) - (Y[1] - Y[0]) * (X[2] - X[0]);
-    if (area == 0) return;
-    if (cull_back && area > 0) return;   // keep the winding the frame's back-face test keeps
-    if (area < 0) {
-        long long tx = X[1]; X[1] = X[2]; X[2] = tx;
-        tx = Y[1]; Y[1] = Y[2]; Y[2] = tx;
-        const float tz = Z[1]; Z[1] = Z[2]; Z[2] = tz;
-        area = -area;
-    }
-    long long mnx = min(X[0], min(X[1], X[2])), mxx = max(X[0], max(X[1], X[2]));
-    long long mny = min(Y[0], min(Y[1], Y[2])), mxy = max(Y[0], max(Y[1], Y[2]));
-    const int px0 = (int)max((mnx - 128 + 255) >> 8, 0LL), px1 = (int)min((mxx - 128) >> 8, (long long)d.W - 1);
-    const int py0 = (int)max((mny - 128 + 255) >> 8, 0LL), py1 = (int)min((mxy - 128) >> 8, (long long)d.H - 1);
-    if (px0 > px1 || py0 > py1) return;
-    long long ex[3], ey[3], ax[3], ay[3];
-    bool tl[3];
-    for (int k = 0; k < 3; ++k) {
-        const int ka = (k + 1) % 3, kb = (k + 2) % 3;
-        ex[k] = X[kb] - X[ka]; ey[k] = Y[kb] - Y[ka]; ax[k] = X[ka]; ay[k] = Y[ka];
-        tl[k] = ey[k] < 0 || (ey[k] == 0 && ex[k] > 0);
-    }
-    const double e1x = (double)(X[1] - X[0]) / 256.0, e1y = (double)(Y[1] - Y[0]) / 256.0;
-    const double e2x = (double)(X[2] - X[0]) / 256.0, e2y = (double)(Y[2] - Y[0]) / 256.0;
-    const double dz1 = (double)Z[1] - (double)Z[0], dz2 = (double)Z[2] - (double)Z[0];
-    const double det = (double)area / 65536.0;
-    const float za = (float)((dz1 * e2y - dz2 * e1y) / det), zb = (float)((dz2 * e1x - dz1 * e2x) / det);
-    const uint32_t id = (uint32_t)(i * d.T + t + 1);
-    unsigned long long* img = keys + (size_t)c * d.H * d.W;
-    for (int py = py0; py <= py1; ++py) {
-        const long long sy = (long long)py * 256 + 128;
-        for (int px = px0; px <= px1; ++px) {
-            const long long sx = (long long)px * 256 + 128;
-            bool in = true;
-            for (int k = 0; k < 3; ++k) {
-                const long long e = ex[k] * (sy - ay[k]) - ey[k] * (sx - ax[k]);
-                in = in && (e > 0 || (e == 0 && tl[k]));
+};
+
+__device__ __forceinline__ void key_min(unsigned long long* p, unsigned long long key)
+{
+    (void)__hip_atomic_fetch_min(p, key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// boxes (may be null): the pixel box of each triangle with a fragment.
+__global__ __launch_bounds__(kBlock) void raster_tris_kernel(const Snap* __restrict__ snap, const int* __restrict__ tris,
+                                                              Dims d, unsigned long long* __restrict__ keys,
+                                                              unsigned long long* __restrict__ boxes, int cull_back)
+{
+    const int t = (int)(blockIdx.x * kBlock + threadIdx.x), lane = (int)(threadIdx.x & 63u);
+    for (int ci = (int)blockIdx.y; ci < d.C * d.I; ci += (int)gridDim.y) {
+        const Snap* sv = snap + (size_t)ci * d.V;
+        unsigned long long* img = keys + (size_t)(ci / d.I) * d.H * d.W;
+        TriWalk w;
+        bool live = false;
+        if (t < d.T) {
+            const Snap a = sv[tris[3 * t]], b = sv[tris[3 * t + 1]], c = sv[tris[3 * t + 2]];
+            w.px0 = max((min(a.x, min(b.x, c.x)) + 127) >> 8, 0);
+            w.px1 = min((max(a.x, max(b.x, c.x)) - 128) >> 8, d.W - 1);
+            w.py0 = max((min(a.y, min(b.y, c.y)) + 127) >> 8, 0);
+            w.py1 = min((max(a.y, max(b.y, c.y)) - 128) >> 8, d.H - 1);
+            live = a.ok & b.ok & c.ok && w.px0 <= w.px1 && w.py0 <= w.py1;
+            if (live) {
+                long long area = (long long)(b.x - a.x) * (c.y - a.y) - (long long)(b.y - a.y) * (c.x - a.x);
+                live = area != 0 && !(cull_back && area > 0);   // the winding the frame's back-face test keeps
+                if (live) {
+                    const bool flip = area < 0;
+                    if (flip) area = -area;
+                    const Snap p = flip ? c : b, q = flip ? b : c;
+                    const int X[3] = { a.x, p.x, q.x }, Y[3] = { a.y, p.y, q.y };
+                    const int sx = w.px0 * 256 + 128, sy = w.py0 * 256 + 128;
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) {
+                        const int ka = (k + 1) % 3, kb = (k + 2) % 3;
+                        const int ex = X[kb] - X[ka], ey = Y[kb] - Y[ka];
+                        const bool tl = ey < 0 || (ey == 0 && ex > 0);
+                        w.e[k] = (long long)ex * (sy - Y[ka]) - (long long)ey * (sx - X[ka]) - (tl ? 0 : 1);
+                        w.ex[k] = ex;
+                        w.ey[k] = ey;
+                    }
+                    w.ox = sx - a.x;
+                    w.oy = sy - a.y;
+                    const double e1x = (double)(p.x - a.x) / 256.0, e1y = (double)(p.y - a.y) / 256.0;
+                    const double e2x = (double)(q.x - a.x) / 256.0, e2y = (double)(q.y - a.y) / 256.0;
+                    const double dz1 = (double)p.z - (double)a.z, dz2 = (double)q.z - (double)a.z;
+                    const double det = (double)area / 65536.0;
+                    w.z0 = a.z;
+                    w.za = (float)((dz1 * e2y - dz2 * e1y) / det);
+                    w.zb = (float)((dz2 * e1x - dz1 * e2x) / det);
+                    w.id = (uint32_t)((ci % d.I) * d.T + t + 1);
+                }
             }
-            if (!in) continue;
-            const float z = Z[0] + (za * ((float)(sx - X[0]) * 0.00390625f) + zb * ((float)(sy - Y[0]) * 0.00390625f));
-            if (!(z >= 0.0f && z <= 1.0f)) continue;
-            (void)__hip_atomic_fetch_min(img + (size_t)py * d.W + px, make_key(z, id), __ATOMIC_RELAXED,
-                                         __HIP_MEMORY_SCOPE_AGENT);
         }
+        const bool wide = live && (long long)(w.px1 - w.px0 + 1) * (w.py1 - w.py0 + 1) > kWaveBox;
+        bool drawn = false;
+        if (live && !wide) {
+            unsigned long long* at = img + (size_t)w.py0 * d.W + w.px0;
+            const int bw = w.px1 - w.px0 + 1, n = bw * (w.py1 - w.py0 + 1);
+            for (int q = 0, i = 0, j = 0; q < n; ++q) {
+                const unsigned long long key = w.key_at(i, j);
+                if (key != ~0ull) {
+                    key_min(at + (size_t)j * d.W + i, key);
+                    drawn = true;
+                }
+                if (++i == bw) {
+                    i = 0;
+                    ++j;
+                }
+            }
+        }
+        // one wide triangle at a time, a pixel per lane
+        unsigned long long pending = __ballot(wide);
+        while (pending != 0ull) {
+            const int j = __ffsll((long long)pending) - 1;
+            pending &= pending - 1ull;
+            TriWalk u;
+            constexpr int kWords = (int)(sizeof(TriWalk) / 4);
+            static_assert(sizeof(TriWalk) % 4 == 0, "broadcast word by word");
+            const uint32_t* from = reinterpret_cast<const uint32_t*>(&w);
+            uint32_t* to = reinterpret_cast<uint32_t*>(&u);
+#pragma unroll
+            for (int k = 0; k < kWords; ++k) to[k] = (uint32_t)__builtin_amdgcn_readlane((int)from[k], j);
+            const int bw = u.px1 - u.px0 + 1, n = bw * (u.py1 - u.py0 + 1);
+            bool any = false;
+            for (int q = lane; q < n; q += 64) {
+                const int j2 = q / bw, i2 = q - j2 * bw;
+                const unsigned long long key = u.key_at(i2, j2);
+                if (key == ~0ull) continue;
+                key_min(img + (size_t)(u.py0 + j2) * d.W + u.px0 + i2, key);
+                any = true;
+            }
+            if (__ballot(any) != 0ull && lane == j) drawn = true;
+        }
+        if (boxes && drawn)
+            boxes[(size_t)ci * d.T + t] = pack_box(Box{ w.px0, w.px1, w.py0, w.py1 });
     }
+}
+
+// Id and depth of a key (0 and 0 for a pixel without a triangle).
+__device__ __forceinline__ void key_parts(unsigned long long k, int& id, float& depth)
+{
+    id = k == ~0ull ? 0 : (int)(0xFFFFFFFEu - (uint32_t)k);
+    depth = k == ~0ull ? 0.0f : __uint_as_float(~(uint32_t)(k >> 32));
 }
 
 __global__ __launch_bounds__(kBlock) void keys_to_ids_kernel(const unsigned long long* __restrict__ keys, size_t n,
@@ -135,10 +295,11 @@ __global__ __launch_bounds__(kBlock) void keys_to_ids_kernel(const unsigned long
 {
     const size_t p = (size_t)blockIdx.x * kBlock + threadIdx.x;
     if (p >= n) return;
-    const unsigned long long k = keys[p];
-    if (k == ~0ull) { ids[p] = 0; depth[p] = 0.0f; return; }
-    ids[p] = (int)(0xFFFFFFFEu - (uint32_t)k);
-    depth[p] = __uint_as_float(~(uint32_t)(k >> 32));
+    int id;
+    float dep;
+    key_parts(keys[p], id, dep);
+    ids[p] = id;
+    depth[p] = dep;
 }
 
 // ---------------------------------------------------------------------------
@@ -149,27 +310,9 @@ __global__ __launch_bounds__(kBlock) void keys_to_ids_kernel(const unsigned long
 // are ill-conditioned in (u below, the screen offsets of the antialiasing)
 // are formed in C and then rounded to R.  The raster above always works on
 // float clip positions.
-template <typename T> struct V2 {
-    T x, y;
-};
-template <typename T> struct V4 {
-    T x, y, z, w;
-};
-// A pair moved by one load or store.
-template <typename T> struct alignas(2 * sizeof(T)) R2 {
-    T x, y;
-};
-
 template <typename T> __device__ __forceinline__ V4<T> load_clip4(const T* clip, const Dims& d, int c, int i, int v)
 {
-    const T* p = clip + (((size_t)c * d.I + i) * d.V + v) * 4;
-    return V4<T>{ p[0], p[1], p[2], p[3] };
-}
-
-template <> __device__ __forceinline__ V4<float> load_clip4<float>(const float* clip, const Dims& d, int c, int i, int v)
-{
-    const float4 p = load_clip(clip, d, c, i, v);
-    return V4<float>{ p.x, p.y, p.z, p.w };
+    return reinterpret_cast<const V4<T>*>(clip)[((size_t)c * d.I + i) * d.V + v];
 }
 
 template <typename T> __device__ __forceinline__ T cross2(V2<T> a, V2<T> b) { return a.x * b.y - a.y * b.x; }
@@ -238,7 +381,7 @@ __device__ __forceinline__ bool bary_at(const C* clip, const int* tris, const Di
 // Gathers.  The backward of interpolation and antialiasing runs in two
 // passes.  A pixel pass computes, with every lane busy, each pixel's terms
 // for the three corners of its triangle (plain stores, contrib).  A vertex
-// pass, one thread per (camera, instance, vertex), walks the vertex's
+// pass, a few lanes per vertex, walks the vertex's
 // incident triangles (a CSR adjacency of the mesh) and sums the terms of the
 // pixels in each triangle's screen box that carry the triangle's id.  No
 // atomics, and the sums run in a fixed order: the gradients are the same
@@ -253,28 +396,7 @@ __device__ __forceinline__ bool bary_at(const C* clip, const int* tris, const Di
 // scatter those pixels' terms with atomics after the vertex pass, in a pass
 // that skips unflagged blocks.
 constexpr int kGatherMaxBox = 64;
-constexpr int kGatherBatch = 8;   // incident triangles whose boxes are loaded together
 constexpr int kPixBatch = 4;      // box pixels whose ids are loaded together
-
-struct Box {
-    int x0, x1, y0, y1;
-};
-
-// boxes[(c * I + i) * T + t]: x0 | x1 << 16 | y0 << 32 | y1 << 48, or kNoBox
-// for a triangle that is not gathered (or has a vertex out of range); an
-// empty box (x0 > x1) for one on no pixel.
-constexpr unsigned long long kNoBox = ~0ull;
-
-__device__ __forceinline__ unsigned long long pack_box(const Box& b)
-{
-    return (unsigned long long)(uint16_t)b.x0 | ((unsigned long long)(uint16_t)b.x1 << 16)
-           | ((unsigned long long)(uint16_t)b.y0 << 32) | ((unsigned long long)(uint16_t)b.y1 << 48);
-}
-
-__device__ __forceinline__ Box unpack_box(unsigned long long v)
-{
-    return Box{ (int)(v & 0xFFFFu), (int)((v >> 16) & 0xFFFFu), (int)((v >> 32) & 0xFFFFu), (int)(v >> 48) };
-}
 
 // Index of (camera c, the instance and triangle of in-range id) in boxes and vis.
 __device__ __forceinline__ size_t tri_index(const Dims& d, int c, int id)
@@ -360,15 +482,6 @@ __device__ __forceinline__ void mark_pixel(const unsigned long long* boxes, cons
 {
     if (pixel_stray(boxes, d, c, id, px, py)) flags[p / kBlock] = 1u;
     else vis[tri_index(d, c, id)] = 1;
-}
-
-// (camera-instance pair, vertex) of a vertex-pass thread; false past the end.
-__device__ __forceinline__ bool gather_thread(const Dims& d, int& ci, int& v)
-{
-    const unsigned nvb = (unsigned)((d.V + (int)kBlock - 1) / (int)kBlock);
-    ci = (int)(blockIdx.x / nvb);
-    v = (int)((blockIdx.x % nvb) * kBlock + threadIdx.x);
-    return v < d.V;
 }
 
 // Channel a of the interpolated attributes.
@@ -508,92 +621,300 @@ __global__ __launch_bounds__(kBlock) void interp_bwd_stray_kernel(const C* __res
     }
 }
 
-// The vertex pass: g_clip[c, i, v] (written, z = 0) and, with the
-// interpolation terms, this camera-instance pair's attribute gradient
-// part[c, i, v, A] (reduced over the pairs by attr_reduce_kernel).  The
-// interpolation terms are contrib_i[p][k][3 + A], the antialiasing ones
-// contrib_a[p][k][3]; MODE says which are summed (1 or 2).  Triangles
-// without a gathered pixel (vis 0) are skipped.
-template <typename C, typename R, int MODE>
+// The sums of a vertex in one camera-instance pair: dL/d(x, y, w) of its clip
+// position and dL/d its attributes.
+template <typename C, typename R, int NA> struct VertexSum {
+    C x, y, w;
+    R a[NA ? NA : kMaxAttr];
+};
+
+// NA: the attribute count, 0 for a count only known at run time (at most kMaxAttr).
+#define VKGV_CHANNELS(a) _Pragma("unroll") for (int a = 0; a < (NA ? NA : kMaxAttr); ++a) if (NA || a < A)
+
+template <typename C, typename R, int NA>
+__device__ __forceinline__ void sum_clear(VertexSum<C, R, NA>& s)
+{
+    s.x = s.y = s.w = C(0);
+#pragma unroll
+    for (int a = 0; a < (NA ? NA : kMaxAttr); ++a) s.a[a] = R(0);
+}
+
+// The value of lane i's partner, i ^ 1, i ^ 2, the mirror lane of its group of
+// eight, or the lane eight away in its row of 16, by a DPP move: the vector
+// ALU alone (__shfl_xor goes through the LDS crossbar, which bound the vertex
+// pass).
+enum { kXor1 = 0xB1, kXor2 = 0x4E, kMirror8 = 0x141, kRor8 = 0x128 };
+template <int CTRL> __device__ __forceinline__ float lane_move(float x)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, true));
+}
+template <int CTRL> __device__ __forceinline__ double lane_move(double x)
+{
+    const long long b = __double_as_longlong(x);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, 0xF, 0xF, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)((unsigned long long)b >> 32), CTRL, 0xF, 0xF, true);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// The sum over a group of eight lanes, in each of them (every lane of the wave
+// takes part): pairs, then quads, then the two quads.
+template <typename T> __device__ __forceinline__ T sum8(T x)
+{
+    x += lane_move<kXor1>(x);
+    x += lane_move<kXor2>(x);
+    x += lane_move<kMirror8>(x);
+    return x;
+}
+
+template <typename C, typename R, int NA> __device__ __forceinline__ void sum8(VertexSum<C, R, NA>& s, int A)
+{
+    s.x = sum8(s.x);
+    s.y = sum8(s.y);
+    s.w = sum8(s.w);
+    VKGV_CHANNELS(a) s.a[a] = sum8(s.a[a]);
+}
+
+// The sum over the wave, in each lane.
+template <typename T> __device__ __forceinline__ T sum64(T x)
+{
+    x = sum8(x);
+    x += lane_move<kRor8>(x);
+    x += __shfl_xor(x, 16, 64);
+    x += __shfl_xor(x, 32, 64);
+    return x;
+}
+
+// Adds pixel p's record of corner k: contrib[p][k][n], n = 3 + A values with
+// the attributes' (ATTR), 3 without.
+template <typename C, typename R, int NA, bool ATTR>
+__device__ __forceinline__ void add_record(const R* contrib, size_t p, int k, int A, VertexSum<C, R, NA>& s)
+{
+    const R* o = contrib + (p * 3 + k) * (ATTR ? 3 + A : 3);
+    if (ATTR && NA == 3) {   // six values by as few loads as there are: the lanes' records lie apart
+        struct alignas(2 * sizeof(R)) Six {
+            R v[6];
+        };
+        const Six r = *reinterpret_cast<const Six*>(o);
+        s.x += C(r.v[0]);
+        s.y += C(r.v[1]);
+        s.w += C(r.v[2]);
+        s.a[0] += r.v[3];
+        s.a[1 % (NA ? NA : 2)] += r.v[4];
+        s.a[2 % (NA ? NA : 3)] += r.v[5];
+        return;
+    }
+    s.x += C(o[0]);
+    s.y += C(o[1]);
+    s.w += C(o[2]);
+    if (ATTR) {
+        VKGV_CHANNELS(a) s.a[a] += o[3 + a];
+    }
+}
+
+// One lane sums the records of the pixels of box b that carry id, kPixBatch
+// ids at a time in flight.  base: the camera's first pixel.  The triangle has
+// a pixel in the box, so that a box of one needs no look at its id.
+template <typename C, typename R, int NA, bool ATTR>
+__device__ __forceinline__ void walk_box(const int* ids, size_t base, int W, const Box& b, int id, int k,
+                                         const R* contrib, int A, VertexSum<C, R, NA>& s)
+{
+    const int bw = b.x1 - b.x0 + 1, n = bw * (b.y1 - b.y0 + 1);
+    int qx = b.x0, qy = b.y0;
+    if (n == 1) {
+        add_record<C, R, NA, ATTR>(contrib, base + (size_t)qy * W + qx, k, A, s);
+        return;
+    }
+    for (int q0 = 0; q0 < n; q0 += kPixBatch) {
+        size_t ip[kPixBatch];
+        int idq[kPixBatch];
+#pragma unroll
+        for (int w = 0; w < kPixBatch; ++w) {
+            ip[w] = base + (size_t)qy * W + qx;
+            idq[w] = q0 + w < n ? ids[ip[w]] : 0;
+            if (++qx > b.x1) {
+                qx = b.x0;
+                ++qy;
+            }
+        }
+#pragma unroll
+        for (int w = 0; w < kPixBatch; ++w)
+            if (idq[w] == id) add_record<C, R, NA, ATTR>(contrib, ip[w], k, A, s);
+    }
+}
+
+// The wave sums a wide box, a pixel per lane; the total goes to lane j.
+template <typename C, typename R, int NA, bool ATTR>
+__device__ __forceinline__ void walk_wide(const int* ids, size_t base, int W, const Box& b, int id, int k,
+                                          const R* contrib, int A, int j, VertexSum<C, R, NA>& s)
+{
+    const int lane = (int)(threadIdx.x & 63u), bw = b.x1 - b.x0 + 1, n = bw * (b.y1 - b.y0 + 1);
+    VertexSum<C, R, NA> p;
+    sum_clear(p);
+    for (int q = lane; q < n; q += 64) {
+        const size_t ip = base + (size_t)(b.y0 + q / bw) * W + (b.x0 + q % bw);
+        if (ids[ip] == id) add_record<C, R, NA, ATTR>(contrib, ip, k, A, p);
+    }
+    p.x = sum64(p.x);
+    p.y = sum64(p.y);
+    p.w = sum64(p.w);
+    VKGV_CHANNELS(a) p.a[a] = sum64(p.a[a]);
+    if (lane == j) {
+        s.x += p.x;
+        s.y += p.y;
+        s.w += p.w;
+        VKGV_CHANNELS(a) s.a[a] += p.a[a];
+    }
+}
+
+// Vertex passes: kVertexLanes lanes share a vertex, lane u taking incident
+// triangles u, u + kVertexLanes, ... (a mesh vertex has about six), and a
+// triangle without a gathered pixel (vis 0, most of them: hidden, facing away,
+// between the pixel centres) costs one byte.  One lane walking all its
+// triangles ran as long as the longest of 64 such walks.
+constexpr int kVertexLanes = 8;   // sum8's group
+constexpr int kBlockVertices = (int)kBlock / kVertexLanes;
+
+// The vertex pass of interpolate, antialias and shade: g_clip[c, i, v]
+// (written, z = 0) and, with the interpolation terms (ATTR), this
+// camera-instance pair's attribute gradient part[c, i, v, A] (reduced over the
+// pairs by attr_reduce_kernel).  contrib[p][k][n] as in add_record.
+template <typename C, typename R, bool ATTR, int NA>
 __global__ __launch_bounds__(kBlock) void vertex_gather_kernel(const int* __restrict__ ids, Dims d, int A,
                                                                 const int* __restrict__ adj_off,
                                                                 const int* __restrict__ adj,
                                                                 const unsigned long long* __restrict__ boxes,
                                                                 const uint8_t* __restrict__ vis,
-                                                                const R* __restrict__ contrib_i,
-                                                                const R* __restrict__ contrib_a,
-                                                                C* __restrict__ g_clip, R* __restrict__ part)
+                                                                const R* __restrict__ contrib, C* __restrict__ g_clip,
+                                                                R* __restrict__ part)
 {
-    int ci, v;
-    if (!gather_thread(d, ci, v)) return;
+    const unsigned nvb = (unsigned)((d.V + kBlockVertices - 1) / kBlockVertices);
+    const int ci = (int)(blockIdx.x / nvb), u = (int)threadIdx.x % kVertexLanes;
+    const int v = (int)(blockIdx.x % nvb) * kBlockVertices + (int)threadIdx.x / kVertexLanes;
     const int i = ci % d.I;
     const size_t base = (size_t)(ci / d.I) * d.H * d.W;
-    const unsigned long long* cbox = boxes + (size_t)ci * d.T;
-    const uint8_t* cvis = vis + (size_t)ci * d.T;
-    C gx = C(0), gy = C(0), gw = C(0);
-    R ga[8];
-    for (int a = 0; a < A; ++a) ga[a] = R(0);
-    const int j0 = adj_off[v], j1 = adj_off[v + 1];
-    for (int jb = j0; jb < j1; jb += kGatherBatch) {
-        // the batch's corners, then its boxes and flags: independent loads in flight together
-        int corner[kGatherBatch];
-        unsigned long long bx[kGatherBatch];
-        uint8_t seen[kGatherBatch];
+    const int j0 = v < d.V ? adj_off[v] : 0, j1 = v < d.V ? adj_off[v + 1] : 0;
+    VertexSum<C, R, NA> s;
+    sum_clear(s);
+    bool any = false;
+    for (int j = j0 + u; j < j1; j += kVertexLanes) {
+        const int corner = adj[j], t = corner / 3;
+        if (!vis[(size_t)ci * d.T + t]) continue;
+        any = true;
+        walk_box<C, R, NA, ATTR>(ids, base, d.W, unpack_box(boxes[(size_t)ci * d.T + t]), i * d.T + t + 1, corner - 3 * t,
+                                 contrib, A, s);
+    }
+    if (__ballot(any) != 0ull) sum8(s, A);
+    if (v >= d.V) return;
+    if (u < 4) g_clip[((size_t)ci * d.V + v) * 4 + u] = u == 0 ? s.x : u == 1 ? s.y : u == 2 ? C(0) : s.w;
+    if (ATTR) {
+        static_assert(kVertexLanes >= kMaxAttr, "a lane writes one channel");
+        VKGV_CHANNELS(a) if (u == a) part[((size_t)ci * d.V + v) * A + a] = s.a[a];
+    }
+}
+
+// The vertex pass of render, which goes on through the vertex transform
+// clip[ci, v] = M[ci] (p_v, 1): the clip gradient, zero for most (pair,
+// vertex) entries, is never stored.  A block takes kBlockVertices vertices and
+// kPairs camera-instance pairs (grid y) and writes the sums over its pairs of
+// M^T g (its positions' gradient) and of the attributes' gradient to
+// part_pos[y][V][3] and part_attr[y][V][A], and adds its sums over the
+// vertices of g (p_v, 1)^T to g_M.  boxes: of the triangles with vis set.
+//
+// Bound by the latency of flag -> box -> ids -> records: a wave goes through
+// the pairs in which any of its triangles has a pixel, the next pair's boxes in
+// flight.  64 pairs of 50k vertices: 125 us, where the gather, the reduction
+// over the pairs and the two passes of the vertex transform's backward over the
+// stored clip gradient took 217 + 22 + 36 + 110.  With the sums over lanes
+// through the LDS crossbar 142 us; each lane through its own pairs with LDS
+// atomics into g_M 165 us.
+constexpr int kPairs = 8;
+template <typename C, typename R, int NA>
+__global__ __launch_bounds__(kBlock) void vertex_render_kernel(const int* __restrict__ ids, Dims d, int A,
+                                                                const C* __restrict__ pos, const C* __restrict__ M,
+                                                                const int* __restrict__ adj_off,
+                                                                const int* __restrict__ adj,
+                                                                const unsigned long long* __restrict__ boxes,
+                                                                const uint8_t* __restrict__ vis,
+                                                                const R* __restrict__ contrib, C* __restrict__ part_pos,
+                                                                R* __restrict__ part_attr, C* __restrict__ g_M)
+{
+    constexpr int kRows = (int)kBlock / 16;   // rows of 16 lanes, two vertices each
+    __shared__ R2<C> s_g[kRows][kPairs][kVertexLanes];
+    const int lane = (int)(threadIdx.x & 63u), row = (int)(threadIdx.x >> 4), u = lane % kVertexLanes;
+    const int v = (int)blockIdx.x * kBlockVertices + (int)threadIdx.x / kVertexLanes;
+    const int ci0 = (int)blockIdx.y * kPairs, np = min(kPairs, d.C * d.I - ci0);
+    // a row's sums belong to its wave alone: no barrier before the end
+    for (int q = u; q < kPairs * kVertexLanes; q += kVertexLanes) (&s_g[row][0][0])[q] = R2<C>{ C(0), C(0) };
+    const bool live = v < d.V;
+    const int j0 = live ? adj_off[v] : 0, j1 = live ? adj_off[v + 1] : 0;
+    // lane u: homogeneous coordinates 2 (u & 1) and the next of its vertex
+    const C h0 = live ? pos[3 * (size_t)v + (u & 1 ? 2 : 0)] : C(0);
+    const C h1 = u & 1 ? C(1) : (live ? pos[3 * (size_t)v + 1] : C(0));
+    C g_pos = C(0);     // lane u < 3: component u
+    R g_attr = R(0);    // lane u < A: channel u
+    // rounds of kVertexLanes triangles; the sums are linear in them
+    for (int r = 0; __ballot(j0 + r < j1) != 0ull; r += kVertexLanes) {
+        const int j = j0 + r + u;
+        const int corner = j < j1 ? adj[j] : -1, t = corner / 3, k = corner - 3 * t;
+        uint32_t seen = 0u;     // bit q: the triangle has a pixel in pair ci0 + q
 #pragma unroll
-        for (int u = 0; u < kGatherBatch; ++u) corner[u] = jb + u < j1 ? adj[jb + u] : -1;
+        for (int q = 0; q < kPairs; ++q)
+            if (corner >= 0 && q < np && vis[(size_t)(ci0 + q) * d.T + t]) seen |= 1u << q;
+        uint32_t pairs = 0u;    // of any lane of the wave
 #pragma unroll
-        for (int u = 0; u < kGatherBatch; ++u) {
-            bx[u] = corner[u] >= 0 ? cbox[corner[u] / 3] : kNoBox;
-            seen[u] = corner[u] >= 0 ? cvis[corner[u] / 3] : 0;
-        }
-#pragma unroll
-        for (int u = 0; u < kGatherBatch; ++u) {
-            if (!seen[u] || bx[u] == kNoBox) continue;   // no gathered pixel: nothing to sum
-            const int t = corner[u] / 3, k = corner[u] % 3, id = i * d.T + t + 1;
-            const Box b = unpack_box(bx[u]);
-            const int bw = b.x1 - b.x0 + 1, n = bw * (b.y1 - b.y0 + 1);
-            // the box's ids kPixBatch at a time, all loads issued before the first compare
-            for (int q0 = 0; q0 < n; q0 += kPixBatch) {
-                size_t ip[kPixBatch];
-                int idq[kPixBatch];
-                int qx = b.x0 + q0 % bw, qy = b.y0 + q0 / bw;
-#pragma unroll
-                for (int w = 0; w < kPixBatch; ++w) {
-                    ip[w] = base + (size_t)qy * d.W + qx;
-                    idq[w] = q0 + w < n ? ids[ip[w]] : 0;
-                    if (++qx > b.x1) {
-                        qx = b.x0;
-                        ++qy;
-                    }
-                }
-#pragma unroll
-                for (int w = 0; w < kPixBatch; ++w) {
-                    if (idq[w] != id) continue;
-                    if (MODE & 1) {
-                        const R* o = contrib_i + (ip[w] * 3 + k) * (3 + A);
-                        gx += C(o[0]);
-                        gy += C(o[1]);
-                        gw += C(o[2]);
-                        for (int a = 0; a < A; ++a) ga[a] += o[3 + a];
-                    }
-                    if (MODE & 2) {
-                        const R* o = contrib_a + ip[w] * 9 + 3 * k;
-                        gx += C(o[0]);
-                        gy += C(o[1]);
-                        gw += C(o[2]);
-                    }
-                }
+        for (int q = 0; q < kPairs; ++q)
+            if (__ballot((seen >> q) & 1u) != 0ull) pairs |= 1u << q;
+        auto box_of = [&](int q) {
+            return (seen >> q) & 1u ? boxes[(size_t)(ci0 + q) * d.T + t] : 1ull;   // 1: an empty box
+        };
+        unsigned long long next = pairs ? box_of(__ffs((int)pairs) - 1) : 1ull;
+        while (pairs) {   // wave-uniform
+            const int q = __ffs((int)pairs) - 1;
+            const Box b = unpack_box(next);
+            pairs &= pairs - 1u;
+            if (pairs) next = box_of(__ffs((int)pairs) - 1);
+            const int ci = ci0 + q, i = ci % d.I, id = i * d.T + t + 1;
+            const size_t base = (size_t)(ci / d.I) * d.H * d.W;
+            VertexSum<C, R, NA> s;
+            sum_clear(s);
+            const bool mine = (seen >> q) & 1u, wide = mine && (b.x1 - b.x0 + 1) * (b.y1 - b.y0 + 1) > kWaveBox;
+            if (mine && !wide) walk_box<C, R, NA, true>(ids, base, d.W, b, id, k, contrib, A, s);
+            unsigned long long pending = __ballot(wide);
+            while (pending != 0ull) {
+                const int l = __ffsll((long long)pending) - 1;
+                pending &= pending - 1ull;
+                const Box wb{ __builtin_amdgcn_readlane(b.x0, l), __builtin_amdgcn_readlane(b.x1, l),
+                              __builtin_amdgcn_readlane(b.y0, l), __builtin_amdgcn_readlane(b.y1, l) };
+                walk_wide<C, R, NA, true>(ids, base, d.W, wb, __builtin_amdgcn_readlane(id, l),
+                                          __builtin_amdgcn_readlane(k, l), contrib, A, l, s);
+            }
+            sum8(s, A);
+            const C* m = M + (size_t)ci * 16;
+            const int c = u < 3 ? u : 0;
+            g_pos += (m[c] * s.x + m[4 + c] * s.y) + m[12 + c] * s.w;
+            VKGV_CHANNELS(a) if (u == a) g_attr += s.a[a];
+            // g_M[row][col] += g_row (p, 1)_col: lane u of each vertex forms row u / 2, columns 2 (u & 1)
+            // and the next, summed over the row's two vertices
+            const C gr = (u >> 1) == 0 ? s.x : (u >> 1) == 1 ? s.y : (u >> 1) == 2 ? C(0) : s.w;
+            C e0 = gr * h0, e1 = gr * h1;
+            e0 += lane_move<kRor8>(e0);
+            e1 += lane_move<kRor8>(e1);
+            if ((lane & 8) == 0) {
+                R2<C>& g = s_g[row][q][u];
+                g.x += e0;
+                g.y += e1;
             }
         }
     }
-    C* g = g_clip + ((size_t)ci * d.V + v) * 4;
-    g[0] = gx;
-    g[1] = gy;
-    g[2] = C(0);
-    g[3] = gw;
-    if (MODE & 1) {
-        R* o = part + ((size_t)ci * d.V + v) * A;
-        for (int a = 0; a < A; ++a) o[a] = ga[a];
+    if (live) {
+        if (u < 3) part_pos[((size_t)blockIdx.y * d.V + v) * 3 + u] = g_pos;
+        VKGV_CHANNELS(a) if (u == a) part_attr[((size_t)blockIdx.y * d.V + v) * A + a] = g_attr;
+    }
+    __syncthreads();
+    for (int k = (int)threadIdx.x; k < np * 16; k += (int)kBlock) {
+        C t = C(0);
+        for (int w = 0; w < kRows; ++w) t += reinterpret_cast<const C*>(&s_g[w][k >> 4][0])[k & 15];
+        if (t != C(0)) unsafeAtomicAdd(&g_M[(size_t)ci0 * 16 + k], t);
     }
 }
 
@@ -607,6 +928,24 @@ __global__ __launch_bounds__(kBlock) void attr_reduce_kernel(const R* __restrict
     R s = R(0);
     for (int ci = 0; ci < CI; ++ci) s += part[(size_t)ci * VA + j];
     g_attr[j] = s;
+}
+
+// Sums of `parts` arrays a[.][na] and b[.][nb], in part order.
+template <typename C, typename R>
+__global__ __launch_bounds__(kBlock) void part_reduce_kernel(const C* __restrict__ a, size_t na, C* __restrict__ out_a,
+                                                              const R* __restrict__ b, size_t nb, R* __restrict__ out_b,
+                                                              int parts)
+{
+    const size_t j = (size_t)blockIdx.x * kBlock + threadIdx.x;
+    if (j < na) {
+        C s = C(0);
+        for (int p = 0; p < parts; ++p) s += a[(size_t)p * na + j];
+        out_a[j] = s;
+    } else if (j < na + nb) {
+        R s = R(0);
+        for (int p = 0; p < parts; ++p) s += b[(size_t)p * nb + (j - na)];
+        out_b[j - na] = s;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -789,7 +1128,6 @@ __device__ __forceinline__ bool pair_of(int q, int px, int py, int& ax, int& ay,
 // antialiasing apart: 44 + 118), backward 106 us (107 + 242).
 constexpr int kTileW = 32, kTileH = 16, kTileThreads = kTileW * kTileH;
 constexpr int kInnerW = kTileW - 2, kInnerH = kTileH - 2;
-constexpr int kMaxAttr = 8;
 
 struct TilePixel {
     int c, x, y;
@@ -847,18 +1185,20 @@ template <typename R> struct TileState {
     }
 };
 
-// NA: the attribute count, 0 for a count only known at run time (at most kMaxAttr).
-#define VKGV_CHANNELS(a) _Pragma("unroll") for (int a = 0; a < (NA ? NA : kMaxAttr); ++a) if (NA || a < A)
-
-// Forward: SHADE interpolates the colour (written to `color`) and marks the
-// pixels for the backward as interp_fwd_kernel does; without it `color` is
-// given.  out = the antialiased colour.
-template <typename C, typename R, bool SHADE, int NA>
+// Forward: out = the antialiased colour.  FROM says what it starts from:
+//   kFromColor  the given `color`, ids and depth;
+//   kFromIds    ids and depth; the colour is interpolated here and written;
+//   kFromKeys   the raster's keys of the same clip positions: ids and depth
+//               are written too, and no pixel can be a stray.
+// The pixels are marked for the backward as interp_fwd_kernel does.
+enum { kFromColor, kFromIds, kFromKeys };
+template <typename C, typename R, int FROM, int NA>
 __global__ __launch_bounds__(kTileThreads) void aa_fwd_kernel(R* __restrict__ color, const C* __restrict__ clip,
                                                                const R* __restrict__ attr,
-                                                               const int* __restrict__ tris, const int* __restrict__ ids,
-                                                               const float* __restrict__ depth, Dims d, int A,
-                                                               R* __restrict__ out,
+                                                               const int* __restrict__ tris, int* __restrict__ ids,
+                                                               float* __restrict__ depth,
+                                                               const unsigned long long* __restrict__ keys, Dims d,
+                                                               int A, R* __restrict__ out,
                                                                const unsigned long long* __restrict__ boxes,
                                                                unsigned* __restrict__ stray_blocks,
                                                                uint8_t* __restrict__ vis)
@@ -867,18 +1207,29 @@ __global__ __launch_bounds__(kTileThreads) void aa_fwd_kernel(R* __restrict__ co
     __shared__ R s_col[NA ? NA : kMaxAttr][kTileThreads];
     const int t = (int)threadIdx.x;
     const TilePixel px = tile_pixel(d);
-    const int raw = px.in ? ids[px.p] : 0;
-    const int id = id_in_range(raw, d) ? raw : 0;
+    int id = 0;
+    float dep = 0.0f;
+    if (FROM == kFromKeys) {
+        if (px.in) key_parts(keys[px.p], id, dep);
+        if (px.inner) {
+            ids[px.p] = id;
+            depth[px.p] = dep;
+        }
+    } else if (px.in) {
+        id = ids[px.p];
+        dep = depth[px.p];
+    }
+    id = id_in_range(id, d) ? id : 0;
     s.id[t] = px.in ? id : -1;
-    s.depth[t] = px.in ? depth[px.p] : 0.0f;
-    if (!SHADE) {
+    s.depth[t] = dep;
+    if (FROM == kFromColor) {
         VKGV_CHANNELS(a) s_col[a][t] = px.in ? color[px.p * A + a] : R(0);
     }
     int i, tri, vi[3];
     V4<C> P[3];
     const bool ok = id > 0 && tri_of(clip, tris, d, px.c, id, i, tri, vi, P);
     const C xn = ndc_x<C>(px.x, d), yn = ndc_y<C>(px.y, d);
-    if (SHADE) {
+    if (FROM != kFromColor) {
         Bary<R> b;
         if (ok) {
             bary_from(P, xn, yn, b);
@@ -890,7 +1241,10 @@ __global__ __launch_bounds__(kTileThreads) void aa_fwd_kernel(R* __restrict__ co
             if (px.inner) color[px.p * A + a] = v;
         }
     }
-    if (ok && px.inner) mark_pixel(boxes, d, px.c, id, px.x, px.y, px.p, stray_blocks, vis);
+    if (ok && px.inner) {
+        if (FROM == kFromKeys) vis[tri_index(d, px.c, id)] = 1;
+        else mark_pixel(boxes, d, px.c, id, px.x, px.y, px.p, stray_blocks, vis);
+    }
     __syncthreads();
     FrontTri<R> f;
     const bool fr = ok && front_tri<C, R>(P, xn, yn, d, f);
@@ -985,7 +1339,7 @@ __device__ __forceinline__ void add_clip_grad(C* g_clip, const Dims& d, int c, i
 // w) of corner k of the pixel's triangle from the blends whose front pixel it
 // is.  SHADE: the colour gradient goes on through the interpolation, and
 // contrib[p][k] = (its corner terms + cg[k], lambda_k g_color[0..A-1]); g_color
-// is written only where the stray pass reads it.  Without SHADE g_color is
+// is written only where the stray pass reads it (stray_blocks null: there is none).  Without SHADE g_color is
 // written and contrib[p][k] = cg[k], for every pixel with an id.
 template <typename C, typename R, bool SHADE, int NA>
 __global__ __launch_bounds__(kTileThreads) void aa_bwd_pixel_kernel(const R* __restrict__ color,
@@ -1079,7 +1433,7 @@ __global__ __launch_bounds__(kTileThreads) void aa_bwd_pixel_kernel(const R* __r
             for (int k = 0; k < 9; ++k) contrib[px.p * 9 + k] = cg[k];
         return;
     }
-    if (stray_blocks[px.p / kBlock] != 0u) {
+    if (stray_blocks && stray_blocks[px.p / kBlock] != 0u) {
         VKGV_CHANNELS(a) g_color[px.p * A + a] = acc[a];
     }
     if (!ok) return;
@@ -1243,10 +1597,9 @@ __global__ __launch_bounds__(kBlock) void transform_fwd_kernel(const C* __restri
     const int v = blockIdx.x * kBlock + threadIdx.x;
     const int ci = blockIdx.y;
     if (v >= V) return;
-    const C* m = A + (size_t)ci * 16;
-    const C x = pos[3 * v], y = pos[3 * v + 1], z = pos[3 * v + 2];
-    C* o = clip + ((size_t)ci * V + v) * 4;
-    for (int r = 0; r < 4; ++r) o[r] = fma(m[4 * r], x, fma(m[4 * r + 1], y, fma(m[4 * r + 2], z, m[4 * r + 3])));
+    V4<C> o;
+    transform_vertex(A + (size_t)ci * 16, pos + 3 * (size_t)v, o);
+    reinterpret_cast<V4<C>*>(clip)[(size_t)ci * V + v] = o;
 }
 
 // g_pos[v] = sum over (c, i) of A[c, i][:, :3]^T g_clip[c, i, v]; one thread per vertex.
@@ -1310,13 +1663,18 @@ inline unsigned blocks(size_t n) { return (unsigned)((n + kBlock - 1) / kBlock);
 } // namespace
 
 // ---------------------------------------------------------------------------
-void raster_tris(const float* clip, const int* tris, int C, int I, int V, int T, int H, int W, int cull_back,
+static dim3 raster_grid(const Dims& d) { return dim3(blocks((size_t)d.T), std::min(d.C * d.I, 65535)); }
+
+void raster_tris(const float* clip, const int* tris, int C, int I, int V, int T, int H, int W, int cull_back, void* snap,
                  unsigned long long* keys, int* ids, float* depth, hipStream_t st)
 {
     const Dims d{ C, I, V, T, H, W };
-    const size_t npx = (size_t)C * H * W;
-    const size_t ntri = (size_t)C * I * T;
-    if (ntri && npx) raster_tris_kernel<<<blocks(ntri), kBlock, 0, st>>>(clip, tris, d, keys, cull_back);
+    const size_t npx = (size_t)C * H * W, nv = (size_t)C * I * V;
+    if (C * I && T && nv && npx) {
+        snap_kernel<<<blocks(nv), kBlock, 0, st>>>(clip, d, nv, static_cast<Snap*>(snap));
+        raster_tris_kernel<<<raster_grid(d), kBlock, 0, st>>>(static_cast<const Snap*>(snap), tris, d, keys, nullptr,
+                                                              cull_back);
+    }
     if (npx) keys_to_ids_kernel<<<blocks(npx), kBlock, 0, st>>>(keys, npx, ids, depth);
 }
 
@@ -1372,8 +1730,21 @@ void tri_boxes(const double* clip, const int* tris, int nc, int I, int V, int T,
     tri_boxes_t<double>(clip, tris, nc, I, V, T, H, W, boxes, stray_blocks, st);
 }
 
-// Blocks of a vertex pass over (camera-instance pair, vertex).
-static unsigned gather_blocks(int nc, int I, int V) { return blocks((size_t)V) * (unsigned)(nc * I); }
+// The vertex pass of interpolate, antialias and shade.
+template <typename C, typename R, bool ATTR>
+static void vertex_gather(const int* ids, const Dims& d, int A, const int* adj_off, const int* adj,
+                          const unsigned long long* boxes, const R* contrib, C* g_clip, R* part, hipStream_t st)
+{
+    const unsigned n = (unsigned)((d.V + kBlockVertices - 1) / kBlockVertices) * (unsigned)(d.C * d.I);
+    if (n == 0) return;
+    const uint8_t* vis = vis_of(boxes, d.C, d.I, d.T);
+    if (A == 3)
+        vertex_gather_kernel<C, R, ATTR, 3><<<n, kBlock, 0, st>>>(ids, d, A, adj_off, adj, boxes, vis, contrib, g_clip,
+                                                                  part);
+    else
+        vertex_gather_kernel<C, R, ATTR, 0><<<n, kBlock, 0, st>>>(ids, d, A, adj_off, adj, boxes, vis, contrib, g_clip,
+                                                                  part);
+}
 
 template <typename C, typename R>
 static void interp_fwd_t(const C* clip, const R* attr, const int* tris, const int* ids, int nc, int I, int V, int T,
@@ -1398,29 +1769,25 @@ static void interp_bwd_t(const C* clip, const R* attr, const int* tris, const in
     if (npx)
         interp_bwd_pixel_kernel<C, R><<<blocks(npx), kBlock, 0, st>>>(clip, attr, tris, ids, d, A, g_out,
                                                                       contrib);
-    if (nc * I)
-        vertex_gather_kernel<C, R, 1><<<gather_blocks(nc, I, V), kBlock, 0, st>>>(
-            ids, d, A, adj_off, adj, boxes, vis_of(boxes, nc, I, T), contrib, nullptr, g_clip, part);
+    vertex_gather<C, R, true>(ids, d, A, adj_off, adj, boxes, contrib, g_clip, part, st);
     attr_reduce_kernel<R><<<blocks((size_t)V * A), kBlock, 0, st>>>(part, nc * I, (size_t)V * A, g_attr);
     if (npx)
         interp_bwd_stray_kernel<C, R><<<blocks(npx), kBlock, 0, st>>>(clip, attr, tris, ids, d, A, g_out, boxes,
                                                                       stray_blocks, g_clip, g_attr);
 }
 
-template <typename C, typename R, bool SHADE>
-static void aa_fwd_t(R* color, const C* clip, const R* attr, const int* tris, const int* ids, const float* depth, int nc,
-                     int I, int V, int T, int H, int W, int A, R* out, unsigned long long* boxes,
-                     unsigned* stray_blocks, hipStream_t st)
+template <typename C, typename R, int FROM>
+static void aa_fwd_t(R* color, const C* clip, const R* attr, const int* tris, int* ids, float* depth,
+                     const unsigned long long* keys, const Dims& d, int A, R* out, const unsigned long long* boxes,
+                     unsigned* stray_blocks, uint8_t* vis, hipStream_t st)
 {
-    const Dims d{ nc, I, V, T, H, W };
-    if ((size_t)nc * H * W == 0) return;
-    uint8_t* vis = vis_of(boxes, nc, I, T);
+    if ((size_t)d.C * d.H * d.W == 0) return;
     if (A == 3)
-        aa_fwd_kernel<C, R, SHADE, 3><<<tile_blocks(d), kTileThreads, 0, st>>>(color, clip, attr, tris, ids, depth, d, A,
-                                                                               out, boxes, stray_blocks, vis);
+        aa_fwd_kernel<C, R, FROM, 3><<<tile_blocks(d), kTileThreads, 0, st>>>(color, clip, attr, tris, ids, depth, keys,
+                                                                              d, A, out, boxes, stray_blocks, vis);
     else
-        aa_fwd_kernel<C, R, SHADE, 0><<<tile_blocks(d), kTileThreads, 0, st>>>(color, clip, attr, tris, ids, depth, d, A,
-                                                                               out, boxes, stray_blocks, vis);
+        aa_fwd_kernel<C, R, FROM, 0><<<tile_blocks(d), kTileThreads, 0, st>>>(color, clip, attr, tris, ids, depth, keys,
+                                                                              d, A, out, boxes, stray_blocks, vis);
 }
 
 template <typename C, typename R, bool SHADE>
@@ -1446,9 +1813,7 @@ static void aa_bwd_t(const R* color, const C* clip, const int* tris, const int* 
     const Dims d{ nc, I, V, T, H, W };
     const size_t npx = (size_t)nc * H * W;
     aa_bwd_pixel<C, R, false>(color, clip, nullptr, tris, ids, depth, d, A, g_out, stray_blocks, g_color, contrib, st);
-    if (V && nc * I)
-        vertex_gather_kernel<C, R, 2><<<gather_blocks(nc, I, V), kBlock, 0, st>>>(
-            ids, d, A, adj_off, adj, boxes, vis_of(boxes, nc, I, T), nullptr, contrib, g_clip, nullptr);
+    vertex_gather<C, R, false>(ids, d, A, adj_off, adj, boxes, contrib, g_clip, static_cast<R*>(nullptr), st);
     if (npx && V)
         aa_bwd_stray_kernel<C, R><<<blocks(npx), kBlock, 0, st>>>(color, clip, tris, ids, depth, d, A, g_out, boxes,
                                                                   stray_blocks, g_clip);
@@ -1467,15 +1832,57 @@ static void shade_bwd_t(const R* color, const C* clip, const R* attr, const int*
     const size_t npx = (size_t)nc * H * W;
     if (V == 0) return;
     aa_bwd_pixel<C, R, true>(color, clip, attr, tris, ids, depth, d, A, g_out, stray_blocks, g_color, contrib, st);
-    if (nc * I)
-        vertex_gather_kernel<C, R, 1><<<gather_blocks(nc, I, V), kBlock, 0, st>>>(
-            ids, d, A, adj_off, adj, boxes, vis_of(boxes, nc, I, T), contrib, nullptr, g_clip, part);
+    vertex_gather<C, R, true>(ids, d, A, adj_off, adj, boxes, contrib, g_clip, part, st);
     attr_reduce_kernel<R><<<blocks((size_t)V * A), kBlock, 0, st>>>(part, nc * I, (size_t)V * A, g_attr);
     if (npx) {
         interp_bwd_stray_kernel<C, R><<<blocks(npx), kBlock, 0, st>>>(clip, attr, tris, ids, d, A, g_color, boxes,
                                                                       stray_blocks, g_clip, g_attr);
         aa_bwd_stray_kernel<C, R><<<blocks(npx), kBlock, 0, st>>>(color, clip, tris, ids, depth, d, A, g_out, boxes,
                                                                   stray_blocks, g_clip);
+    }
+}
+
+// Projection, raster and shading of a mesh, from its own keys.
+template <typename C, typename R>
+static void render_fwd_t(const C* pos, const C* M, const R* attr, const int* tris, const Dims& d, int A, C* clip,
+                         void* snap, unsigned long long* keys, unsigned long long* boxes, uint8_t* vis, int* ids,
+                         float* depth, R* color, R* out, hipStream_t st)
+{
+    const size_t npx = (size_t)d.C * d.H * d.W, nvis = ((size_t)d.C * d.I * d.T + 3) / 4;
+    if (npx == 0) return;
+    // at least one block, which clears the keys, also without vertices
+    project_kernel<C><<<dim3(std::max(1u, blocks((size_t)d.V)), std::max(1, d.C * d.I)), kBlock, 0, st>>>(
+        pos, M, d, clip, static_cast<Snap*>(snap), keys, npx, reinterpret_cast<uint32_t*>(vis), nvis);
+    if (d.C * d.I && d.T && d.V)
+        raster_tris_kernel<<<raster_grid(d), kBlock, 0, st>>>(static_cast<const Snap*>(snap), tris, d, keys, boxes, 0);
+    aa_fwd_t<C, R, kFromKeys>(color, clip, attr, tris, ids, depth, keys, d, A, out, nullptr, nullptr, vis, st);
+}
+
+int render_parts(int nc, int I) { return std::max(1, (nc * I + kPairs - 1) / kPairs); }
+
+// part_pos and part_attr: render_parts(nc, I) gradients, reduced into g_pos and
+// g_attr (with one part they are those themselves).
+template <typename C, typename R>
+static void render_bwd_t(const C* pos, const C* M, const R* attr, const int* tris, const Dims& d, int A, const C* clip,
+                         const unsigned long long* boxes, const uint8_t* vis, const int* ids, const float* depth,
+                         const R* color, const int* adj_off, const int* adj, const R* g_out, R* contrib, C* part_pos,
+                         R* part_attr, C* g_pos, C* g_M, R* g_attr, hipStream_t st)
+{
+    if (d.V == 0) return;
+    const int parts = render_parts(d.C, d.I);
+    aa_bwd_pixel<C, R, true>(color, clip, attr, tris, ids, depth, d, A, g_out, nullptr, nullptr, contrib, st);
+    const dim3 grid((unsigned)((d.V + kBlockVertices - 1) / kBlockVertices), (unsigned)parts);
+    C* pp = parts > 1 ? part_pos : g_pos;
+    R* pa = parts > 1 ? part_attr : g_attr;
+    if (A == 3)
+        vertex_render_kernel<C, R, 3><<<grid, kBlock, 0, st>>>(ids, d, A, pos, M, adj_off, adj, boxes, vis, contrib, pp,
+                                                               pa, g_M);
+    else
+        vertex_render_kernel<C, R, 0><<<grid, kBlock, 0, st>>>(ids, d, A, pos, M, adj_off, adj, boxes, vis, contrib, pp,
+                                                               pa, g_M);
+    if (parts > 1) {
+        const size_t np = (size_t)d.V * 3, na = (size_t)d.V * A;
+        part_reduce_kernel<C, R><<<blocks(np + na), kBlock, 0, st>>>(part_pos, np, g_pos, part_attr, na, g_attr, parts);
     }
 }
 
@@ -1530,14 +1937,34 @@ void transform_bwd(const double* g_clip, const double* pos, const double* A, int
                 int V, int T, int H, int W, int A, R* out, unsigned long long* boxes, unsigned* stray_blocks,          \
                 hipStream_t st)                                                                                        \
     {                                                                                                                  \
-        aa_fwd_t<C, R, false>(const_cast<R*>(color), clip, nullptr, tris, ids, depth, nc, I, V, T, H, W, A, out,       \
-                              boxes, stray_blocks, st);                                                                \
+        const Dims d{ nc, I, V, T, H, W };                                                                             \
+        aa_fwd_t<C, R, kFromColor>(const_cast<R*>(color), clip, nullptr, tris, const_cast<int*>(ids),                  \
+                                   const_cast<float*>(depth), nullptr, d, A, out, boxes, stray_blocks,                 \
+                                   vis_of(boxes, nc, I, T), st);                                                       \
     }                                                                                                                  \
     void shade_fwd(const C* clip, const R* attr, const int* tris, const int* ids, const float* depth, int nc, int I,   \
                    int V, int T, int H, int W, int A, R* color, R* out, unsigned long long* boxes,                     \
                    unsigned* stray_blocks, hipStream_t st)                                                             \
     {                                                                                                                  \
-        aa_fwd_t<C, R, true>(color, clip, attr, tris, ids, depth, nc, I, V, T, H, W, A, out, boxes, stray_blocks, st); \
+        const Dims d{ nc, I, V, T, H, W };                                                                             \
+        aa_fwd_t<C, R, kFromIds>(color, clip, attr, tris, const_cast<int*>(ids), const_cast<float*>(depth), nullptr,   \
+                                 d, A, out, boxes, stray_blocks, vis_of(boxes, nc, I, T), st);                         \
+    }                                                                                                                  \
+    void render_fwd(const C* pos, const C* M, const R* attr, const int* tris, int nc, int I, int V, int T, int H,      \
+                    int W, int A, C* clip, void* snap, unsigned long long* keys, unsigned long long* boxes,            \
+                    uint8_t* vis, int* ids, float* depth, R* color, R* out, hipStream_t st)                            \
+    {                                                                                                                  \
+        const Dims d{ nc, I, V, T, H, W };                                                                             \
+        render_fwd_t<C, R>(pos, M, attr, tris, d, A, clip, snap, keys, boxes, vis, ids, depth, color, out, st);        \
+    }                                                                                                                  \
+    void render_bwd(const C* pos, const C* M, const R* attr, const int* tris, int nc, int I, int V, int T, int H,      \
+                    int W, int A, const C* clip, const unsigned long long* boxes, const uint8_t* vis, const int* ids,  \
+                    const float* depth, const R* color, const int* adj_off, const int* adj, const R* g_out,            \
+                    R* contrib, C* part_pos, R* part_attr, C* g_pos, C* g_M, R* g_attr, hipStream_t st)                \
+    {                                                                                                                  \
+        const Dims d{ nc, I, V, T, H, W };                                                                             \
+        render_bwd_t<C, R>(pos, M, attr, tris, d, A, clip, boxes, vis, ids, depth, color, adj_off, adj, g_out,         \
+                           contrib, part_pos, part_attr, g_pos, g_M, g_attr, st);                                      \
     }                                                                                                                  \
     void aa_bwd(const R* color, const C* clip, const int* tris, const int* ids, const float* depth, int nc, int I,     \
                 int V, int T, int H, int W, int A, const unsigned long long* boxes, const unsigned* stray_blocks,      \

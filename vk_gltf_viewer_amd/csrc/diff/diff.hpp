@@ -2,11 +2,13 @@
 // the torch bindings (diff_ext.cpp) own the tensors and the autograd graph.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <stdint.h>
 
 namespace vkgv_diff {
 
-// keys: C*H*W u64 set to all ones by the caller; ids / depth: C*H*W.
-void raster_tris(const float* clip, const int* tris, int C, int I, int V, int T, int H, int W, int cull_back,
+// keys: C*H*W u64 set to all ones by the caller; ids / depth: C*H*W; snap:
+// scratch of 16 bytes per clip position.
+void raster_tris(const float* clip, const int* tris, int C, int I, int V, int T, int H, int W, int cull_back, void* snap,
                  unsigned long long* keys, int* ids, float* depth, hipStream_t st);
 // Vertex transform: clip [CI, V, 4] = A [CI, 4, 4] (pos [V, 3], 1), and its
 // backward: g_pos [V, 3] (written) and g_A [CI, 4, 4] (accumulated into,
@@ -48,6 +50,14 @@ size_t stray_flag_count(int nc, int H, int W);
 // Scratch: contrib, nc * H * W * 3 * (3 + A) entries for interp_bwd and
 // shade_bwd and nc * H * W * 9 for aa_bwd; part, nc * I * V * A entries; the
 // g_color of shade_bwd.
+// render_fwd / render_bwd: projection (clip = M (pos, 1)), raster and shading
+// of a mesh in one.  Scratch: snap, 16 bytes per clip position; keys, C * H * W
+// entries; contrib as for shade_bwd; part_pos [render_parts][V][3] and
+// part_attr [render_parts][V][A].  Kept for the backward: clip, boxes (one
+// entry per camera, instance and triangle, written for those with a fragment),
+// vis (as many bytes, rounded up to 4), ids, depth, color.  g_M is accumulated
+// into, zeroed by the caller.
+int render_parts(int nc, int I);
 #define VKGV_DIFF_DECLARE(C, R)                                                                                       \
     void interp_fwd(const C* clip, const R* attr, const int* tris, const int* ids, int nc, int I, int V, int T, int H, \
                     int W, int A, R* out, unsigned long long* boxes, unsigned* stray_blocks, hipStream_t st);          \
@@ -60,6 +70,13 @@ size_t stray_flag_count(int nc, int H, int W);
     void shade_fwd(const C* clip, const R* attr, const int* tris, const int* ids, const float* depth, int nc, int I,   \
                    int V, int T, int H, int W, int A, R* color, R* out, unsigned long long* boxes,                     \
                    unsigned* stray_blocks, hipStream_t st);                                                            \
+    void render_fwd(const C* pos, const C* M, const R* attr, const int* tris, int nc, int I, int V, int T, int H,      \
+                    int W, int A, C* clip, void* snap, unsigned long long* keys, unsigned long long* boxes,            \
+                    uint8_t* vis, int* ids, float* depth, R* color, R* out, hipStream_t st);                           \
+    void render_bwd(const C* pos, const C* M, const R* attr, const int* tris, int nc, int I, int V, int T, int H,      \
+                    int W, int A, const C* clip, const unsigned long long* boxes, const uint8_t* vis, const int* ids,  \
+                    const float* depth, const R* color, const int* adj_off, const int* adj, const R* g_out,            \
+                    R* contrib, C* part_pos, R* part_attr, C* g_pos, C* g_M, R* g_attr, hipStream_t st);               \
     void aa_bwd(const R* color, const C* clip, const int* tris, const int* ids, const float* depth, int nc, int I,     \
                 int V, int T, int H, int W, int A, const unsigned long long* boxes, const unsigned* stray_blocks,      \
                 const int* adj_off, const int* adj, const R* g_out, R* contrib, R* g_color, C* g_clip,                 \

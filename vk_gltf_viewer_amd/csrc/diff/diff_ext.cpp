@@ -145,7 +145,7 @@ const unsigned* flag_ptr(const Tensor& flags) { return reinterpret_cast<const un
 
 void check_gather(const Shape& s)
 {
-    TORCH_CHECK(((int64_t)s.V + 255) / 256 * s.C * s.I < ((int64_t)1 << 31), "too many camera-instance-vertex triples");
+    TORCH_CHECK(((int64_t)s.V + 31) / 32 * s.C * s.I < ((int64_t)1 << 31), "too many camera-instance-vertex triples");
 }
 
 struct InterpolateFn : public torch::autograd::Function<InterpolateFn> {
@@ -355,24 +355,111 @@ void check_vertex_range(const Tensor& tris, int64_t V)
     if (seen->size() > 8) seen->pop_back();
 }
 
+// What rasterize and render ask of a mesh and a view.
+void check_raster(const Tensor& tris, int64_t I, int64_t V, int64_t H, int64_t W)
+{
+    check_i32(tris, "tris");
+    TORCH_CHECK(H > 0 && W > 0 && H <= 16384 && W <= 16384, "resolution 1..16384");
+    TORCH_CHECK(I * tris.size(0) < (int64_t)0x7FFFFFFF, "instances x triangles must fit the 31-bit id");
+    check_vertex_range(tris, V);
+}
+
 std::vector<Tensor> rasterize(Tensor clip, Tensor tris, int64_t H, int64_t W, bool cull_back)
 {
     check_f32(clip, "clip");
-    check_i32(tris, "tris");
     TORCH_CHECK(clip.dim() == 4 && clip.size(3) == 4, "clip must be [C, I, V, 4]");
-    TORCH_CHECK(H > 0 && W > 0 && H <= 16384 && W <= 16384, "resolution 1..16384");
-    TORCH_CHECK(clip.size(1) * tris.size(0) < (int64_t)0x7FFFFFFF, "instances x triangles must fit the 31-bit id");
-    check_vertex_range(tris, clip.size(2));
+    check_raster(tris, clip.size(1), clip.size(2), H, W);
     const int C = (int)clip.size(0);
     auto opt = clip.options();
     Tensor keys = torch::full({ C, H, W }, -1, opt.dtype(torch::kInt64));
     Tensor ids = torch::empty({ C, H, W }, opt.dtype(torch::kInt32));
     Tensor depth = torch::empty({ C, H, W }, opt);
+    Tensor snap = torch::empty_like(clip);   // 16 bytes per vertex, as the clip positions
     vkgv_diff::raster_tris(clip.data_ptr<float>(), tris.data_ptr<int>(), C, (int)clip.size(1), (int)clip.size(2),
-                           (int)tris.size(0), (int)H, (int)W, cull_back ? 1 : 0,
+                           (int)tris.size(0), (int)H, (int)W, cull_back ? 1 : 0, snap.data_ptr<float>(),
                            reinterpret_cast<unsigned long long*>(keys.data_ptr<int64_t>()), ids.data_ptr<int>(),
                            depth.data_ptr<float>(), stream());
     return { ids, depth };
+}
+
+// transform, rasterize and shade as one function of the mesh: the same image
+// and ids, and gradients to the positions, the matrices and the attributes
+// without a clip gradient in between.
+struct RenderFn : public torch::autograd::Function<RenderFn> {
+    static variable_list forward(AutogradContext* ctx, Tensor pos, Tensor M, Tensor attr, Tensor tris, int64_t H,
+                                 int64_t W)
+    {
+        check_real(pos, "pos", pos);
+        check_real(M, "A", pos);
+        check_real(attr, "attr", pos);
+        TORCH_CHECK(M.scalar_type() == pos.scalar_type(), "A must have the positions' type");
+        TORCH_CHECK(pos.dim() == 2 && pos.size(1) == 3, "pos must be [V, 3]");
+        TORCH_CHECK(M.dim() == 4 && M.size(2) == 4 && M.size(3) == 4, "A must be [C, I, 4, 4]");
+        TORCH_CHECK(M.size(0) * M.size(1) < 65536, "at most 65535 camera-instance pairs");
+        TORCH_CHECK(pos.size(0) < (int64_t)0x7FFFFFFF, "too many vertices");
+        TORCH_CHECK(tris.dim() == 2 && tris.size(1) == 3, "tris must be [T, 3]");
+        TORCH_CHECK(attr.dim() == 2 && attr.size(0) == pos.size(0), "attr must be [V, A]");
+        TORCH_CHECK(attr.size(1) >= 1 && attr.size(1) <= 8, "1..8 attribute channels");
+        check_raster(tris, M.size(1), pos.size(0), H, W);
+        const Shape s{ (int)M.size(0), (int)M.size(1), (int)pos.size(0), (int)tris.size(0), (int)H, (int)W,
+                       (int)attr.size(1) };
+        check_gather(s);
+        const int64_t nt = (int64_t)s.C * s.I * s.T;
+        auto i64 = pos.options().dtype(torch::kInt64);
+        Tensor clip = torch::empty({ s.C, s.I, s.V, 4 }, pos.options());
+        Tensor snap = torch::empty({ s.C, s.I, s.V, 4 }, pos.options().dtype(torch::kInt32));
+        Tensor keys = torch::empty({ s.C, H, W }, i64), boxes = torch::empty({ std::max<int64_t>(nt, 1) }, i64);
+        Tensor vis = torch::empty({ (nt + 7) / 4 * 4 }, pos.options().dtype(torch::kUInt8));
+        Tensor ids = torch::empty({ s.C, H, W }, pos.options().dtype(torch::kInt32));
+        Tensor depth = torch::empty({ s.C, H, W }, pos.options().dtype(torch::kFloat32));
+        Tensor color = torch::empty({ s.C, H, W, s.A }, attr.options()), out = torch::empty_like(color);
+        dispatch_real(pos, attr, [&](auto cc, auto r) {
+            using C = decltype(cc);
+            using R = decltype(r);
+            vkgv_diff::render_fwd(pos.data_ptr<C>(), M.data_ptr<C>(), attr.data_ptr<R>(), tris.data_ptr<int>(), s.C, s.I,
+                                  s.V, s.T, s.H, s.W, s.A, clip.data_ptr<C>(), snap.data_ptr<int>(),
+                                  reinterpret_cast<unsigned long long*>(keys.data_ptr<int64_t>()), box_ptr(boxes),
+                                  vis.data_ptr<uint8_t>(), ids.data_ptr<int>(), depth.data_ptr<float>(),
+                                  color.data_ptr<R>(), out.data_ptr<R>(), stream());
+        });
+        ctx->save_for_backward({ pos, M, attr, tris, clip, boxes, vis, ids, depth, color });
+        ctx->mark_non_differentiable({ ids, depth });
+        ctx->set_materialize_grads(false);   // no zero images for the ids and the depth
+        return { out, ids, depth };
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads)
+    {
+        if (!grads[0].defined()) return { Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor() };
+        const auto saved = ctx->get_saved_variables();
+        const Tensor &pos = saved[0], &M = saved[1], &attr = saved[2], &tris = saved[3], &clip = saved[4];
+        const Tensor &boxes = saved[5], &vis = saved[6], &ids = saved[7], &depth = saved[8], &color = saved[9];
+        const Shape s{ (int)M.size(0), (int)M.size(1), (int)pos.size(0), (int)tris.size(0), (int)ids.size(1),
+                       (int)ids.size(2), (int)attr.size(1) };
+        Tensor g_out = grads[0].to(attr.scalar_type()).contiguous();
+        Tensor g_pos = torch::empty_like(pos), g_M = torch::zeros_like(M), g_attr = torch::empty_like(attr);
+        const int64_t npx = (int64_t)s.C * s.H * s.W, parts = vkgv_diff::render_parts(s.C, s.I);
+        Tensor contrib = torch::empty({ std::max<int64_t>(npx * 3 * (3 + s.A), 1) }, attr.options());
+        const int64_t scratch = parts > 1 ? parts * s.V : 0;
+        Tensor part_pos = torch::empty({ std::max<int64_t>(scratch * 3, 1) }, pos.options());
+        Tensor part_attr = torch::empty({ std::max<int64_t>(scratch * s.A, 1) }, attr.options());
+        const auto adj = adjacency(tris, s.V);
+        dispatch_real(pos, attr, [&](auto cc, auto r) {
+            using C = decltype(cc);
+            using R = decltype(r);
+            vkgv_diff::render_bwd(pos.data_ptr<C>(), M.data_ptr<C>(), attr.data_ptr<R>(), tris.data_ptr<int>(), s.C, s.I,
+                                  s.V, s.T, s.H, s.W, s.A, clip.data_ptr<C>(), box_ptr(boxes), vis.data_ptr<uint8_t>(),
+                                  ids.data_ptr<int>(), depth.data_ptr<float>(), color.data_ptr<R>(),
+                                  adj.first.data_ptr<int>(), adj.second.data_ptr<int>(), g_out.data_ptr<R>(),
+                                  contrib.data_ptr<R>(), part_pos.data_ptr<C>(), part_attr.data_ptr<R>(),
+                                  g_pos.data_ptr<C>(), g_M.data_ptr<C>(), g_attr.data_ptr<R>(), stream());
+        });
+        return { g_pos, g_M, g_attr, Tensor(), Tensor(), Tensor() };
+    }
+};
+
+std::vector<Tensor> render(Tensor pos, Tensor A, Tensor attr, Tensor tris, int64_t H, int64_t W)
+{
+    return RenderFn::apply(pos, A, attr, tris, H, W);
 }
 
 Tensor interpolate(Tensor clip, Tensor attr, Tensor tris, Tensor ids)
@@ -399,5 +486,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("rasterize", &rasterize, "triangle raster -> (ids, depth); no gradient");
     m.def("interpolate", &interpolate, "perspective-correct interpolation of per-vertex attributes");
     m.def("antialias", &antialias, "analytic edge antialiasing");
+    m.def("render", &render, "(image, ids, depth): transform, rasterize and shade as one function of the mesh");
     m.def("shade", &shade, "antialias(interpolate(clip, attr, tris, ids), clip, tris, ids, depth) with one backward");
 }

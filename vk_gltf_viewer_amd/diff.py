@@ -48,8 +48,12 @@ def clip_positions(pos, xforms, view_projs):
     """pos [V, 3], xforms [I, 4, 4], view_projs [C, 4, 4] (row-major, column
     vectors) -> clip [C, I, V, 4], by the extension's vertex-transform
     kernels (gradients to positions and to both matrix sets)."""
-    A = (view_projs[:, None, :, :, None] * xforms[None, :, None, :, :]).sum(-2)   # VP_c M_i, [C, I, 4, 4]
-    return ext().transform(pos.contiguous(), A.contiguous())
+    return ext().transform(pos.contiguous(), _matrices(xforms, view_projs))
+
+
+def _matrices(xforms, view_projs):
+    """VP_c M_i, [C, I, 4, 4] contiguous."""
+    return (view_projs[:, None, :, :, None] * xforms[None, :, None, :, :]).sum(-2).contiguous()
 
 
 PRECISIONS = ("float32", "mixed", "float64")
@@ -76,14 +80,14 @@ def render(pos, attr, tris, xforms, view_projs, height: int, width: int, antiali
         raise ValueError(f"precision must be one of {PRECISIONS}")
     cdt = torch.float32 if precision == "float32" else torch.float64
     adt = torch.float64 if precision == "float64" else torch.float32
+    attr = attr.to(adt).contiguous()
+    if antialias:   # transform, raster and shading as one function: no clip gradient in between
+        img, ids, depth = e.render(pos.to(cdt).contiguous(), _matrices(xforms.to(cdt), view_projs.to(cdt)), attr, tris,
+                                   height, width)
+        return img, ids, depth
     clip = clip_positions(pos.to(cdt), xforms.to(cdt), view_projs.to(cdt))
     ids, depth = e.rasterize(clip.detach().float().contiguous(), tris, height, width, False)
-    attr = attr.to(adt).contiguous()
-    if antialias:   # interpolation and antialiasing as one function: one backward vertex pass
-        img = e.shade(clip, attr, tris, ids, depth)
-    else:
-        img = e.interpolate(clip, attr, tris, ids)
-    return img, ids, depth
+    return e.interpolate(clip, attr, tris, ids), ids, depth
 
 
 @dataclass
