@@ -522,6 +522,7 @@ int vkgv_create(const vkgv_create_info* info, vkgv_ctx** out)
     if (hipGetDeviceProperties(&prop, c->device) == hipSuccess && prop.multiProcessorCount > 0)
         c->cus = prop.multiProcessorCount;
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) { delete c; return VKGV_ERROR_HIP; }
+    read_back_user(true);
     SrgbTables tab;
     std::memset(&tab, 0, sizeof tab);
     srgb_thresholds(tab.thr);
@@ -612,6 +613,7 @@ void vkgv_destroy(vkgv_ctx* c)
                        &c->an_trs, &c->an_chain_first, &c->an_chain })
         dfree(*b);
     (void)hipStreamDestroy(c->stream);
+    read_back_user(false);
     delete c;
 }
 
@@ -1127,7 +1129,7 @@ int vkgv_read_transforms(vkgv_ctx* c, float* mat4s, uint32_t count)
     if (count && !mat4s) return fail(c, VKGV_ERROR_INVALID_ARGUMENT, "read_transforms: null destination");
     HIP_TRY(c, hipSetDevice(c->device));
     HIP_TRY(c, hipDeviceSynchronize());   // updates may run on any stream
-    if (count) HIP_TRY(c, hipMemcpy(mat4s, c->transforms.p, sizeof(float) * 16 * (size_t)count, hipMemcpyDeviceToHost));
+    if (count) HIP_TRY(c, read_back(mat4s, c->transforms.p, sizeof(float) * 16 * (size_t)count, c->stream));
     return VKGV_OK;
 }
 
@@ -1349,9 +1351,9 @@ static int copy_out(vkgv_ctx* c, vkgv_view* v, void* dst, const void* src, size_
     if (rc) return rc;
     if (!dst) return fail(c, VKGV_ERROR_INVALID_ARGUMENT, "readback: null destination");
     HIP_TRY(c, hipSetDevice(c->device));
-    if ((rc = sync_view(c, v))) return rc;
-    HIP_TRY(c, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    // the copies follow the context stream's own work; another stream's frame is waited for
+    if (v->last_stream && v->last_stream != c->stream) HIP_TRY(c, hipStreamSynchronize(v->last_stream));
+    HIP_TRY(c, read_back(dst, src, bytes, c->stream));
     return VKGV_OK;
 }
 

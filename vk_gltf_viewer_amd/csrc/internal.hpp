@@ -372,6 +372,13 @@ struct MeshCheck {
 hipError_t launch_check_meshes(const MeshCheck* meshes, uint32_t mesh_count, uint64_t meshlets, const uint32_t* vidx,
                                const uint8_t* tri, const uint8_t* ml, unsigned long long* bad, hipStream_t st);
 
+// Device to host copy on stream st, after its work and complete on return
+// (readback.hip); reads of kReadStaged bytes and more go through a pinned
+// stage.  read_back_user(true / false): a context that may read joins / leaves.
+constexpr size_t kReadStaged = 64u << 10;
+hipError_t read_back(void* dst, const void* src, size_t bytes, hipStream_t st);
+void read_back_user(bool joins);
+
 // Calibration (calib.hip): 64-bit atomicMin throughput on a 3840 x 2160 key
 // buffer of calib_key_count() keys, coalesced or scattered; 0 on success.
 int measure_atomic_rate(unsigned long long* keys, uint32_t cus, uint32_t scattered, hipStream_t st, double* rate);
