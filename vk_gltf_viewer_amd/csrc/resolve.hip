@@ -107,17 +107,22 @@ __device__ __forceinline__ float half_bits_to_float(uint32_t h)
     return __uint_as_float(bits);
 }
 
-// Texel index of integer coordinate k under a wrap mode.
-__device__ __forceinline__ uint32_t wrap_texel(long long k, uint32_t n, uint32_t mode)
+// Texel indices i0 of integer coordinate k and i1 of k + 1 under a wrap mode;
+// |k| <= 2^30, n <= 16384.  One 32-bit remainder an axis: i1 follows from i0
+// (four 64-bit ones a pixel took most of the textured resolve).
+__device__ __forceinline__ void wrap_texels(int k, int n, uint32_t mode, uint32_t& i0, uint32_t& i1)
 {
-    if (mode == VKGV_WRAP_CLAMP_TO_EDGE) return (uint32_t)(k < 0 ? 0 : (k >= (long long)n ? n - 1 : k));
-    if (mode == VKGV_WRAP_MIRRORED_REPEAT) {
-        long long m = k % (2ll * n);
-        if (m < 0) m += 2ll * n;
-        return (uint32_t)(m < (long long)n ? m : 2ll * n - 1 - m);
+    if (mode == VKGV_WRAP_CLAMP_TO_EDGE) {
+        i0 = (uint32_t)min(max(k, 0), n - 1);
+        i1 = (uint32_t)min(max(k + 1, 0), n - 1);
+        return;
     }
-    long long r = k % (long long)n;
-    return (uint32_t)(r < 0 ? r + n : r);
+    const int period = mode == VKGV_WRAP_MIRRORED_REPEAT ? 2 * n : n;
+    int m0 = k % period;
+    m0 += m0 < 0 ? period : 0;
+    const int m1 = m0 + 1 == period ? 0 : m0 + 1;
+    i0 = (uint32_t)(m0 < n ? m0 : period - 1 - m0);   // the second half of a mirrored period runs back
+    i1 = (uint32_t)(m1 < n ? m1 : period - 1 - m1);
 }
 
 // Bilinear footprint along one axis: texels i0, i1 and the weight of i1.
@@ -128,9 +133,7 @@ __device__ __forceinline__ float texel_pair(float u, uint32_t n, uint32_t mode, 
     if (!(x == x)) x = 0.0f;
     x = x < -1073741824.0f ? -1073741824.0f : (x > 1073741824.0f ? 1073741824.0f : x);
     const float fl = floorf(x);
-    const long long k = (long long)fl;
-    i0 = wrap_texel(k, n, mode);
-    i1 = wrap_texel(k + 1, n, mode);
+    wrap_texels((int)fl, (int)n, mode, i0, i1);
     return x - fl;
 }
 
