@@ -67,7 +67,7 @@ struct vkgv_ctx {
     DevBuf prev_transforms;          // the transforms the last update replaced (motion vectors)
     uint32_t prev_count = 0;
     // node hierarchy and animations (vkgv_set_hierarchy)
-    DevBuf an_nodes, an_chan_first, an_channels, an_samplers, an_times, an_values, an_trs, an_chain_first, an_chain;
+    DevBuf an_channels, an_times, an_values, an_trs, an_chain_first, an_chain;
     AnimDev anim{};
     bool anim_set = false;
     int64_t max_albedo_index = -1;   // largest texture handle a material names (-1: none)
@@ -609,8 +609,7 @@ void vkgv_destroy(vkgv_ctx* c)
     dfree(c->prims); dfree(c->materials); dfree(c->cone_base); dfree(c->cones);
     dfree(c->draws); dfree(c->cull); dfree(c->rrec); dfree(c->transforms); dfree(c->srgb);
     dfree(c->srgb_decode); dfree(c->tex_recs); dfree(c->texels); dfree(c->mat_tex); dfree(c->prev_transforms);
-    for (DevBuf* b : { &c->an_nodes, &c->an_chan_first, &c->an_channels, &c->an_samplers, &c->an_times, &c->an_values,
-                       &c->an_trs, &c->an_chain_first, &c->an_chain })
+    for (DevBuf* b : { &c->an_channels, &c->an_times, &c->an_values, &c->an_trs, &c->an_chain_first, &c->an_chain })
         dfree(*b);
     (void)hipStreamDestroy(c->stream);
     read_back_user(false);
@@ -1015,7 +1014,6 @@ int vkgv_set_hierarchy(vkgv_ctx* c, const vkgv_node* nodes, uint32_t node_count,
             || a.interpolation > VKGV_INTERP_CUBICSPLINE)
             return fail(c, VKGV_ERROR_INVALID_ARGUMENT, "set_hierarchy: sampler " + std::to_string(sp) + " is malformed");
     }
-    std::vector<uint32_t> per_node(node_count + 1, 0);
     for (uint32_t k = 0; k < channel_count; ++k) {
         const vkgv_anim_channel& ch = channels[k];
         if (ch.node >= node_count || ch.sampler >= sampler_count || ch.path > VKGV_PATH_SCALE)
@@ -1025,14 +1023,27 @@ int vkgv_set_hierarchy(vkgv_ctx* c, const vkgv_node* nodes, uint32_t node_count,
         const uint64_t outs = (uint64_t)a.input_count * (a.interpolation == VKGV_INTERP_CUBICSPLINE ? 3u : 1u);
         if ((uint64_t)a.output_offset + outs * comps > value_count)
             return fail(c, VKGV_ERROR_INVALID_ARGUMENT, "set_hierarchy: channel " + std::to_string(k) + " reads past the values");
-        per_node[ch.node + 1]++;
     }
-    // channels grouped by node, in array order within a node
-    for (uint32_t n = 0; n < node_count; ++n) per_node[n + 1] += per_node[n];
-    std::vector<vkgv_anim_channel> grouped(std::max<uint32_t>(channel_count, 1u));
-    {
-        std::vector<uint32_t> fill(per_node.begin(), per_node.end() - 1);
-        for (uint32_t k = 0; k < channel_count; ++k) grouped[fill[channels[k].node]++] = channels[k];
+    // the last channel of each node and path wins: the device samples only that one
+    std::vector<uint32_t> winner(3 * (size_t)node_count, ~0u);
+    for (uint32_t k = 0; k < channel_count; ++k) winner[3 * (size_t)channels[k].node + channels[k].path] = k;
+    std::vector<AnimChan> chans;
+    for (uint32_t k : winner) {
+        if (k == ~0u) continue;
+        const vkgv_anim_sampler& a = samplers[channels[k].sampler];
+        chans.push_back({ channels[k].node, channels[k].path | (a.interpolation << 8), a.input_offset, a.input_count,
+                          a.output_offset, times[a.input_offset + a.input_count - 1], {} });
+    }
+    // rotations together and by interpolation: a wave runs one kind of sampling
+    std::stable_sort(chans.begin(), chans.end(), [](const AnimChan& x, const AnimChan& y) {
+        auto key = [](uint32_t kind) { return ((kind & 0xFFu) == VKGV_PATH_ROTATION ? 0x100u : 0u) | (kind >> 8); };
+        return key(x.kind) < key(y.kind);
+    });
+    std::vector<NodeTrs> trs(std::max<uint32_t>(node_count, 1u));
+    for (uint32_t n = 0; n < node_count; ++n) {
+        std::memcpy(trs[n].t, nodes[n].translation, sizeof trs[n].t);
+        std::memcpy(trs[n].q, nodes[n].rotation, sizeof trs[n].q);
+        std::memcpy(trs[n].s, nodes[n].scale, sizeof trs[n].s);
     }
     // depth-first walk of the roots (World::iterateNode order, as vkgv_world_build):
     // every mesh node takes the next transform and records its root-to-node chain
@@ -1074,22 +1085,16 @@ int vkgv_set_hierarchy(vkgv_ctx* c, const vkgv_node* nodes, uint32_t node_count,
     HIP_TRY(c, hipDeviceSynchronize());   // updates of any stream may still read the old arrays
     c->anim_set = false;
     int rc;
-    if ((rc = upload(c, c->an_nodes, nodes, sizeof(vkgv_node) * node_count))) return rc;
-    if ((rc = upload(c, c->an_chan_first, per_node.data(), sizeof(uint32_t) * per_node.size()))) return rc;
-    if ((rc = upload(c, c->an_channels, grouped.data(), sizeof(vkgv_anim_channel) * channel_count))) return rc;
-    if ((rc = upload(c, c->an_samplers, samplers, sizeof(vkgv_anim_sampler) * sampler_count))) return rc;
+    if ((rc = upload(c, c->an_channels, chans.data(), sizeof(AnimChan) * chans.size()))) return rc;
     if ((rc = upload(c, c->an_times, times, sizeof(float) * time_count))) return rc;
     if ((rc = upload(c, c->an_values, values, sizeof(float) * value_count))) return rc;
-    if ((rc = dalloc(c, c->an_trs, sizeof(NodeTrs) * std::max<uint32_t>(node_count, 1u)))) return rc;
+    if ((rc = upload(c, c->an_trs, trs.data(), sizeof(NodeTrs) * trs.size()))) return rc;
     if ((rc = upload(c, c->an_chain_first, chain_first.data(), sizeof(uint32_t) * chain_first.size()))) return rc;
     if ((rc = upload(c, c->an_chain, chain.data(), sizeof(uint32_t) * chain.size()))) return rc;
     HIP_TRY(c, hipStreamSynchronize(c->stream));
     AnimDev& d = c->anim;
-    d.nodes = static_cast<const vkgv_node*>(c->an_nodes.p);
-    d.node_count = node_count;
-    d.chan_first = static_cast<const uint32_t*>(c->an_chan_first.p);
-    d.channels = static_cast<const vkgv_anim_channel*>(c->an_channels.p);
-    d.samplers = static_cast<const vkgv_anim_sampler*>(c->an_samplers.p);
+    d.channels = static_cast<const AnimChan*>(c->an_channels.p);
+    d.channel_count = (uint32_t)chans.size();
     d.times = static_cast<const float*>(c->an_times.p);
     d.values = static_cast<const float*>(c->an_values.p);
     d.trs = static_cast<NodeTrs*>(c->an_trs.p);
@@ -1099,7 +1104,7 @@ int vkgv_set_hierarchy(vkgv_ctx* c, const vkgv_node* nodes, uint32_t node_count,
     // the transform buffer holds the mesh nodes' matrices at time 0 (no previous frame yet)
     if ((rc = reserve_transforms(c, mesh_count, c->stream))) return rc;
     c->prev_count = 0;
-    launch_update_transforms(d, 0.0f, static_cast<float*>(c->transforms.p), c->stream);
+    launch_update_transforms(d, 0.0f, static_cast<float*>(c->transforms.p), nullptr, c->stream);
     HIP_TRY(c, hipGetLastError());
     if ((rc = finish_transforms(c, mesh_count, c->stream))) return rc;
     HIP_TRY(c, hipStreamSynchronize(c->stream));
@@ -1115,9 +1120,8 @@ int vkgv_update_transforms(vkgv_ctx* c, float time, void* stream)
         return fail(c, VKGV_ERROR_STATE, "update_transforms: the transforms were replaced since set_hierarchy");
     HIP_TRY(c, hipSetDevice(c->device));
     hipStream_t st = stream ? static_cast<hipStream_t>(stream) : c->stream;
-    const size_t bytes = sizeof(float) * 16 * (size_t)c->anim.mesh_count;
-    if (bytes) HIP_TRY(c, hipMemcpyAsync(c->prev_transforms.p, c->transforms.p, bytes, hipMemcpyDeviceToDevice, st));
-    launch_update_transforms(c->anim, time, static_cast<float*>(c->transforms.p), st);
+    launch_update_transforms(c->anim, time, static_cast<float*>(c->transforms.p),
+                             static_cast<float*>(c->prev_transforms.p), st);
     HIP_TRY(c, hipGetLastError());
     return VKGV_OK;
 }

@@ -41,16 +41,24 @@ static_assert(sizeof(RasterRec) == 32, "RasterRec layout");
 // Animated TRS of one node for the device transform update.
 struct NodeTrs { float t[3], q[4], s[3]; };
 
+// One animation channel with its sampler, as the device update reads it.
+struct AnimChan {
+    uint32_t node;
+    uint32_t kind;                       // path | interpolation << 8
+    uint32_t input_offset, input_count;  // key times
+    uint32_t output_offset;              // first output value
+    float last;                          // the last key time
+    uint32_t pad[2];
+};
+static_assert(sizeof(AnimChan) == 32, "AnimChan layout");
+
 // Node hierarchy and animations on the device (vkgv_set_hierarchy).
 struct AnimDev {
-    const vkgv_node* nodes;
-    uint32_t node_count;
-    const uint32_t* chan_first;          // node_count + 1: the node's channels, in application order
-    const vkgv_anim_channel* channels;
-    const vkgv_anim_sampler* samplers;
+    const AnimChan* channels;            // at most one per node and path, grouped by kind
+    uint32_t channel_count;
     const float* times;
     const float* values;
-    NodeTrs* trs;                        // per node, this update
+    NodeTrs* trs;                        // per node: its static TRS, the animated parts of this update
     uint32_t mesh_count;                 // mesh nodes = transforms
     const uint32_t* chain_first;         // mesh_count + 1
     const uint32_t* chain_nodes;         // root-to-node chain of each mesh node
@@ -326,8 +334,9 @@ struct BatchGrid {
 enum CullMode : uint32_t { CULL_SINGLE = 0, CULL_EARLY = 1, CULL_LATE = 2 };
 
 // ---- launchers (stream-ordered, no host synchronization) -----------------
-// Animation sampling and world matrices of the mesh nodes into `transforms`.
-void launch_update_transforms(const AnimDev& d, float time, float* transforms, hipStream_t st);
+// Animation sampling and world matrices of the mesh nodes into `transforms`;
+// the matrices they replace go to `prev` unless it is null.
+void launch_update_transforms(const AnimDev& d, float time, float* transforms, float* prev, hipStream_t st);
 void launch_build_cull_records(const SceneDev& s, CullRec* out, RasterRec* rrec, hipStream_t st);
 void launch_clear_keys(unsigned long long* keys, uint64_t n, hipStream_t st);
 // Frame start of every view of the batch: all counters zeroed, keys cleared,
