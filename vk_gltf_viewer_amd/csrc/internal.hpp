@@ -319,6 +319,30 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Inclusive scans over the wave's 64 lanes by DPP moves: within rows of 16,
+// then the rows' last lanes broadcast to the following rows.  Six vector
+// instructions; __shfl_up takes six trips through the LDS crossbar.
+template <typename F> __device__ __forceinline__ uint32_t wave_scan(uint32_t x, F f)
+{
+#define VKGV_SCAN_STEP(ctrl, rows) x = f(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, ctrl, rows, 0xF, false))
+    VKGV_SCAN_STEP(0x111, 0xF);   // row_shr 1, 2, 4, 8
+    VKGV_SCAN_STEP(0x112, 0xF);
+    VKGV_SCAN_STEP(0x114, 0xF);
+    VKGV_SCAN_STEP(0x118, 0xF);
+    VKGV_SCAN_STEP(0x142, 0xA);   // row_bcast15 into rows 1 and 3
+    VKGV_SCAN_STEP(0x143, 0xC);   // row_bcast31 into rows 2 and 3
+#undef VKGV_SCAN_STEP
+    return x;
+}
+__device__ __forceinline__ uint32_t wave_scan_add(uint32_t x)
+{
+    return wave_scan(x, [](uint32_t a, uint32_t b) { return a + b; });
+}
+__device__ __forceinline__ uint32_t wave_scan_max(uint32_t x)   // lanes without a source take 0
+{
+    return wave_scan(x, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
+}
+
 constexpr uint32_t kMvpStride = 20;          // floats per transform in a view's VP M table (80-byte rows)
 constexpr uint32_t kHizMaxLevels = 16;
 constexpr uint32_t kHizTailTexels = 8192;   // largest first tail level (the tail keeps it in LDS)

@@ -416,36 +416,30 @@ __device__ __forceinline__ bool push_big(const TriSetup& t, uint32_t id, const B
     return store_big(t, id, slot, c0, chunks, q);
 }
 
-// Wave-wide append (called by all 64 lanes): a prefix sum of the lanes'
-// (1, chunks) pairs and one atomic per counter and wave reserve consecutive
-// slots and chunks in lane order.  A lane's chunk count is at most the chunk
+// Wave-wide append (called by all 64 lanes): the lanes' ranks, a prefix sum of
+// their chunks and one atomic per counter and wave reserve consecutive slots
+// and chunks in lane order.  A lane's chunk count is at most the chunk
 // list's chunk capacity (below 2^19), so the 64-lane sums fit their 32-bit
 // halves.  Returns true on a lane whose triangle found no room.
 __device__ __forceinline__ bool push_big_wave(bool want, const TriSetup& t, uint32_t id, uint32_t lane,
                                               const BigQueue& q)
 {
+    const unsigned long long wanting = __ballot(want);
+    if (wanting == 0ull) return false;   // wave-uniform; most meshlets have none
     const uint32_t chunks = want ? reserve_chunks(t, q.chunk_cap) : 0u;
-    const unsigned long long mine = want ? ((1ull << 32) | (unsigned long long)chunks) : 0ull;
-    unsigned long long x = mine;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const unsigned long long y = __shfl_up(x, off);
-        if (lane >= (uint32_t)off) x += y;
-    }
-    const unsigned long long total = __shfl(x, 63);
-    if (total == 0ull) return false;   // wave-uniform
+    const uint32_t incl = wave_scan_add(chunks);
+    const uint32_t nwant = (uint32_t)__popcll(wanting), nchunk = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
     // slot base << 32 | chunk base (saturated: a base past the list fails either way)
     unsigned long long base = 0ull;
     if (lane == 0) {
-        const uint32_t sb = atomicAdd(&q.ctr->big_count, (uint32_t)(total >> 32));
-        const unsigned long long cb =
-            (uint32_t)total ? atomicAdd(&q.ctr->big_chunks, (unsigned long long)(uint32_t)total) : 0ull;
+        const uint32_t sb = atomicAdd(&q.ctr->big_count, nwant);
+        const unsigned long long cb = nchunk ? atomicAdd(&q.ctr->big_chunks, (unsigned long long)nchunk) : 0ull;
         base = ((unsigned long long)sb << 32) | (cb < 0xFFFFFFFFull ? cb : 0xFFFFFFFFull);
     }
     base = __shfl(base, 0);
-    const unsigned long long before = x - mine;
-    return want && !store_big(t, id, (uint32_t)(base >> 32) + (uint32_t)(before >> 32),
-                              (base & 0xFFFFFFFFull) + (uint32_t)before, chunks, q);
+    const uint32_t before = __builtin_amdgcn_mbcnt_hi((uint32_t)(wanting >> 32),
+                                                      __builtin_amdgcn_mbcnt_lo((uint32_t)wanting, 0u));
+    return want && !store_big(t, id, (uint32_t)(base >> 32) + before, (base & 0xFFFFFFFFull) + (incl - chunks), chunks, q);
 }
 
 // Clipping (rare): Sutherland-Hodgman against pa*x + pb*y + pc*z + pd*w >= 0.
@@ -530,6 +524,14 @@ __device__ __forceinline__ bool fan_setup(const Poly p, int f, float hw, float h
     return setup_tri(s0, s1, s2, W, H, t);
 }
 
+// The three vertex bytes of triangle t (byte 3 t on), in the low 24 bits of
+// one word: two words and a shift.  `words` has one word past the last used.
+__device__ __forceinline__ uint32_t tri_bytes(const uint32_t* words, uint32_t t)
+{
+    const uint32_t b = 3u * t, w = b >> 2;
+    return __builtin_amdgcn_alignbyte(words[w + 1u], words[w], b & 3u);
+}
+
 __device__ __forceinline__ uint32_t tri_byte(const uint32_t* words, uint32_t b)
 {
     return (words[b >> 2] >> ((b & 3u) * 8u)) & 0xFFu;
@@ -542,28 +544,44 @@ constexpr uint32_t kStageTri4 = kStageTriWords / 4;                 // the trian
 static_assert(kStageTriWords % 4 == 0, "the staged triangles are copied 16 bytes at a time");
 static_assert(kStageTriWords + 128u + 4u <= kFragStageWords, "a staged meshlet fits its record");
 
-// Pixel slots [k, kend) of a meshlet's small triangles (tri[] staged setups,
-// pre[] the 128-entry exclusive prefix of their bounding-box pixel counts,
-// `total` their sum), walked by one lane: one search finds the triangle of
-// the first slot, then the lane walks the run with integer edge steps and
-// moves to the next triangle when the run crosses a triangle's start (no
-// search per pixel).  Covered centres with 0 <= z <= 1 update the
-// visibility buffer with a 64-bit atomicMin.
-template <bool STATS>
-__device__ __forceinline__ void walk_small(const SmallTri* tri, const uint32_t* pre, uint32_t total, uint32_t k,
-                                           uint32_t kend, unsigned long long* keys, uint32_t W, RasterCount<STATS>& rc)
+// Last triangle whose first slot is <= k.
+__device__ __forceinline__ uint32_t slot_triangle(const uint32_t* pre, uint32_t k)
 {
-    if (k >= kend) return;
-    uint32_t lo = 0, hi = 127;   // last triangle whose first slot is <= k
+    uint32_t lo = 0, hi = 127;
     while (lo < hi) {
         const uint32_t mid = (lo + hi + 1u) >> 1;
         if (pre[mid] <= k) lo = mid; else hi = mid - 1u;
     }
+    return lo;
+}
+
+// n / d by the hardware reciprocal, exact for n < 2^20 (a meshlet's slots are at
+// most 124 x 65^2, and a lane's share of them less): (n + 1/2) / d lies at least
+// 1 / (2 d) from an integer, and the reciprocal's and the product's roundings
+// move it by less than (n + 1/2) / d x 2^-22 < 1 / (4 d).
+__device__ __forceinline__ uint32_t small_div(uint32_t n, uint32_t d)
+{
+    return (uint32_t)(((float)n + 0.5f) * __builtin_amdgcn_rcpf((float)d));
+}
+
+// Pixel slots [k, kend) of a meshlet's small triangles (tri[] staged setups,
+// pre[] the 128-entry exclusive prefix of their bounding-box pixel counts,
+// `total` their sum), walked by one lane from triangle lo, the one that holds
+// slot k: the lane walks the run with integer edge steps and moves to the next
+// triangle when the run crosses a triangle's start (no search per pixel).
+// Covered centres with 0 <= z <= 1 update the visibility buffer with a 64-bit
+// atomicMin.
+template <bool STATS>
+__device__ __forceinline__ void walk_small(const SmallTri* tri, const uint32_t* pre, uint32_t total, uint32_t lo,
+                                           uint32_t k, uint32_t kend, unsigned long long* keys, uint32_t W,
+                                           RasterCount<STATS>& rc)
+{
+    if (k >= kend) return;
     uint32_t next = lo < 127u ? pre[lo + 1u] : total;
     SmallTriR st = load_small(tri[lo]);
     uint32_t bw = st.bw;
     const uint32_t r = k - pre[lo];
-    int jj = (int)(r / bw), ii = (int)(r - (uint32_t)jj * bw);
+    int jj = (int)small_div(r, bw), ii = (int)(r - (uint32_t)jj * bw);
     int e0 = st.C[0] + st.A[0] * ii + st.B[0] * jj;
     int e1 = st.C[1] + st.A[1] * ii + st.B[1] * jj;
     int e2 = st.C[2] + st.A[2] * ii + st.B[2] * jj;
@@ -602,16 +620,22 @@ __device__ __forceinline__ void walk_small(const SmallTri* tri, const uint32_t* 
 
 // One view's share of the meshlet raster (wave w of the grid takes meshlets
 // w, w + waves, ... of the view's list).
+// Bound by vector instructions where meshlets are many (views up to 3840x2160 of
+// sub-pixel triangles: VALU 63% busy, 795 instructions a meshlet and wave) and by
+// the cache's stores where most triangles face away.  Scans and searches on
+// DPP moves instead of LDS round trips: 4417 -> 3561 us there, 16.5 -> 12.0 us for
+// one 640x360 frame.
 template <bool STATS>
 __device__ __forceinline__ void raster_view(const RasterArgs& a)
 {
     RasterCount<STATS> rc;
     __shared__ float4 s_clip[kWaves][64];
     __shared__ SVtx s_sv[kWaves][64];
-    __shared__ uint32_t s_tri[kWaves][96];
+    __shared__ uint32_t s_tri[kWaves][97];   // a word past the 93 of 124 triangles is read (and not used)
     __shared__ __align__(16) SmallTri s_st[kWaves][VKGV_MESHLET_TRIANGLES];
     __shared__ __align__(16) uint32_t s_pre[kWaves][128];
     __shared__ uint32_t s_list[kWaves][128];   // the meshlet's triangles past the per-slot tests
+    __shared__ uint32_t s_own[kWaves][64];     // triangle of each lane's first pixel slot
 
     const int w = threadIdx.x >> 6;
     const uint32_t lane = threadIdx.x & 63u;
@@ -737,8 +761,8 @@ __device__ __forceinline__ void raster_view(const RasterArgs& a)
         r2 = rec_word(nidx + 2u * nwaves);
         wave_sync();
 
-        // Stage 1, every triangle slot: the resolve cache, the back-face test
-        // and setup_tri's pixel-range test (a projected triangle whose
+        // Stage 1, every triangle slot: the resolve cache, back-face test and setup_tri's
+        // pixel-range test (a projected triangle whose
         // bounding box holds no pixel centre rasterizes nothing).  The
         // triangles left (and those that need clipping) are packed into
         // s_list (t | i0 << 8 | i1 << 16 | i2 << 24), so that the setup below
@@ -752,8 +776,8 @@ __device__ __forceinline__ void raster_view(const RasterArgs& a)
             bool live = false;
             uint32_t packed = 0u;
             if (t < tc) {
-                const uint32_t i0 = tri_byte(s_tri[w], 3u * t), i1 = tri_byte(s_tri[w], 3u * t + 1u),
-                               i2 = tri_byte(s_tri[w], 3u * t + 2u);
+                const uint32_t tb = tri_bytes(s_tri[w], t);
+                const uint32_t i0 = tb & 0xFFu, i1 = (tb >> 8) & 0xFFu, i2 = (tb >> 16) & 0xFFu;
                 const float4 c0 = s_clip[w][i0], c1 = s_clip[w][i1], c2 = s_clip[w][i2];
                 if (cached && bary) {
                     // TriCache: r[k] = v_{k+1} x v_{k+2} over the clip (x, y, w) of the
@@ -774,7 +798,6 @@ __device__ __forceinline__ void raster_view(const RasterArgs& a)
                     gstore(dst + 2, make_uint4(__float_as_uint(r22), s_col[w][i0], s_col[w][i1], s_col[w][i2]));
                     if (tex) gstore(dst + 3, make_uint4(s_uv[w][i0], s_uv[w][i1], s_uv[w][i2], 0u));
                 }
-                static_assert(offsetof(TriCache, col) == 36 && offsetof(TriCache, uv) == 48, "TriCache words");
                 live = true;
                 if (cull_faces) {
                     const float det = det3_xyw(c0, c1, c2);
@@ -790,7 +813,7 @@ __device__ __forceinline__ void raster_view(const RasterArgs& a)
                                && max((miny - 128 + 255) >> 8, 0) <= min((maxy - 128) >> 8, H - 1);
                     }
                 }
-                packed = t | (i0 << 8) | (i1 << 16) | (i2 << 24);
+                packed = t | (tb << 8);
             }
             const unsigned long long m = __ballot(live);
             const uint32_t pos = nlive + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
@@ -814,6 +837,7 @@ __device__ __forceinline__ void raster_view(const RasterArgs& a)
                 const uint32_t e = s_list[w][pos];
                 const uint32_t t = e & 0xFFu, i0 = (e >> 8) & 0xFFu, i1 = (e >> 16) & 0xFFu, i2 = e >> 24;
                 id = (d << VKGV_TRIANGLE_BITS) | t;
+                static_assert(offsetof(TriCache, col) == 36 && offsetof(TriCache, uv) == 48, "TriCache words");
                 const SVtx v0 = s_sv[w][i0], v1 = s_sv[w][i1], v2 = s_sv[w][i2];
                 if (!(v0.ok & v1.ok & v2.ok)) {
                     const uint32_t slot = atomicAdd(&a.ctr->clip_count, 1u);
@@ -862,16 +886,17 @@ __device__ __forceinline__ void raster_view(const RasterArgs& a)
         }
 
         // exclusive prefix of pixel counts over the 128 triangle slots
-        uint32_t x0 = npix[0], x1 = npix[1];
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const uint32_t y0 = __shfl_up(x0, off), y1 = __shfl_up(x1, off);
-            if (lane >= (uint32_t)off) { x0 += y0; x1 += y1; }
+        const uint32_t x0 = wave_scan_add(npix[0]);
+        const uint32_t tot0 = (uint32_t)__builtin_amdgcn_readlane((int)x0, 63);
+        uint32_t pre0 = x0 - npix[0], pre1 = tot0, total = tot0;
+        if (nlive > 64u) {   // wave-uniform
+            const uint32_t x1 = wave_scan_add(npix[1]);
+            pre1 = tot0 + x1 - npix[1];
+            total += (uint32_t)__builtin_amdgcn_readlane((int)x1, 63);
         }
-        const uint32_t tot0 = __shfl(x0, 63), tot1 = __shfl(x1, 63);
-        s_pre[w][lane] = x0 - npix[0];
-        s_pre[w][64 + lane] = tot0 + x1 - npix[1];
-        const uint32_t total = tot0 + tot1;
+        s_pre[w][lane] = pre0;
+        s_pre[w][64 + lane] = pre1;
+        s_own[w][lane] = 0u;
         wave_sync();
 
         // A heavy meshlet keeps the first kJobKeep slots and defers the rest
@@ -904,10 +929,24 @@ __device__ __forceinline__ void raster_view(const RasterArgs& a)
                 keep = kJobKeep;
             }
         }
+        // Lane l walks slots l * per, ...: the triangle that holds lane l's first
+        // slot names itself there if no earlier lane's first slot is in it, and
+        // the lanes after take the last name (a search of the prefix was seven
+        // dependent LDS reads).
         {
             const uint32_t per = (keep + 63u) >> 6;
-            const uint32_t k = lane * per;
-            walk_small(s_st[w], s_pre[w], total, k, min(k + per, keep), a.keys, a.W, rc);
+            if (per) {   // wave-uniform
+                const uint32_t l0 = per == 1u ? pre0 : small_div(pre0 + per - 1u, per);
+                if (npix[0] && l0 * per < pre0 + npix[0] && l0 < 64u) s_own[w][l0] = lane;
+                if (nlive > 64u) {
+                    const uint32_t l1 = per == 1u ? pre1 : small_div(pre1 + per - 1u, per);
+                    if (npix[1] && l1 * per < pre1 + npix[1] && l1 < 64u) s_own[w][l1] = 64u + lane;
+                }
+                wave_sync();
+                const uint32_t lo = wave_scan_max(s_own[w][lane]);
+                const uint32_t k = lane * per;
+                walk_small(s_st[w], s_pre[w], total, lo, k, min(k + per, keep), a.keys, a.W, rc);
+            }
         }
         wave_sync();
         // the meshlet is redone by the direct path after this kernel
@@ -1019,7 +1058,7 @@ __device__ __forceinline__ void frag_job(const BigArgs& a, uint32_t j, RasterCou
     const uint32_t end = min(first + kJobSlots, total);
     const uint32_t per = (end - first + 63u) >> 6;
     const uint32_t k = first + lane * per;
-    walk_small(tri, pre, total, k, min(k + per, end), a.keys, a.W, rc);
+    walk_small(tri, pre, total, slot_triangle(pre, min(k, total)), k, min(k + per, end), a.keys, a.W, rc);
 }
 
 // The bin pass's work items: the 64-tile chunks of the big triangles, then
@@ -1481,14 +1520,9 @@ __global__ __launch_bounds__(kBlock, 3) void raster_kernel(RasterBatchArgs ab)
             cnt = c->vis_count[ab.list];
             base = ab.list ? c->vis_count[0] : 0u;
         }
-        // exclusive prefix of the counts over the 64 views, modulo nwaves
-        uint32_t incl = cnt % nwaves;
-#pragma unroll
-        for (uint32_t off = 1; off < 64u; off <<= 1) {
-            const uint32_t y = __shfl_up(incl, off);
-            if (lane >= off) incl = (incl + y) % nwaves;
-        }
-        const uint32_t excl = (incl + nwaves - cnt % nwaves) % nwaves;
+        // exclusive prefix of the counts over the 64 views (at most 2^31), modulo nwaves
+        const uint32_t sum = wave_scan_add(cnt);
+        const uint32_t incl = sum % nwaves, excl = (sum - cnt) % nwaves;
         const uint32_t m = min(64u, ab.b.nviews - v0);
         for (uint32_t j = 0; j < m; ++j) {
             const uint32_t count = __builtin_amdgcn_readlane(cnt, j);
@@ -1665,13 +1699,8 @@ __global__ __launch_bounds__(256) void bin_kernel(BatchDev b, uint32_t pass)
             cnt = nchunks + njobs;
             if (gw == 0 && nbig) atomicAdd(&v.counters->big_total_tris, nbig);
         }
-        uint32_t incl = cnt % nw;
-#pragma unroll
-        for (uint32_t off = 1; off < 64u; off <<= 1) {
-            const uint32_t y = __shfl_up(incl, off);
-            if (lane >= off) incl = (incl + y) % nw;
-        }
-        const uint32_t excl = (incl + nw - cnt % nw) % nw;
+        const uint32_t sum = wave_scan_add(cnt);   // below 2^25
+        const uint32_t incl = sum % nw, excl = (sum - cnt) % nw;
         const uint32_t m = min(64u, b.nviews - v0);
         for (uint32_t j = 0; j < m; ++j) {
             const uint32_t count = __builtin_amdgcn_readlane(cnt, j);
