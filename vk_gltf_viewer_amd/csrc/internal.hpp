@@ -190,7 +190,7 @@ struct Counters {
     unsigned long long fragments;       // covered pixel centres with 0 <= z <= 1 (visibility-buffer updates)
     unsigned long long frag_atomics;    // global 64-bit atomicMin writes of those updates
     unsigned long long frag_stores;     // tile merges written with a plain read-min-store instead
-    // deferred fragment runs of the current pass: staged meshlets << kJobCountBits | jobs reserved
+    // deferred fragment runs of the current pass: staged batches << kJobCountBits | jobs reserved
     unsigned long long frag_jobs;
     unsigned long long pad2[3];
 };
@@ -198,21 +198,25 @@ static_assert(sizeof(Counters) == 128, "Counters layout");
 
 constexpr uint32_t kTileSplit = 8;      // most tile-pass parts sharing one screen tile's triangle list
 
-// Deferred fragment runs.  A meshlet whose small triangles cover more than
+// The meshlet raster sets up and walks batches of 64 triangles.  Deferred
+// fragment runs: a batch whose small triangles cover more than
 // kJobKeep + kJobSlots / 2 pixel slots keeps the first kJobKeep for its own
 // raster wave and hands the rest, kJobSlots at a time, to the bin pass: its
 // triangle setups and slot prefix are staged in a FragStage record (an
-// opaque copy of the raster's LDS arrays, 124 x 52 B + 128 x 4 B + total),
+// opaque copy of the raster's LDS arrays, 64 x 52 B + 64 x 4 B + total),
 // and each job names the record and its first slot.
-constexpr uint32_t kJobKeep = 512;
+constexpr uint32_t kRasterBatch = 64;
+// 256 kept slots a batch: 512 made a heavy meshlet's two batches the longest of
+// the pass (raster of a 1921x1081 frame 17.3 us against 22.3).
+constexpr uint32_t kJobKeep = 256;
 constexpr uint32_t kJobSlots = 256;
-constexpr uint32_t kFragStageWords = 1744;   // 16-byte multiple
+constexpr uint32_t kFragStageWords = 900;    // 16-byte multiple
 struct FragStage {
     uint32_t w[kFragStageWords];
 };
 static_assert(sizeof(FragStage) % 16 == 0, "FragStage records are copied 16 bytes at a time");
-constexpr uint32_t kJobCountBits = 38;           // jobs field of Counters::frag_jobs (at most 2^25 meshlets x 140 jobs)
-constexpr uint32_t kFragStageCapacity = 1024;    // staged meshlets per view and pass (7.1 MB)
+constexpr uint32_t kJobCountBits = 37;           // jobs field of Counters::frag_jobs (at most 2^26 batches x 1057 jobs)
+constexpr uint32_t kFragStageCapacity = 2048;    // staged batches per view and pass (7.4 MB)
 constexpr uint32_t kFragJobCapacity = 1u << 15;  // their jobs per view and pass
 struct FragJob {
     uint32_t stage;                 // FragStage record, ~0u: reserved but unused
@@ -248,7 +252,7 @@ struct ViewDev {
     uint32_t tile_capacity;         // triangles a tile's list holds (the rest take the direct path)
     uint32_t chunk_capacity;        // 64-tile chunks of big triangles per pass
     BigSetup* setups;               // per big triangle
-    FragStage* frag_stage;          // deferred fragment runs: staged meshlets
+    FragStage* frag_stage;          // deferred fragment runs: staged batches
     FragJob* frag_jobs;             // and their jobs
     uint32_t stage_capacity, job_capacity;
     // resolve cache: triangle t of the meshlet in visible-list slot s is

@@ -16,11 +16,12 @@
 // Work split.
 //  raster_kernel  persistent grid of 4-wave blocks; wave g takes visible
 //                 meshlets g, g + waves, ..., transforms its <= 64 vertices into
-//                 LDS, back-face culls its <= 124 triangles (2 per lane) and
+//                 LDS, back-face culls its <= 124 triangles (2 per lane), sets
+//                 the rest up in batches of 64 that may span three meshlets, and
 //                 rasterizes the small ones cooperatively: a wave prefix sum
 //                 over their bounding-box pixel counts gives each lane an equal
 //                 run of pixel slots, walked with integer edge steps (a heavy
-//                 meshlet hands most of its slots to the bin pass as deferred
+//                 batch hands most of its slots to the bin pass as deferred
 //                 runs).  Large triangles go to the big queue (a slot, and the
 //                 64-tile chunks of the triangle's 32x32-pixel bounding-box
 //                 tiles in the chunk list), triangles needing clipping to the
@@ -48,6 +49,7 @@ namespace vkgv {
 namespace {
 
 constexpr int kWaves = 4;
+constexpr uint32_t kGroup = 3;   // meshlets whose triangles share batches in the raster
 constexpr uint32_t kBlock = 64 * kWaves;
 constexpr float kGuardPx = 2097152.0f;       // 2^21 pixels
 constexpr float kClipGuardPx = 1048576.0f;   // guard clip planes at 2^20 pixels
@@ -537,17 +539,17 @@ __device__ __forceinline__ uint32_t tri_byte(const uint32_t* words, uint32_t b)
     return (words[b >> 2] >> ((b & 3u) * 8u)) & 0xFFu;
 }
 
-// Words of a FragStage record: the staged triangles, then the 128-entry slot
+// Words of a FragStage record: a batch's staged triangles, then their slot
 // prefix, then the slot total.
-constexpr uint32_t kStageTriWords = VKGV_MESHLET_TRIANGLES * (uint32_t)(sizeof(SmallTri) / 4);
+constexpr uint32_t kStageTriWords = kRasterBatch * (uint32_t)(sizeof(SmallTri) / 4);
 constexpr uint32_t kStageTri4 = kStageTriWords / 4;                 // the triangles as 16-byte words
 static_assert(kStageTriWords % 4 == 0, "the staged triangles are copied 16 bytes at a time");
-static_assert(kStageTriWords + 128u + 4u <= kFragStageWords, "a staged meshlet fits its record");
+static_assert(kStageTriWords + kRasterBatch + 4u <= kFragStageWords, "a staged batch fits its record");
 
 // Last triangle whose first slot is <= k.
 __device__ __forceinline__ uint32_t slot_triangle(const uint32_t* pre, uint32_t k)
 {
-    uint32_t lo = 0, hi = 127;
+    uint32_t lo = 0, hi = kRasterBatch - 1u;
     while (lo < hi) {
         const uint32_t mid = (lo + hi + 1u) >> 1;
         if (pre[mid] <= k) lo = mid; else hi = mid - 1u;
@@ -555,8 +557,8 @@ __device__ __forceinline__ uint32_t slot_triangle(const uint32_t* pre, uint32_t 
     return lo;
 }
 
-// n / d by the hardware reciprocal, exact for n < 2^20 (a meshlet's slots are at
-// most 124 x 65^2, and a lane's share of them less): (n + 1/2) / d lies at least
+// n / d by the hardware reciprocal, exact for n < 2^20 (a batch's slots are at
+// most 64 x 65^2, and a lane's share of them less): (n + 1/2) / d lies at least
 // 1 / (2 d) from an integer, and the reciprocal's and the product's roundings
 // move it by less than (n + 1/2) / d x 2^-22 < 1 / (4 d).
 __device__ __forceinline__ uint32_t small_div(uint32_t n, uint32_t d)
@@ -564,8 +566,8 @@ __device__ __forceinline__ uint32_t small_div(uint32_t n, uint32_t d)
     return (uint32_t)(((float)n + 0.5f) * __builtin_amdgcn_rcpf((float)d));
 }
 
-// Pixel slots [k, kend) of a meshlet's small triangles (tri[] staged setups,
-// pre[] the 128-entry exclusive prefix of their bounding-box pixel counts,
+// Pixel slots [k, kend) of a batch's small triangles (tri[] staged setups,
+// pre[] the exclusive prefix of their bounding-box pixel counts,
 // `total` their sum), walked by one lane from triangle lo, the one that holds
 // slot k: the lane walks the run with integer edge steps and moves to the next
 // triangle when the run crosses a triangle's start (no search per pixel).
@@ -577,7 +579,7 @@ __device__ __forceinline__ void walk_small(const SmallTri* tri, const uint32_t* 
                                            RasterCount<STATS>& rc)
 {
     if (k >= kend) return;
-    uint32_t next = lo < 127u ? pre[lo + 1u] : total;
+    uint32_t next = lo < kRasterBatch - 1u ? pre[lo + 1u] : total;
     SmallTriR st = load_small(tri[lo]);
     uint32_t bw = st.bw;
     const uint32_t r = k - pre[lo];
@@ -595,8 +597,8 @@ __device__ __forceinline__ void walk_small(const SmallTri* tri, const uint32_t* 
         }
         if (++k >= kend) break;
         if (k == next) {   // first slot of a later triangle (empty ones skipped)
-            while (lo < 127u && pre[lo + 1u] <= k) ++lo;
-            next = lo < 127u ? pre[lo + 1u] : total;
+            while (lo < kRasterBatch - 1u && pre[lo + 1u] <= k) ++lo;
+            next = lo < kRasterBatch - 1u ? pre[lo + 1u] : total;
             st = load_small(tri[lo]);
             bw = st.bw;
             ii = 0;
@@ -621,36 +623,44 @@ __device__ __forceinline__ void walk_small(const SmallTri* tri, const uint32_t* 
 // One view's share of the meshlet raster (wave w of the grid takes meshlets
 // w, w + waves, ... of the view's list).
 // Bound by vector instructions where meshlets are many (views up to 3840x2160 of
-// sub-pixel triangles: VALU 63% busy, 795 instructions a meshlet and wave) and by
-// the cache's stores where most triangles face away.  Scans and searches on
-// DPP moves instead of LDS round trips: 4417 -> 3561 us there, 16.5 -> 12.0 us for
-// one 640x360 frame.  Cache entries only for triangles that may own a pixel:
-// 320 -> 218 us for 16 views of 1024x832 (570 MB of stores less).
+// sub-pixel triangles) and by the cache's stores where most triangles face away.
+// Measured, in us a launch:
+//  - scans and searches on DPP moves instead of LDS round trips: 4417 -> 3561
+//    there, 16.5 -> 12.0 for one 640x360 frame;
+//  - cache entries only for triangles that may own a pixel: 320 -> 218 for 16
+//    views of 1024x832 (570 MB of stores less);
+//  - setup and walk over batches of 64 triangles of up to kGroup meshlets
+//    instead of one or two part-filled rounds a meshlet (few of a meshlet's
+//    triangles pass the per-triangle tests where they are small): 3535 -> 2962
+//    on the sub-pixel views, 132 -> 98 for 8 views of 640x480, 12.3 -> 10.6 for
+//    the 640x360 frame.  Three meshlets are what the LDS of three blocks a CU
+//    holds.
 template <bool STATS>
 __device__ __forceinline__ void raster_view(const RasterArgs& a)
 {
     RasterCount<STATS> rc;
-    __shared__ float4 s_clip[kWaves][64];
-    __shared__ SVtx s_sv[kWaves][64];
+    // vertices of the group's meshlets, kGroup x 64
+    __shared__ float4 s_clip[kWaves][kGroup * 64];
+    __shared__ SVtx s_sv[kWaves][kGroup * 64];
+    __shared__ uint32_t s_col[kWaves][kGroup * 64];
+    __shared__ uint32_t s_uv[kWaves][kGroup * 64];
+    __shared__ uint4 s_meta[kWaves][kGroup];   // draw, resolve-cache slot (~0u: none), list index
+    __shared__ uint32_t s_spill[kWaves][kGroup];   // non-zero: a triangle of that meshlet found a queue full
     __shared__ uint32_t s_tri[kWaves][97];   // a word past the 93 of 124 triangles is read (and not used)
-    __shared__ __align__(16) SmallTri s_st[kWaves][VKGV_MESHLET_TRIANGLES];
-    __shared__ __align__(16) uint32_t s_pre[kWaves][128];
-    __shared__ uint32_t s_list[kWaves][128];   // the meshlet's triangles past the per-slot tests
+    __shared__ uint32_t s_list[kWaves][kRasterBatch + VKGV_MESHLET_TRIANGLES];   // triangles past the per-slot tests
+    __shared__ __align__(16) SmallTri s_st[kWaves][kRasterBatch];
+    __shared__ __align__(16) uint32_t s_pre[kWaves][kRasterBatch];
     __shared__ uint32_t s_own[kWaves][64];     // triangle of each lane's first pixel slot
 
     const int w = threadIdx.x >> 6;
     const uint32_t lane = threadIdx.x & 63u;
-    __shared__ uint32_t s_col[kWaves][64];
-    __shared__ uint32_t s_uv[kWaves][64];
     const uint32_t count = a.count;
     const uint32_t slot0 = a.slot0;
     const uint32_t nwaves = gridDim.x * kWaves;
     const float hw = (float)a.W * 0.5f, hh = (float)a.H * 0.5f;
     const int W = (int)a.W, H = (int)a.H;
     const BigQueue bq{ a.big, a.big_chunk, a.big_cap, a.chunk_tri, a.chunk_cap, a.ctr, a.keys, a.W };
-    // non-zero when a triangle of the wave's meshlet found a queue full
-    __shared__ uint32_t s_spill[kWaves];
-    if (lane == 0) s_spill[w] = 0u;
+    if (lane < kGroup) s_spill[w][lane] = 0u;
 
     // A software pipeline over the wave's meshlets i = first, first + nwaves,
     // ...: each input of a meshlet is loaded while earlier meshlets are
@@ -709,6 +719,7 @@ __device__ __forceinline__ void raster_view(const RasterArgs& a)
     uint32_t x1 = vidx_of(r1, idx + nwaves < count);
     Fetch f0;
     fetch(r0, vidx_of(r0, idx < count), idx < count, f0);
+    uint32_t g = 0, n = 0;   // the meshlet's place in the group, triangles on the list
     while (idx < count) {
         const uint32_t d = field(r0, 0);
         const uint32_t matw = field(r0, 5);
@@ -730,6 +741,7 @@ __device__ __forceinline__ void raster_view(const RasterArgs& a)
             const float4 albedo = make_float4(__uint_as_float(field(f0.mat, 0)), __uint_as_float(field(f0.mat, 1)),
                                               __uint_as_float(field(f0.mat, 2)), __uint_as_float(field(f0.mat, 3)));
             if (lane == 0) {
+                s_meta[w][g] = make_uint4(d, cached ? slot : 0xFFFFFFFFu, idx, 0u);
                 gstore(a.draw_slot + d, cached ? slot : 0xFFFFFFFFu);
                 if (cached) {
                     gstore(a.slot_albedo + slot, albedo);
@@ -739,15 +751,16 @@ __device__ __forceinline__ void raster_view(const RasterArgs& a)
         }
 
         // vertices: clip = (VP * M) * (pos, 1) (visbuffer.mesh.glsl:44-65)
+        const uint32_t vb = g * 64u;
         if (lane < vc) {
             const float4 c = mat4_point(mvp, f0.x, f0.y, f0.z);
-            s_clip[w][lane] = c;
-            s_col[w][lane] = f0.col;
-            if (tex) s_uv[w][lane] = f0.uv;
+            s_clip[w][vb + lane] = c;
+            s_col[w][vb + lane] = f0.col;
+            if (tex) s_uv[w][vb + lane] = f0.uv;
             SVtx sv;
             sv.x = 0; sv.y = 0; sv.z = 0.0f;
             sv.ok = project_vtx(c, hw, hh, sv) ? 1u : 0u;
-            s_sv[w][lane] = sv;
+            s_sv[w][vb + lane] = sv;
         }
         {
             const uint32_t ndw = (tc * 3u + 3u) >> 2;
@@ -763,21 +776,18 @@ __device__ __forceinline__ void raster_view(const RasterArgs& a)
         wave_sync();
 
         // Stage 1, every triangle slot: the back-face test and setup_tri's
-        // pixel-range test (a projected triangle whose
-        // bounding box holds no pixel centre rasterizes nothing).  The
-        // triangles left (and those that need clipping) are packed into
-        // s_list (t | i0 << 8 | i1 << 16 | i2 << 24), so that the setup below
-        // runs over them in as few 64-lane rounds as there are: one for a
-        // typical meshlet, whose back faces and pixel-less triangles are most
-        // of its slots.
-        uint32_t nlive = 0;
+        // pixel-range test (a projected triangle whose bounding box holds no
+        // pixel centre rasterizes nothing).  The triangles left (and those that
+        // need clipping) join s_list (t | j0 << 7 | j1 << 15 | j2 << 23, the j
+        // vertices of the group), so that the setup below runs over full
+        // batches of 64 of them.
 #pragma unroll
         for (int sl = 0; sl < 2; ++sl) {
             const uint32_t t = lane + 64u * (uint32_t)sl;
             bool live = false;
             uint32_t packed = 0u;
             if (t < tc) {
-                const uint32_t tb = tri_bytes(s_tri[w], t);
+                const uint32_t tb = tri_bytes(s_tri[w], t) + g * 0x404040u;
                 const uint32_t i0 = tb & 0xFFu, i1 = (tb >> 8) & 0xFFu, i2 = (tb >> 16) & 0xFFu;
                 const float4 c0 = s_clip[w][i0], c1 = s_clip[w][i1], c2 = s_clip[w][i2];
                 live = true;
@@ -795,33 +805,35 @@ __device__ __forceinline__ void raster_view(const RasterArgs& a)
                                && max((miny - 128 + 255) >> 8, 0) <= min((maxy - 128) >> 8, H - 1);
                     }
                 }
-                packed = t | (tb << 8);
+                packed = t | (tb << 7);
             }
             const unsigned long long m = __ballot(live);
-            const uint32_t pos = nlive + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+            const uint32_t pos = n + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
                                                                     __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
             if (live) s_list[w][pos] = packed;
-            nlive += (uint32_t)__popcll(m);
+            n += (uint32_t)__popcll(m);
         }
         wave_sync();
 
-        // Stage 2, the packed triangles: the resolve cache (a triangle dropped
-        // above owns no pixel, so that its entry is never read), clip queue,
-        // setup, small or big.
-        uint32_t npix[2] = { 0u, 0u };
-#pragma unroll
-        for (int sl = 0; sl < 2; ++sl) {
-            if (64u * (uint32_t)sl >= nlive) break;   // wave-uniform
-            const uint32_t pos = lane + 64u * (uint32_t)sl;
+        // Stage 2 over batches of 64 triangles of the list: full ones as soon as
+        // there are, the rest when the group is full or the wave's meshlets end.
+        const bool last = g + 1u == kGroup || nidx >= count;   // wave-uniform
+        uint32_t done = 0;
+        while (n - done >= kRasterBatch || (last && done < n)) {
+            // The resolve cache (a triangle dropped above owns no pixel, so that
+            // its entry is never read), clip queue, setup, small or big.
+            uint32_t npix = 0u;
             bool want_big = false;
             TriSetup ts;
-            uint32_t id = 0;
+            uint32_t id = 0, i0 = 0;
             do {   // per-lane triangle work; `continue` leaves it
-                if (pos >= nlive) continue;
-                const uint32_t e = s_list[w][pos];
-                const uint32_t t = e & 0xFFu, i0 = (e >> 8) & 0xFFu, i1 = (e >> 16) & 0xFFu, i2 = e >> 24;
-                id = (d << VKGV_TRIANGLE_BITS) | t;
-                if (cached && bary) {
+                if (lane >= n - done) continue;
+                const uint32_t e = s_list[w][done + lane];
+                const uint32_t t = e & 0x7Fu, i1 = (e >> 15) & 0xFFu, i2 = (e >> 23) & 0xFFu;
+                i0 = (e >> 7) & 0xFFu;
+                const uint4 meta = s_meta[w][i0 >> 6];
+                id = (meta.x << VKGV_TRIANGLE_BITS) | t;
+                if (bary && meta.y != 0xFFFFFFFFu) {
                     const float4 c0 = s_clip[w][i0], c1 = s_clip[w][i1], c2 = s_clip[w][i2];
                     // TriCache: r[k] = v_{k+1} x v_{k+2} over the clip (x, y, w) of the
                     // vertices, then the colours; 48 bytes always, the uv words only
@@ -833,7 +845,7 @@ __device__ __forceinline__ void raster_view(const RasterArgs& a)
                                 r12 = c2.x * c0.y - c2.y * c0.x;
                     const float r20 = c0.y * c1.w - c0.w * c1.y, r21 = c0.w * c1.x - c0.x * c1.w,
                                 r22 = c0.x * c1.y - c0.y * c1.x;
-                    uint4* dst = reinterpret_cast<uint4*>(a.tri_cache + (size_t)slot * 128u + t);
+                    uint4* dst = reinterpret_cast<uint4*>(a.tri_cache + (size_t)meta.y * 128u + t);
                     gstore(dst, make_uint4(__float_as_uint(r00), __float_as_uint(r01), __float_as_uint(r02),
                                            __float_as_uint(r10)));
                     gstore(dst + 1, make_uint4(__float_as_uint(r11), __float_as_uint(r12), __float_as_uint(r20),
@@ -854,7 +866,7 @@ __device__ __forceinline__ void raster_view(const RasterArgs& a)
                         gstore(reinterpret_cast<uint4*>(q) + 3, make_uint4(id, 0u, 0u, 0u));
                     } else {
                         atomicOr(&a.ctr->overflow, 2u);
-                        s_spill[w] = 1u;
+                        s_spill[w][i0 >> 6] = 1u;
                     }
                     continue;
                 }
@@ -880,87 +892,85 @@ __device__ __forceinline__ void raster_view(const RasterArgs& a)
                     st.dim = (uint16_t)(bw | (bh << 8));
                     st.pad = 0;
                     st.id = id;
-                    s_st[w][pos] = st;
-                    npix[sl] = bw * bh;
+                    s_st[w][lane] = st;
+                    npix = bw * bh;
                 } else {
                     want_big = true;
                 }
             } while (false);
-            if (push_big_wave(want_big, ts, id, lane, bq)) s_spill[w] = 1u;
-        }
+            if (push_big_wave(want_big, ts, id, lane, bq)) s_spill[w][i0 >> 6] = 1u;
 
-        // exclusive prefix of pixel counts over the 128 triangle slots
-        const uint32_t x0 = wave_scan_add(npix[0]);
-        const uint32_t tot0 = (uint32_t)__builtin_amdgcn_readlane((int)x0, 63);
-        uint32_t pre0 = x0 - npix[0], pre1 = tot0, total = tot0;
-        if (nlive > 64u) {   // wave-uniform
-            const uint32_t x1 = wave_scan_add(npix[1]);
-            pre1 = tot0 + x1 - npix[1];
-            total += (uint32_t)__builtin_amdgcn_readlane((int)x1, 63);
-        }
-        s_pre[w][lane] = pre0;
-        s_pre[w][64 + lane] = pre1;
-        s_own[w][lane] = 0u;
-        wave_sync();
+            // exclusive prefix of the batch's pixel counts
+            const uint32_t incl = wave_scan_add(npix);
+            const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+            const uint32_t pre = incl - npix;
+            s_pre[w][lane] = pre;
+            s_own[w][lane] = 0u;
+            wave_sync();
 
-        // A heavy meshlet keeps the first kJobKeep slots and defers the rest
-        // to the bin pass in runs of kJobSlots (staged record + jobs), so that
-        // its fragment atomics spread over many CUs instead of queueing in
-        // this wave's.  Without room for the record or its jobs the wave walks
-        // every slot itself.
-        uint32_t keep = total;
-        if (total > kJobKeep + kJobSlots / 2u) {   // wave-uniform
-            const uint32_t njobs = (total - kJobKeep + kJobSlots - 1u) / kJobSlots;
-            // one atomic reserves the record (high bits) and the jobs (low bits)
-            unsigned long long res = 0ull;
-            if (lane == 0) res = atomicAdd(&a.ctr->frag_jobs, (1ull << kJobCountBits) | (unsigned long long)njobs);
-            res = __shfl(res, 0);
-            const uint32_t sidx = (uint32_t)(res >> kJobCountBits);
-            const unsigned long long j0 = res & ((1ull << kJobCountBits) - 1ull);
-            const bool room = sidx < a.stage_cap && j0 + njobs <= (unsigned long long)a.job_cap;
-            // every reserved job inside the list is written, marked unused without room
+            // A heavy batch keeps the first kJobKeep slots and defers the rest
+            // to the bin pass in runs of kJobSlots (staged record + jobs), so that
+            // its fragment atomics spread over many CUs instead of queueing in
+            // this wave's.  Without room for the record or its jobs the wave walks
+            // every slot itself.
+            uint32_t keep = total;
+            if (total > kJobKeep + kJobSlots / 2u) {   // wave-uniform
+                const uint32_t njobs = (total - kJobKeep + kJobSlots - 1u) / kJobSlots;
+                // one atomic reserves the record (high bits) and the jobs (low bits)
+                unsigned long long res = 0ull;
+                if (lane == 0) res = atomicAdd(&a.ctr->frag_jobs, (1ull << kJobCountBits) | (unsigned long long)njobs);
+                res = __shfl(res, 0);
+                const uint32_t sidx = (uint32_t)(res >> kJobCountBits);
+                const unsigned long long j0 = res & ((1ull << kJobCountBits) - 1ull);
+                const bool room = sidx < a.stage_cap && j0 + njobs <= (unsigned long long)a.job_cap;
+                // every reserved job inside the list is written, marked unused without room
 #pragma unroll 1
-            for (uint32_t q = lane; q < njobs; q += 64u)
-                if (j0 + q < (unsigned long long)a.job_cap)
-                    gstore(a.jobs + j0 + q, room ? FragJob{ sidx, kJobKeep + q * kJobSlots } : FragJob{ 0xFFFFFFFFu, 0u });
-            if (room) {
-                uint4* dst = reinterpret_cast<uint4*>(a.stage[sidx].w);
-                const uint4* st4 = reinterpret_cast<const uint4*>(s_st[w]);
+                for (uint32_t q = lane; q < njobs; q += 64u)
+                    if (j0 + q < (unsigned long long)a.job_cap)
+                        gstore(a.jobs + j0 + q, room ? FragJob{ sidx, kJobKeep + q * kJobSlots } : FragJob{ 0xFFFFFFFFu, 0u });
+                if (room) {
+                    uint4* dst = reinterpret_cast<uint4*>(a.stage[sidx].w);
+                    const uint4* st4 = reinterpret_cast<const uint4*>(s_st[w]);
 #pragma unroll 2
-                for (uint32_t q = lane; q < kStageTri4; q += 64u) gstore(dst + q, st4[q]);
-                if (lane < 32u) gstore(dst + kStageTri4 + lane, reinterpret_cast<const uint4*>(s_pre[w])[lane]);
-                if (lane == 0) gstore(dst + kStageTri4 + 32u, make_uint4(total, 0u, 0u, 0u));
-                keep = kJobKeep;
+                    for (uint32_t q = lane; q < kStageTri4; q += 64u) gstore(dst + q, st4[q]);
+                    if (lane < kRasterBatch / 4u) gstore(dst + kStageTri4 + lane, reinterpret_cast<const uint4*>(s_pre[w])[lane]);
+                    if (lane == 0) gstore(dst + kStageTri4 + kRasterBatch / 4u, make_uint4(total, 0u, 0u, 0u));
+                    keep = kJobKeep;
+                }
             }
-        }
-        // Lane l walks slots l * per, ...: the triangle that holds lane l's first
-        // slot names itself there if no earlier lane's first slot is in it, and
-        // the lanes after take the last name (a search of the prefix was seven
-        // dependent LDS reads).
-        {
+            // Lane l walks slots l * per, ...: the triangle that holds lane l's first
+            // slot names itself there if no earlier lane's first slot is in it, and
+            // the lanes after take the last name (a search of the prefix was seven
+            // dependent LDS reads).
             const uint32_t per = (keep + 63u) >> 6;
             if (per) {   // wave-uniform
-                const uint32_t l0 = per == 1u ? pre0 : small_div(pre0 + per - 1u, per);
-                if (npix[0] && l0 * per < pre0 + npix[0] && l0 < 64u) s_own[w][l0] = lane;
-                if (nlive > 64u) {
-                    const uint32_t l1 = per == 1u ? pre1 : small_div(pre1 + per - 1u, per);
-                    if (npix[1] && l1 * per < pre1 + npix[1] && l1 < 64u) s_own[w][l1] = 64u + lane;
-                }
+                const uint32_t l0 = per == 1u ? pre : small_div(pre + per - 1u, per);
+                if (npix && l0 * per < pre + npix && l0 < 64u) s_own[w][l0] = lane;
                 wave_sync();
                 const uint32_t lo = wave_scan_max(s_own[w][lane]);
                 const uint32_t k = lane * per;
                 walk_small(s_st[w], s_pre[w], total, lo, k, min(k + per, keep), a.keys, a.W, rc);
             }
+            wave_sync();
+            done = min(done + kRasterBatch, n);
+        }
+        if (done) {   // the rest, fewer than 64, moves to the front
+            n -= done;
+            const uint32_t e = lane < n ? s_list[w][done + lane] : 0u;
+            wave_sync();
+            if (lane < n) s_list[w][lane] = e;
+        }
+        if (last || n == 0u) {   // no triangle of the group is left
+            // its meshlets that are redone by the direct path after this kernel
+            if (lane <= g && s_spill[w][lane]) {
+                a.redo[atomicAdd(&a.ctr->redo_count, 1u)] = s_meta[w][lane].z;
+                s_spill[w][lane] = 0u;
+            }
+            g = 0u;
+        } else {
+            ++g;
         }
         wave_sync();
-        // the meshlet is redone by the direct path after this kernel
-        if (__builtin_amdgcn_readfirstlane(s_spill[w])) {
-            if (lane == 0) {
-                a.redo[atomicAdd(&a.ctr->redo_count, 1u)] = idx;
-                s_spill[w] = 0u;
-            }
-            wave_sync();
-        }
         idx = nidx;      // static stride: no shared cursor
     }
     rc.flush(a.ctr);
@@ -1058,7 +1068,7 @@ __device__ __forceinline__ void frag_job(const BigArgs& a, uint32_t j, RasterCou
     const uint32_t* rec = a.stage[stage].w;
     const SmallTri* tri = reinterpret_cast<const SmallTri*>(rec);
     const uint32_t* pre = rec + kStageTriWords;
-    const uint32_t total = __builtin_amdgcn_readfirstlane(rec[kStageTriWords + 128u]);
+    const uint32_t total = __builtin_amdgcn_readfirstlane(rec[kStageTriWords + kRasterBatch]);
     const uint32_t end = min(first + kJobSlots, total);
     const uint32_t per = (end - first + 63u) >> 6;
     const uint32_t k = first + lane * per;
