@@ -48,7 +48,10 @@ __global__ __launch_bounds__(kThreads) void stage_kernel(const uint8_t* __restri
     }
 }
 
-// A pinned stage: the two halves' bytes, then their flags.
+// A pinned stage: the two halves' bytes, then their flags.  The host reads both
+// while the kernel that stores them runs, so the memory is asked for as
+// coherent: without the flag its kind is left to the environment, and other
+// memory is only promised to be up to date once the kernel has ended.
 struct Stage {
     uint8_t* bytes = nullptr;
     uint32_t* flags = nullptr;
@@ -75,7 +78,7 @@ bool take_stage(Stage& s)
     }
     void* p = nullptr;
     const size_t flag_bytes = sizeof(uint32_t) * 2 * kHalfPieces;
-    if (hipHostMalloc(&p, 2 * kHalfBytes + flag_bytes, hipHostMallocPortable) != hipSuccess) {
+    if (hipHostMalloc(&p, 2 * kHalfBytes + flag_bytes, hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
         (void)hipGetLastError();
         return false;
     }
