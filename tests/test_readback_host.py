@@ -95,9 +95,23 @@ def test_the_stage_is_coherent_memory(fake):
     """)
 
 
+def test_small_reads_are_staged_only_behind_work(fake):
+    """On an idle stream a plain copy is faster below 896 KB."""
+    child(fake, """
+        user(True)
+        for n, busy, launches in ((65536, 0, 0), (917500, 0, 0), (917504, 0, 1), (65536, 1, 1), (65532, 1, 0)):
+            setv("busy", busy)
+            before = count("launches")
+            read(n)
+            assert count("launches") - before == launches, (n, busy)
+        user(False)
+    """)
+
+
 def test_any_size_arrives_whole(fake):
     child(fake, """
         user(True)
+        setv("busy", 1)
         for n in (1, 4, 65532, 65536, 65540, 2**20 - 4, 2**20, 2**21, 2**21 + 4, 2**22 + 16388, 9 * 2**20):
             read(n)
         before = count("launches")
