@@ -17,7 +17,8 @@ FAKE = r"""
 #include <string.h>
 typedef struct { uint32_t x, y, z; } dim3;
 unsigned host_flags = 0;
-int allocs = 0, frees = 0, copies = 0, launches = 0, busy = 0;
+int allocs = 0, frees = 0, copies = 0, launches = 0, busy = 0, news = 0;
+void* _Znwm(size_t n) { ++news; return malloc(n ? n : 1); }   /* operator new */
 int hipHostMalloc(void** p, size_t n, unsigned flags) { ++allocs; host_flags = flags; return posix_memalign(p, 4096, n) ? 2 : 0; }
 int hipHostFree(void* p) { ++frees; free(p); return 0; }
 int hipPointerGetAttributes(void* a, const void* p) { (void)a; (void)p; return 1; }
@@ -104,6 +105,18 @@ def test_small_reads_are_staged_only_behind_work(fake):
             before = count("launches")
             read(n)
             assert count("launches") - before == launches, (n, busy)
+        user(False)
+    """)
+
+
+def test_a_read_allocates_nothing_that_could_throw(fake):
+    """No exception can leave the C entry points from here."""
+    child(fake, """
+        user(True)
+        before = count("news")
+        for _ in range(3):
+            read(2**20)
+        assert count("news") == before
         user(False)
     """)
 

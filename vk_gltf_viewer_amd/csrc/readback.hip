@@ -20,10 +20,10 @@
 // read of kReadStaged bytes is staged while the stream is busy, one of
 // kReadStagedIdle always.
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <cstring>
 #include <mutex>
-#include <vector>
 
 #include "internal.hpp"
 
@@ -71,16 +71,16 @@ struct Stage {
 // gone; a readback owns the stage it took until it returns.
 constexpr size_t kIdle = 2;
 std::mutex g_mutex;
-std::vector<Stage> g_idle;
+std::array<Stage, kIdle> g_idle;   // the first g_idle_count
+size_t g_idle_count = 0;
 uint32_t g_users = 0;
 
 bool take_stage(Stage& s)
 {
     {
         std::lock_guard<std::mutex> lock(g_mutex);
-        if (!g_idle.empty()) {
-            s = g_idle.back();
-            g_idle.pop_back();
+        if (g_idle_count) {
+            s = g_idle[--g_idle_count];
             return true;
         }
     }
@@ -100,8 +100,8 @@ void give_stage(const Stage& s)
 {
     {
         std::lock_guard<std::mutex> lock(g_mutex);
-        if (g_users && g_idle.size() < kIdle) {
-            g_idle.push_back(s);
+        if (g_users && g_idle_count < kIdle) {
+            g_idle[g_idle_count++] = s;
             return;
         }
     }
@@ -147,13 +147,18 @@ bool pageable(const void* p)
 
 void read_back_user(bool joins)
 {
-    std::vector<Stage> gone;
+    std::array<Stage, kIdle> gone;
+    size_t n = 0;
     {
         std::lock_guard<std::mutex> lock(g_mutex);
         g_users += joins ? 1u : ~0u;
-        if (g_users == 0) gone.swap(g_idle);
+        if (g_users == 0) {
+            gone = g_idle;
+            n = g_idle_count;
+            g_idle_count = 0;
+        }
     }
-    for (const Stage& s : gone) (void)hipHostFree(s.bytes);
+    for (size_t k = 0; k < n; ++k) (void)hipHostFree(gone[k].bytes);
 }
 
 hipError_t read_back(void* dst, const void* src, size_t bytes, hipStream_t st)
