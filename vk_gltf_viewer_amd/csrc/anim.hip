@@ -142,12 +142,17 @@ __device__ __forceinline__ void sample(const AnimDev& d, const AnimChan& sp, flo
     }
 }
 
+__device__ __forceinline__ NodeTrs& node_trs(const AnimDev& d, uint32_t n)
+{
+    return *reinterpret_cast<NodeTrs*>(d.nodes[n].translation);
+}
+
 __global__ __launch_bounds__(64) void anim_channels_kernel(AnimDev d, float time)
 {
     const uint32_t c = blockIdx.x * 64u + threadIdx.x;
     if (c >= d.channel_count) return;
     const AnimChan ch = d.channels[c];
-    NodeTrs& x = d.trs[ch.node];
+    NodeTrs& x = node_trs(d, ch.node);
     const uint32_t path = ch.kind & 0xFFu;
     if (path == VKGV_PATH_ROTATION) {
         float q[4];
@@ -201,11 +206,11 @@ __global__ __launch_bounds__(256) void world_transforms_kernel(AnimDev d, float*
     float4 m = make_float4(r == 0 ? 1.0f : 0.0f, r == 1 ? 1.0f : 0.0f, r == 2 ? 1.0f : 0.0f, r == 3 ? 1.0f : 0.0f);
     const uint32_t* chain = d.chain_nodes + d.chain_first[i];
     const uint32_t len = d.chain_first[i + 1] - d.chain_first[i];   // at least the node itself
-    NodeTrs next = d.trs[chain[0]];
+    NodeTrs next = node_trs(d, chain[0]);
     uint32_t after = len > 1 ? chain[1] : 0u;
     for (uint32_t k = 0; k < len; ++k) {
         const NodeTrs cur = next;
-        if (k + 1 < len) next = d.trs[after];
+        if (k + 1 < len) next = node_trs(d, after);
         if (k + 2 < len) after = chain[k + 2];
         m = apply_trs(m, cur);
     }

@@ -38,8 +38,9 @@ struct RasterRec {
 static_assert(sizeof(RasterRec) == 32, "RasterRec layout");
 
 // Device view of the uploaded scene.
-// Animated TRS of one node for the device transform update.
+// The TRS within a vkgv_node, as the device transform update reads and writes it.
 struct NodeTrs { float t[3], q[4], s[3]; };
+static_assert(offsetof(vkgv_node, translation) + sizeof(NodeTrs) == sizeof(vkgv_node), "a node ends with its TRS");
 
 // One animation channel with its sampler, as the device update reads it.
 struct AnimChan {
@@ -48,9 +49,8 @@ struct AnimChan {
     uint32_t input_offset, input_count;  // key times
     uint32_t output_offset;              // first output value
     float last;                          // the last key time
-    uint32_t pad[2];
 };
-static_assert(sizeof(AnimChan) == 32, "AnimChan layout");
+static_assert(sizeof(AnimChan) == 24, "AnimChan layout");
 
 // Node hierarchy and animations on the device (vkgv_set_hierarchy).
 struct AnimDev {
@@ -58,7 +58,7 @@ struct AnimDev {
     uint32_t channel_count;
     const float* times;
     const float* values;
-    NodeTrs* trs;                        // per node: its static TRS, the animated parts of this update
+    vkgv_node* nodes;                    // with their static TRS, the animated parts of this update in place
     uint32_t mesh_count;                 // mesh nodes = transforms
     const uint32_t* chain_first;         // mesh_count + 1
     const uint32_t* chain_nodes;         // root-to-node chain of each mesh node
