@@ -133,7 +133,8 @@ __device__ __forceinline__ Snap snap_vertex(float4 p, const Dims& d)
 
 // The start of render: clip[ci, v] = M[ci] (p_v, 1), its snapped vertex (of the
 // position rounded to float), and the buffers of the passes that follow
-// cleared: npx keys and nvis words of flags, spread over the grid.
+// cleared: npx keys and nvis words of flags (the vis bytes and the wide flag
+// behind them), spread over the grid.
 template <typename C>
 __global__ __launch_bounds__(kBlock) void project_kernel(const C* __restrict__ pos, const C* __restrict__ M, Dims d,
                                                           C* __restrict__ clip, Snap* __restrict__ snap,
@@ -171,6 +172,7 @@ struct TriWalk {
     int ox, oy;         // first centre from vertex 0, 1/256 pixel
     int px0, px1, py0, py1;
     uint32_t id;
+    float size;         // area in pixels
 
     // Visibility-buffer key of pixel (i, j) of the box; all ones where the
     // centre is not covered.
@@ -189,10 +191,31 @@ __device__ __forceinline__ void key_min(unsigned long long* p, unsigned long lon
     (void)__hip_atomic_fetch_min(p, key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// boxes (may be null): the pixel box of each triangle with a fragment.
+// What render keeps a byte of per (camera, instance, triangle), vis: kSeen for
+// one with a visible pixel whose box the vertex pass walks, kWide for one with a
+// fragment whose terms the backward's pixel pass sums instead.  `wide` is a flag
+// for the whole call: there is a kWide byte.
+//
+// kWide is a box of more than kWideBox pixels, or one of more than kWaveBox of
+// which the triangle's area is less than 1 / kSliver.  The vertex pass reads the
+// whole box, once a corner, in the one wave of the vertex, triangle after
+// triangle; the pixel pass reads own pixels only but pays for every tile.  A step
+// of 1, 8 or 8 cameras, 512x512, spheres of 1280 triangles (boxes up to 5000
+// pixels) 1029 -> 736 us, 1841 -> 1358, of 2880 (boxes around 2000) equal; limits
+// of 512 and 256 take these to 975 and 733, but cost 8 and 15 % for 8 instances
+// of 5120 and 11520 triangles in float64.  Slivers: 200 triangles around one
+// vertex at 96x96 854 -> 568 us, 2000 at 400x400 in 4 cameras 198 -> 5.1 ms.
+constexpr int kWideBox = 1024;
+constexpr float kSliver = 16.0f;
+enum : uint8_t { kHidden = 0, kSeen = 1, kWide = 2 };
+
+// boxes (null with vis and wide, for a raster alone): the pixel box of each
+// triangle with a fragment.
 __global__ __launch_bounds__(kBlock) void raster_tris_kernel(const Snap* __restrict__ snap, const int* __restrict__ tris,
                                                               Dims d, unsigned long long* __restrict__ keys,
-                                                              unsigned long long* __restrict__ boxes, int cull_back)
+                                                              unsigned long long* __restrict__ boxes,
+                                                              uint8_t* __restrict__ vis, uint32_t* __restrict__ wide_flag,
+                                                              int cull_back)
 {
     const int t = (int)(blockIdx.x * kBlock + threadIdx.x), lane = (int)(threadIdx.x & 63u);
     for (int ci = (int)blockIdx.y; ci < d.C * d.I; ci += (int)gridDim.y) {
@@ -231,6 +254,7 @@ __global__ __launch_bounds__(kBlock) void raster_tris_kernel(const Snap* __restr
                     const double e2x = (double)(q.x - a.x) / 256.0, e2y = (double)(q.y - a.y) / 256.0;
                     const double dz1 = (double)p.z - (double)a.z, dz2 = (double)q.z - (double)a.z;
                     const double det = (double)area / 65536.0;
+                    w.size = 0.5f * (float)det;
                     w.z0 = a.z;
                     w.za = (float)((dz1 * e2y - dz2 * e1y) / det);
                     w.zb = (float)((dz2 * e1x - dz1 * e2x) / det);
@@ -278,8 +302,14 @@ __global__ __launch_bounds__(kBlock) void raster_tris_kernel(const Snap* __restr
             }
             if (__ballot(any) != 0ull && lane == j) drawn = true;
         }
-        if (boxes && drawn)
+        if (boxes && drawn) {
             boxes[(size_t)ci * d.T + t] = pack_box(Box{ w.px0, w.px1, w.py0, w.py1 });
+            const int box = (w.px1 - w.px0 + 1) * (w.py1 - w.py0 + 1);   // below 2^28
+            if (box > kWideBox || (box > kWaveBox && (float)box > kSliver * w.size)) {
+                vis[(size_t)ci * d.T + t] = kWide;
+                *wide_flag = 1u;   // every writer stores the same value
+            }
+        }
     }
 }
 
@@ -818,7 +848,9 @@ __global__ __launch_bounds__(kBlock) void vertex_gather_kernel(const int* __rest
 // kPairs camera-instance pairs (grid y) and writes the sums over its pairs of
 // M^T g (its positions' gradient) and of the attributes' gradient to
 // part_pos[y][V][3] and part_attr[y][V][A], and adds its sums over the
-// vertices of g (p_v, 1)^T to g_M.  boxes: of the triangles with vis set.
+// vertices of g (p_v, 1)^T to g_M.  boxes: of the triangles with vis kSeen;
+// what the pixel pass summed of the kWide ones, wide_pos and wide_attr, joins
+// part 0.
 //
 // Bound by the latency of flag -> box -> ids -> records: a wave goes through
 // the pairs in which any of its triangles has a pixel, the next pair's boxes in
@@ -836,7 +868,10 @@ __global__ __launch_bounds__(kBlock) void vertex_render_kernel(const int* __rest
                                                                 const unsigned long long* __restrict__ boxes,
                                                                 const uint8_t* __restrict__ vis,
                                                                 const R* __restrict__ contrib, C* __restrict__ part_pos,
-                                                                R* __restrict__ part_attr, C* __restrict__ g_M)
+                                                                R* __restrict__ part_attr, C* __restrict__ g_M,
+                                                                const uint32_t* __restrict__ wide_flag,
+                                                                const C* __restrict__ wide_pos,
+                                                                const R* __restrict__ wide_attr)
 {
     constexpr int kRows = (int)kBlock / 16;   // rows of 16 lanes, two vertices each
     __shared__ R2<C> s_g[kRows][kPairs][kVertexLanes];
@@ -856,10 +891,10 @@ __global__ __launch_bounds__(kBlock) void vertex_render_kernel(const int* __rest
     for (int r = 0; __ballot(j0 + r < j1) != 0ull; r += kVertexLanes) {
         const int j = j0 + r + u;
         const int corner = j < j1 ? adj[j] : -1, t = corner / 3, k = corner - 3 * t;
-        uint32_t seen = 0u;     // bit q: the triangle has a pixel in pair ci0 + q
+        uint32_t seen = 0u;     // bit q: the triangle has a gathered pixel in pair ci0 + q
 #pragma unroll
         for (int q = 0; q < kPairs; ++q)
-            if (corner >= 0 && q < np && vis[(size_t)(ci0 + q) * d.T + t]) seen |= 1u << q;
+            if (corner >= 0 && q < np && vis[(size_t)(ci0 + q) * d.T + t] == kSeen) seen |= 1u << q;
         uint32_t pairs = 0u;    // of any lane of the wave
 #pragma unroll
         for (int q = 0; q < kPairs; ++q)
@@ -907,6 +942,10 @@ __global__ __launch_bounds__(kBlock) void vertex_render_kernel(const int* __rest
         }
     }
     if (live) {
+        if (blockIdx.y == 0 && *wide_flag != 0u) {
+            if (u < 3) g_pos += wide_pos[(size_t)v * 3 + u];
+            VKGV_CHANNELS(a) if (u == a) g_attr += wide_attr[(size_t)v * A + a];
+        }
         if (u < 3) part_pos[((size_t)blockIdx.y * d.V + v) * 3 + u] = g_pos;
         VKGV_CHANNELS(a) if (u == a) part_attr[((size_t)blockIdx.y * d.V + v) * A + a] = g_attr;
     }
@@ -1189,7 +1228,8 @@ template <typename R> struct TileState {
 //   kFromColor  the given `color`, ids and depth;
 //   kFromIds    ids and depth; the colour is interpolated here and written;
 //   kFromKeys   the raster's keys of the same clip positions: ids and depth
-//               are written too, and no pixel can be a stray.
+//               are written too, no pixel can be a stray, and the bytes of
+//               triangles that the raster left as kWide stay.
 // The pixels are marked for the backward as interp_fwd_kernel does.
 enum { kFromColor, kFromIds, kFromKeys };
 template <typename C, typename R, int FROM, int NA>
@@ -1201,7 +1241,8 @@ __global__ __launch_bounds__(kTileThreads) void aa_fwd_kernel(R* __restrict__ co
                                                                int A, R* __restrict__ out,
                                                                const unsigned long long* __restrict__ boxes,
                                                                unsigned* __restrict__ stray_blocks,
-                                                               uint8_t* __restrict__ vis)
+                                                               uint8_t* __restrict__ vis,
+                                                               const uint32_t* __restrict__ wide_flag)
 {
     __shared__ TileState<R> s;
     __shared__ R s_col[NA ? NA : kMaxAttr][kTileThreads];
@@ -1242,8 +1283,10 @@ __global__ __launch_bounds__(kTileThreads) void aa_fwd_kernel(R* __restrict__ co
         }
     }
     if (ok && px.inner) {
-        if (FROM == kFromKeys) vis[tri_index(d, px.c, id)] = 1;
-        else mark_pixel(boxes, d, px.c, id, px.x, px.y, px.p, stray_blocks, vis);
+        if (FROM == kFromKeys) {
+            uint8_t& seen = vis[tri_index(d, px.c, id)];
+            if (*wide_flag == 0u || seen != kWide) seen = kSeen;
+        } else mark_pixel(boxes, d, px.c, id, px.x, px.y, px.p, stray_blocks, vis);
     }
     __syncthreads();
     FrontTri<R> f;
@@ -1333,15 +1376,159 @@ __device__ __forceinline__ void add_clip_grad(C* g_clip, const Dims& d, int c, i
     atomicAdd(&g[3], C(gw));
 }
 
+// Orders the wave's LDS accesses before and after it.
+__device__ __forceinline__ void wave_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// What render's pixel pass needs for the kWide triangles: the flags, the mesh
+// and the matrices, and the gradients it adds to (zeroed before).
+template <typename C, typename R> struct WideArgs {
+    const uint8_t* vis;
+    const uint32_t* flag;
+    const C* pos;
+    const C* M;
+    C* g_pos;
+    C* g_M;
+    R* g_attr;
+};
+
+// The sums of a tile's kWide triangles in LDS: kWideSlots of them by a hash of
+// the id, then one slot a wave for the triangles that find none.
+constexpr int kWideSlots = 32, kTileWaves = kTileThreads / 64;
+template <typename C, typename R, int NA> struct WideTile {
+    static constexpr int kSlots = kWideSlots + kTileWaves, kAttr = 3 * (NA ? NA : kMaxAttr);
+    int id[kSlots];         // 0: free
+    C pos[kSlots][9];       // dL/d(x, y, w) of corner 0, 1, 2
+    R attr[kSlots][kAttr];  // dL/d the attributes of corner 0, 1, 2
+};
+
+// Adds a slot to the gradients through the vertex transform (g_pos = M^T g, g_M =
+// g (p, 1)^T), an atomic a lane; g_M is summed in lanes 16 .. 31 (entry lane - 16)
+// while the instance stays the same.
+template <typename C, typename R, int NA> struct WideFlush {
+    const WideArgs<C, R>& w;
+    const Dims& d;
+    int A, c, lane;
+    int inst = -1;
+    C sum_M = C(0);
+
+    __device__ __forceinline__ void add_M()
+    {
+        if (inst >= 0 && lane >= 16 && lane < 32 && (lane & 12) != 8)   // row 2 (z) has none
+            unsafeAtomicAdd(&w.g_M[((size_t)c * d.I + inst) * 16 + (size_t)(lane - 16)], sum_M);
+        sum_M = C(0);
+    }
+    __device__ __forceinline__ void add(const int* tris, const WideTile<C, R, NA>& t, int slot)
+    {
+        const int id = t.id[slot], i = (id - 1) / d.T;
+        const int* tri = tris + 3 * (size_t)(id - 1 - i * d.T);
+        if (i != inst) {
+            add_M();
+            inst = i;
+        }
+        if (lane < 9) {             // corner lane / 3, component lane % 3 of its position
+            const int k = lane / 3, j = lane - 3 * k;
+            const C* m = w.M + ((size_t)c * d.I + i) * 16;
+            const C* g = t.pos[slot] + 3 * k;
+            unsafeAtomicAdd(&w.g_pos[3 * (size_t)tri[k] + j], (m[j] * g[0] + m[4 + j] * g[1]) + m[12 + j] * g[2]);
+        } else if (lane >= 16 && lane < 32) {
+            const int row = (lane - 16) >> 2, col = lane & 3;
+            for (int k = 0; k < 3; ++k) {
+                const C p = col < 3 ? w.pos[3 * (size_t)tri[k] + col] : C(1);
+                sum_M += t.pos[slot][3 * k + min(row, 2)] * p;
+            }
+        } else if (lane >= 32 && lane < 32 + 3 * A) {   // corner (lane - 32) / A, channel (lane - 32) % A
+            const int k = (lane - 32) / A, a = (lane - 32) - k * A;
+            unsafeAtomicAdd(&w.g_attr[(size_t)tri[k] * A + a], t.attr[slot][lane - 32]);
+        }
+    }
+};
+
+// The terms of the tile's pixels on kWide triangles, to the gradients: a
+// triangle's records are summed over the wave, then over the tile's waves in
+// LDS.  key: the pixel's id, 0 for one that has nothing to add; o: its record.
+// Every thread of the block calls it.
+//
+// With atomics from every wave instead of from every tile, 2000 triangles around
+// one vertex in 4 views of 400x400 take 10 ms a step instead of 4.8, and 8 views
+// of 512x512 of 20 triangles 2.5 instead of 1.8; the entries of g_M are what the
+// atomics meet at.
+template <typename C, typename R, int NA>
+__device__ __forceinline__ void add_wide(const WideArgs<C, R>& w, WideTile<C, R, NA>& t, const int* tris, const Dims& d,
+                                         int A, int c, int key, const R* o)
+{
+    using Tile = WideTile<C, R, NA>;
+    const int lane = (int)(threadIdx.x & 63u), wave = (int)(threadIdx.x >> 6);
+    for (int k = (int)threadIdx.x; k < kWideSlots; k += kTileThreads) t.id[k] = 0;
+    for (int k = (int)threadIdx.x; k < kWideSlots * 9; k += kTileThreads) (&t.pos[0][0])[k] = C(0);
+    for (int k = (int)threadIdx.x; k < kWideSlots * Tile::kAttr; k += kTileThreads) (&t.attr[0][0])[k] = R(0);
+    __syncthreads();
+    WideFlush<C, R, NA> flush{ w, d, A, c, lane };
+    unsigned long long pending = __ballot(key != 0);
+    while (pending != 0ull) {
+        const int id = __builtin_amdgcn_readlane(key, __ffsll((long long)pending) - 1);
+        const bool mine = key == id;
+        pending &= ~__ballot(mine);
+        C gp = C(0);    // lane l < 9: entry l of the slot's pos
+        R ga = R(0);    // lane 32 + l: entry l of its attr
+#pragma unroll 1
+        for (int k = 0; k < 3; ++k) {   // not unrolled: the pixel pass keeps its registers
+            const R* ok = o + k * (3 + A);
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                const C s = sum64(mine ? C(ok[j]) : C(0));
+                gp = lane == 3 * k + j ? s : gp;
+            }
+            VKGV_CHANNELS(a) {
+                const R s = sum64(mine ? ok[3 + a] : R(0));
+                ga = lane == 32 + k * A + a ? s : ga;
+            }
+        }
+        int slot = (int)((uint32_t)id * 2654435761u >> 27), tries = 0;   // the hash's 5 bits
+        for (; tries < 4; ++tries, slot = (slot + 1) % kWideSlots) {
+            int was = 0;
+            if (lane == 0) was = atomicCAS(&t.id[slot], 0, id);
+            was = __builtin_amdgcn_readfirstlane(was);
+            if (was == 0 || was == id) break;
+        }
+        if (tries < 4) {
+            if (lane < 9) unsafeAtomicAdd(&t.pos[slot][lane], gp);
+            if (lane >= 32 && lane < 32 + 3 * A) unsafeAtomicAdd(&t.attr[slot][lane - 32], ga);
+        } else {
+            slot = kWideSlots + wave;
+            if (lane == 0) t.id[slot] = id;
+            if (lane < 9) t.pos[slot][lane] = gp;
+            if (lane >= 32 && lane < 32 + 3 * A) t.attr[slot][lane - 32] = ga;
+            wave_fence();
+            flush.add(tris, t, slot);
+            wave_fence();
+        }
+    }
+    __syncthreads();
+    for (int slot = wave; slot < kWideSlots; slot += kTileWaves)
+        if (t.id[slot] != 0) flush.add(tris, t, slot);
+    flush.add_M();
+}
+
 // Pixel pass.  The colour gradient of a pixel is g_out (the identity part)
 // plus its share of the blends of its four pairs, -alpha g_out[p] where it is
 // the target and alpha g_out[tgt] where it is the source.  cg[k] is dL/d(x, y,
 // w) of corner k of the pixel's triangle from the blends whose front pixel it
-// is.  SHADE: the colour gradient goes on through the interpolation, and
-// contrib[p][k] = (its corner terms + cg[k], lambda_k g_color[0..A-1]); g_color
-// is written only where the stray pass reads it (stray_blocks null: there is none).  Without SHADE g_color is
-// written and contrib[p][k] = cg[k], for every pixel with an id.
-template <typename C, typename R, bool SHADE, int NA>
+// is.  OF says what it is the backward of:
+//   kAntialias  the antialiasing alone: g_color is written, and contrib[p][k]
+//               = cg[k] for every pixel with an id;
+//   kShade      the colour gradient goes on through the interpolation, and
+//               contrib[p][k] = (its corner terms + cg[k], lambda_k
+//               g_color[0..A-1]); g_color is written only where the stray pass
+//               reads it;
+//   kRender     the same without a stray pass; the terms of kWide triangles
+//               also go to the gradients here (add_wide).
+enum { kAntialias, kShade, kRender };
+template <typename C, typename R, int OF, int NA>
 __global__ __launch_bounds__(kTileThreads) void aa_bwd_pixel_kernel(const R* __restrict__ color,
                                                                      const C* __restrict__ clip,
                                                                      const R* __restrict__ attr,
@@ -1350,11 +1537,13 @@ __global__ __launch_bounds__(kTileThreads) void aa_bwd_pixel_kernel(const R* __r
                                                                      const float* __restrict__ depth, Dims d, int A,
                                                                      const R* __restrict__ g_out,
                                                                      const unsigned* __restrict__ stray_blocks,
-                                                                     R* __restrict__ g_color, R* __restrict__ contrib)
+                                                                     R* __restrict__ g_color, R* __restrict__ contrib,
+                                                                     WideArgs<C, R> wide)
 {
     __shared__ TileState<R> s;
     constexpr int kStaged = NA ? NA : 1;   // a run-time channel count reads the neighbours from memory
     __shared__ R s_col[kStaged][kTileThreads], s_g[kStaged][kTileThreads];
+    __shared__ WideTile<C, R, NA> s_wide;   // unused, and so not allocated, but for kRender
     const int t = (int)threadIdx.x;
     const TilePixel px = tile_pixel(d);
     const int raw = px.in ? ids[px.p] : 0;
@@ -1413,63 +1602,71 @@ __global__ __launch_bounds__(kTileThreads) void aa_bwd_pixel_kernel(const R* __r
         s.blend[q][t] = v;
     }
     __syncthreads();
-    if (!px.inner) return;
-    R acc[NA ? NA : kMaxAttr];
-    VKGV_CHANNELS(a) acc[a] = g_of(t, px.p, a);
+    R* const o = contrib + px.p * 3 * (3 + A);
+    // the pixel's record; false for a pixel without one
+    auto record = [&]() {
+        R acc[NA ? NA : kMaxAttr];
+        VKGV_CHANNELS(a) acc[a] = g_of(t, px.p, a);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int n = t + dir_thread(q);
-        const R own = s.blend[q][t], nb = s.blend[q ^ 1][n];
-        const bool mine = own == own;
-        if (!mine && !(nb == nb)) continue;
-        const R v = mine ? own : nb, alpha = blend_to_back(v) ? -v : v;
-        const bool target = mine != blend_to_back(v);   // the front pixel of a blend into the front, or the back one's
-        const size_t pn = pixel_at(q);
-        VKGV_CHANNELS(a) acc[a] += target ? -alpha * g_of(t, px.p, a) : alpha * g_of(n, pn, a);
-    }
-    if (!SHADE) {
-        VKGV_CHANNELS(a) g_color[px.p * A + a] = acc[a];
-        if (id > 0)
-            for (int k = 0; k < 9; ++k) contrib[px.p * 9 + k] = cg[k];
-        return;
-    }
-    if (stray_blocks && stray_blocks[px.p / kBlock] != 0u) {
-        VKGV_CHANNELS(a) g_color[px.p * A + a] = acc[a];
-    }
-    if (!ok) return;
-    InterpTerms<C, R> it;
-    bary_from(P, xn, yn, it.b);
-    for (int k = 0; k < 3; ++k) it.b.v[k] = vi[k];
-    {
-        const R xr = ndc_x<R>(px.x, d), yr = ndc_y<R>(px.y, d);
-        R glam[3] = { R(0), R(0), R(0) };
-        VKGV_CHANNELS(a) {
-#pragma unroll
-            for (int k = 0; k < 3; ++k) glam[k] += acc[a] * attr[vi[k] * A + a];
+        for (int q = 0; q < 4; ++q) {
+            const int n = t + dir_thread(q);
+            const R own = s.blend[q][t], nb = s.blend[q ^ 1][n];
+            const bool mine = own == own;
+            if (!mine && !(nb == nb)) continue;
+            const R v = mine ? own : nb, alpha = blend_to_back(v) ? -v : v;
+            const bool target = mine != blend_to_back(v);   // the front pixel of a blend into the front, or the back one's
+            const size_t pn = pixel_at(q);
+            VKGV_CHANNELS(a) acc[a] += target ? -alpha * g_of(t, px.p, a) : alpha * g_of(n, pn, a);
         }
-        interp_terms_of(glam, xr, yr, it);
-    }
-    R* o = contrib + px.p * 3 * (3 + A);
-    if (NA == 3) {   // 18 values as pairs (the record is a whole number of them)
-        R v[18];
+        if (OF == kAntialias) {
+            VKGV_CHANNELS(a) g_color[px.p * A + a] = acc[a];
+            if (id > 0)
+                for (int k = 0; k < 9; ++k) contrib[px.p * 9 + k] = cg[k];
+            return false;
+        }
+        if (OF == kShade && stray_blocks[px.p / kBlock] != 0u) {
+            VKGV_CHANNELS(a) g_color[px.p * A + a] = acc[a];
+        }
+        if (!ok) return false;
+        InterpTerms<C, R> it;
+        bary_from(P, xn, yn, it.b);
+        for (int k = 0; k < 3; ++k) it.b.v[k] = vi[k];
+        {
+            const R xr = ndc_x<R>(px.x, d), yr = ndc_y<R>(px.y, d);
+            R glam[3] = { R(0), R(0), R(0) };
+            VKGV_CHANNELS(a) {
+#pragma unroll
+                for (int k = 0; k < 3; ++k) glam[k] += acc[a] * attr[vi[k] * A + a];
+            }
+            interp_terms_of(glam, xr, yr, it);
+        }
+        if (NA == 3) {   // 18 values as pairs (the record is a whole number of them)
+            R v[18];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                v[6 * k] = it.gu[k].x + cg[3 * k];
+                v[6 * k + 1] = it.gu[k].y + cg[3 * k + 1];
+                v[6 * k + 2] = it.gw[k] + cg[3 * k + 2];
+                VKGV_CHANNELS(a) v[6 * k + 3 + a % 3] = it.b.lam[k] * acc[a];
+            }
+#pragma unroll
+            for (int k = 0; k < 9; ++k) reinterpret_cast<R2<R>*>(o)[k] = R2<R>{ v[2 * k], v[2 * k + 1] };
+            return true;
+        }
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
-            v[6 * k] = it.gu[k].x + cg[3 * k];
-            v[6 * k + 1] = it.gu[k].y + cg[3 * k + 1];
-            v[6 * k + 2] = it.gw[k] + cg[3 * k + 2];
-            VKGV_CHANNELS(a) v[6 * k + 3 + a % 3] = it.b.lam[k] * acc[a];
+            R* ok3 = o + k * (3 + A);
+            ok3[0] = it.gu[k].x + cg[3 * k];
+            ok3[1] = it.gu[k].y + cg[3 * k + 1];
+            ok3[2] = it.gw[k] + cg[3 * k + 2];
+            VKGV_CHANNELS(a) ok3[3 + a] = it.b.lam[k] * acc[a];
         }
-#pragma unroll
-        for (int k = 0; k < 9; ++k) reinterpret_cast<R2<R>*>(o)[k] = R2<R>{ v[2 * k], v[2 * k + 1] };
-        return;
-    }
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        R* ok3 = o + k * (3 + A);
-        ok3[0] = it.gu[k].x + cg[3 * k];
-        ok3[1] = it.gu[k].y + cg[3 * k + 1];
-        ok3[2] = it.gw[k] + cg[3 * k + 2];
-        VKGV_CHANNELS(a) ok3[3 + a] = it.b.lam[k] * acc[a];
+        return true;
+    };
+    const bool has = px.inner && record();
+    if (OF == kRender && *wide.flag != 0u) {   // uniform over the grid
+        const bool on_wide = has && wide.vis[tri_index(d, px.c, id)] == kWide;
+        if (__syncthreads_or(on_wide)) add_wide<C, R, NA>(wide, s_wide, tris, d, A, px.c, on_wide ? id : 0, o);
     }
 }
 
@@ -1673,7 +1870,7 @@ void raster_tris(const float* clip, const int* tris, int C, int I, int V, int T,
     if (C * I && T && nv && npx) {
         snap_kernel<<<blocks(nv), kBlock, 0, st>>>(clip, d, nv, static_cast<Snap*>(snap));
         raster_tris_kernel<<<raster_grid(d), kBlock, 0, st>>>(static_cast<const Snap*>(snap), tris, d, keys, nullptr,
-                                                              cull_back);
+                                                              nullptr, nullptr, cull_back);
     }
     if (npx) keys_to_ids_kernel<<<blocks(npx), kBlock, 0, st>>>(keys, npx, ids, depth);
 }
@@ -1779,29 +1976,29 @@ static void interp_bwd_t(const C* clip, const R* attr, const int* tris, const in
 template <typename C, typename R, int FROM>
 static void aa_fwd_t(R* color, const C* clip, const R* attr, const int* tris, int* ids, float* depth,
                      const unsigned long long* keys, const Dims& d, int A, R* out, const unsigned long long* boxes,
-                     unsigned* stray_blocks, uint8_t* vis, hipStream_t st)
+                     unsigned* stray_blocks, uint8_t* vis, const uint32_t* wide_flag, hipStream_t st)
 {
     if ((size_t)d.C * d.H * d.W == 0) return;
     if (A == 3)
         aa_fwd_kernel<C, R, FROM, 3><<<tile_blocks(d), kTileThreads, 0, st>>>(color, clip, attr, tris, ids, depth, keys,
-                                                                              d, A, out, boxes, stray_blocks, vis);
+                                                                              d, A, out, boxes, stray_blocks, vis, wide_flag);
     else
         aa_fwd_kernel<C, R, FROM, 0><<<tile_blocks(d), kTileThreads, 0, st>>>(color, clip, attr, tris, ids, depth, keys,
-                                                                              d, A, out, boxes, stray_blocks, vis);
+                                                                              d, A, out, boxes, stray_blocks, vis, wide_flag);
 }
 
-template <typename C, typename R, bool SHADE>
+template <typename C, typename R, int OF>
 static void aa_bwd_pixel(const R* color, const C* clip, const R* attr, const int* tris, const int* ids,
                          const float* depth, const Dims& d, int A, const R* g_out, const unsigned* stray_blocks,
-                         R* g_color, R* contrib, hipStream_t st)
+                         R* g_color, R* contrib, const WideArgs<C, R>& wide, hipStream_t st)
 {
     if ((size_t)d.C * d.H * d.W == 0) return;
     if (A == 3)
-        aa_bwd_pixel_kernel<C, R, SHADE, 3><<<tile_blocks(d), kTileThreads, 0, st>>>(
-            color, clip, attr, tris, ids, depth, d, A, g_out, stray_blocks, g_color, contrib);
+        aa_bwd_pixel_kernel<C, R, OF, 3><<<tile_blocks(d), kTileThreads, 0, st>>>(
+            color, clip, attr, tris, ids, depth, d, A, g_out, stray_blocks, g_color, contrib, wide);
     else
-        aa_bwd_pixel_kernel<C, R, SHADE, 0><<<tile_blocks(d), kTileThreads, 0, st>>>(
-            color, clip, attr, tris, ids, depth, d, A, g_out, stray_blocks, g_color, contrib);
+        aa_bwd_pixel_kernel<C, R, OF, 0><<<tile_blocks(d), kTileThreads, 0, st>>>(
+            color, clip, attr, tris, ids, depth, d, A, g_out, stray_blocks, g_color, contrib, wide);
 }
 
 template <typename C, typename R>
@@ -1812,7 +2009,8 @@ static void aa_bwd_t(const R* color, const C* clip, const int* tris, const int* 
 {
     const Dims d{ nc, I, V, T, H, W };
     const size_t npx = (size_t)nc * H * W;
-    aa_bwd_pixel<C, R, false>(color, clip, nullptr, tris, ids, depth, d, A, g_out, stray_blocks, g_color, contrib, st);
+    aa_bwd_pixel<C, R, kAntialias>(color, clip, nullptr, tris, ids, depth, d, A, g_out, stray_blocks, g_color, contrib,
+                                   {}, st);
     vertex_gather<C, R, false>(ids, d, A, adj_off, adj, boxes, contrib, g_clip, static_cast<R*>(nullptr), st);
     if (npx && V)
         aa_bwd_stray_kernel<C, R><<<blocks(npx), kBlock, 0, st>>>(color, clip, tris, ids, depth, d, A, g_out, boxes,
@@ -1831,7 +2029,7 @@ static void shade_bwd_t(const R* color, const C* clip, const R* attr, const int*
     const Dims d{ nc, I, V, T, H, W };
     const size_t npx = (size_t)nc * H * W;
     if (V == 0) return;
-    aa_bwd_pixel<C, R, true>(color, clip, attr, tris, ids, depth, d, A, g_out, stray_blocks, g_color, contrib, st);
+    aa_bwd_pixel<C, R, kShade>(color, clip, attr, tris, ids, depth, d, A, g_out, stray_blocks, g_color, contrib, {}, st);
     vertex_gather<C, R, true>(ids, d, A, adj_off, adj, boxes, contrib, g_clip, part, st);
     attr_reduce_kernel<R><<<blocks((size_t)V * A), kBlock, 0, st>>>(part, nc * I, (size_t)V * A, g_attr);
     if (npx) {
@@ -1842,44 +2040,52 @@ static void shade_bwd_t(const R* color, const C* clip, const R* attr, const int*
     }
 }
 
+// The word of vis that holds the wide flag, behind the bytes.
+static size_t wide_word(const Dims& d) { return ((size_t)d.C * d.I * d.T + 3) / 4; }
+
 // Projection, raster and shading of a mesh, from its own keys.
 template <typename C, typename R>
 static void render_fwd_t(const C* pos, const C* M, const R* attr, const int* tris, const Dims& d, int A, C* clip,
                          void* snap, unsigned long long* keys, unsigned long long* boxes, uint8_t* vis, int* ids,
                          float* depth, R* color, R* out, hipStream_t st)
 {
-    const size_t npx = (size_t)d.C * d.H * d.W, nvis = ((size_t)d.C * d.I * d.T + 3) / 4;
+    const size_t npx = (size_t)d.C * d.H * d.W, nvis = wide_word(d) + 1;
     if (npx == 0) return;
+    uint32_t* flag = reinterpret_cast<uint32_t*>(vis) + wide_word(d);
     // at least one block, which clears the keys, also without vertices
     project_kernel<C><<<dim3(std::max(1u, blocks((size_t)d.V)), std::max(1, d.C * d.I)), kBlock, 0, st>>>(
         pos, M, d, clip, static_cast<Snap*>(snap), keys, npx, reinterpret_cast<uint32_t*>(vis), nvis);
     if (d.C * d.I && d.T && d.V)
-        raster_tris_kernel<<<raster_grid(d), kBlock, 0, st>>>(static_cast<const Snap*>(snap), tris, d, keys, boxes, 0);
-    aa_fwd_t<C, R, kFromKeys>(color, clip, attr, tris, ids, depth, keys, d, A, out, nullptr, nullptr, vis, st);
+        raster_tris_kernel<<<raster_grid(d), kBlock, 0, st>>>(static_cast<const Snap*>(snap), tris, d, keys, boxes, vis,
+                                                              flag, 0);
+    aa_fwd_t<C, R, kFromKeys>(color, clip, attr, tris, ids, depth, keys, d, A, out, nullptr, nullptr, vis, flag, st);
 }
 
 int render_parts(int nc, int I) { return std::max(1, (nc * I + kPairs - 1) / kPairs); }
 
 // part_pos and part_attr: render_parts(nc, I) gradients, reduced into g_pos and
-// g_attr (with one part they are those themselves).
+// g_attr (with one part they are those themselves).  g_M, wide_pos and wide_attr
+// are zero.
 template <typename C, typename R>
 static void render_bwd_t(const C* pos, const C* M, const R* attr, const int* tris, const Dims& d, int A, const C* clip,
                          const unsigned long long* boxes, const uint8_t* vis, const int* ids, const float* depth,
                          const R* color, const int* adj_off, const int* adj, const R* g_out, R* contrib, C* part_pos,
-                         R* part_attr, C* g_pos, C* g_M, R* g_attr, hipStream_t st)
+                         R* part_attr, C* wide_pos, R* wide_attr, C* g_pos, C* g_M, R* g_attr, hipStream_t st)
 {
     if (d.V == 0) return;
     const int parts = render_parts(d.C, d.I);
-    aa_bwd_pixel<C, R, true>(color, clip, attr, tris, ids, depth, d, A, g_out, nullptr, nullptr, contrib, st);
+    const uint32_t* flag = reinterpret_cast<const uint32_t*>(vis) + wide_word(d);
+    aa_bwd_pixel<C, R, kRender>(color, clip, attr, tris, ids, depth, d, A, g_out, nullptr, nullptr, contrib,
+                                { vis, flag, pos, M, wide_pos, g_M, wide_attr }, st);
     const dim3 grid((unsigned)((d.V + kBlockVertices - 1) / kBlockVertices), (unsigned)parts);
     C* pp = parts > 1 ? part_pos : g_pos;
     R* pa = parts > 1 ? part_attr : g_attr;
     if (A == 3)
         vertex_render_kernel<C, R, 3><<<grid, kBlock, 0, st>>>(ids, d, A, pos, M, adj_off, adj, boxes, vis, contrib, pp,
-                                                               pa, g_M);
+                                                               pa, g_M, flag, wide_pos, wide_attr);
     else
         vertex_render_kernel<C, R, 0><<<grid, kBlock, 0, st>>>(ids, d, A, pos, M, adj_off, adj, boxes, vis, contrib, pp,
-                                                               pa, g_M);
+                                                               pa, g_M, flag, wide_pos, wide_attr);
     if (parts > 1) {
         const size_t np = (size_t)d.V * 3, na = (size_t)d.V * A;
         part_reduce_kernel<C, R><<<blocks(np + na), kBlock, 0, st>>>(part_pos, np, g_pos, part_attr, na, g_attr, parts);
@@ -1940,7 +2146,7 @@ void transform_bwd(const double* g_clip, const double* pos, const double* A, int
         const Dims d{ nc, I, V, T, H, W };                                                                             \
         aa_fwd_t<C, R, kFromColor>(const_cast<R*>(color), clip, nullptr, tris, const_cast<int*>(ids),                  \
                                    const_cast<float*>(depth), nullptr, d, A, out, boxes, stray_blocks,                 \
-                                   vis_of(boxes, nc, I, T), st);                                                       \
+                                   vis_of(boxes, nc, I, T), nullptr, st);                                                       \
     }                                                                                                                  \
     void shade_fwd(const C* clip, const R* attr, const int* tris, const int* ids, const float* depth, int nc, int I,   \
                    int V, int T, int H, int W, int A, R* color, R* out, unsigned long long* boxes,                     \
@@ -1948,7 +2154,7 @@ void transform_bwd(const double* g_clip, const double* pos, const double* A, int
     {                                                                                                                  \
         const Dims d{ nc, I, V, T, H, W };                                                                             \
         aa_fwd_t<C, R, kFromIds>(color, clip, attr, tris, const_cast<int*>(ids), const_cast<float*>(depth), nullptr,   \
-                                 d, A, out, boxes, stray_blocks, vis_of(boxes, nc, I, T), st);                         \
+                                 d, A, out, boxes, stray_blocks, vis_of(boxes, nc, I, T), nullptr, st);                \
     }                                                                                                                  \
     void render_fwd(const C* pos, const C* M, const R* attr, const int* tris, int nc, int I, int V, int T, int H,      \
                     int W, int A, C* clip, void* snap, unsigned long long* keys, unsigned long long* boxes,            \
@@ -1960,11 +2166,12 @@ void transform_bwd(const double* g_clip, const double* pos, const double* A, int
     void render_bwd(const C* pos, const C* M, const R* attr, const int* tris, int nc, int I, int V, int T, int H,      \
                     int W, int A, const C* clip, const unsigned long long* boxes, const uint8_t* vis, const int* ids,  \
                     const float* depth, const R* color, const int* adj_off, const int* adj, const R* g_out,            \
-                    R* contrib, C* part_pos, R* part_attr, C* g_pos, C* g_M, R* g_attr, hipStream_t st)                \
+                    R* contrib, C* part_pos, R* part_attr, C* wide_pos, R* wide_attr, C* g_pos, C* g_M, R* g_attr,     \
+                    hipStream_t st)                                                                                    \
     {                                                                                                                  \
         const Dims d{ nc, I, V, T, H, W };                                                                             \
         render_bwd_t<C, R>(pos, M, attr, tris, d, A, clip, boxes, vis, ids, depth, color, adj_off, adj, g_out,         \
-                           contrib, part_pos, part_attr, g_pos, g_M, g_attr, st);                                      \
+                           contrib, part_pos, part_attr, wide_pos, wide_attr, g_pos, g_M, g_attr, st);                 \
     }                                                                                                                  \
     void aa_bwd(const R* color, const C* clip, const int* tris, const int* ids, const float* depth, int nc, int I,     \
                 int V, int T, int H, int W, int A, const unsigned long long* boxes, const unsigned* stray_blocks,      \

@@ -436,7 +436,14 @@ struct RenderFn : public torch::autograd::Function<RenderFn> {
         const Shape s{ (int)M.size(0), (int)M.size(1), (int)pos.size(0), (int)tris.size(0), (int)ids.size(1),
                        (int)ids.size(2), (int)attr.size(1) };
         Tensor g_out = grads[0].to(attr.scalar_type()).contiguous();
-        Tensor g_pos = torch::empty_like(pos), g_M = torch::zeros_like(M), g_attr = torch::empty_like(attr);
+        Tensor g_pos = torch::empty_like(pos), g_attr = torch::empty_like(attr);
+        // The gradients that are added to, cleared by one launch: g_M, then those of
+        // wide triangles, which are scratch.  g_M is the storage's first part (a view
+        // would cost a small step's host 1.5 us).
+        const int64_t nm = M.numel(), np3 = pos.numel();
+        const int64_t na = (attr.numel() * attr.element_size() + pos.element_size() - 1) / pos.element_size();
+        Tensor g_M = torch::zeros({ nm + np3 + na }, M.options());
+        g_M.unsafeGetTensorImpl()->set_sizes_contiguous(M.sizes());
         const int64_t npx = (int64_t)s.C * s.H * s.W, parts = vkgv_diff::render_parts(s.C, s.I);
         Tensor contrib = torch::empty({ std::max<int64_t>(npx * 3 * (3 + s.A), 1) }, attr.options());
         const int64_t scratch = parts > 1 ? parts * s.V : 0;
@@ -451,7 +458,9 @@ struct RenderFn : public torch::autograd::Function<RenderFn> {
                                   ids.data_ptr<int>(), depth.data_ptr<float>(), color.data_ptr<R>(),
                                   adj.first.data_ptr<int>(), adj.second.data_ptr<int>(), g_out.data_ptr<R>(),
                                   contrib.data_ptr<R>(), part_pos.data_ptr<C>(), part_attr.data_ptr<R>(),
-                                  g_pos.data_ptr<C>(), g_M.data_ptr<C>(), g_attr.data_ptr<R>(), stream());
+                                  g_M.data_ptr<C>() + nm, reinterpret_cast<R*>(g_M.data_ptr<C>() + nm + np3),
+                                  g_pos.data_ptr<C>(),
+                                  g_M.data_ptr<C>(), g_attr.data_ptr<R>(), stream());
         });
         return { g_pos, g_M, g_attr, Tensor(), Tensor(), Tensor() };
     }
