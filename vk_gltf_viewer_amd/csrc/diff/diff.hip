@@ -100,11 +100,11 @@ __device__ __forceinline__ Box unpack_box(unsigned long long v)
 // pixel centres, 64-bit atomicMin of (depth, id).  Triangles with a vertex at
 // w <= 0 are skipped (the cameras of this form see the mesh from outside).
 //
-// The vertices are projected and snapped once each (Snap, 16 bytes), not once
-// for each of the about six triangles that share one: the triangle pass then
-// has no division until a triangle's box holds a pixel centre, and its
-// coordinates are 32-bit (below 2^28), its edge functions 64-bit.  A box of more than kWaveBox pixels is walked by
-// the whole wave.  Bound by the vector ALU (36.9M instructions) and the
+// render projects and snaps the vertices once each (Snap, 16 bytes), not once
+// for each of the about six triangles that share one: its triangle pass has no
+// division until a triangle's box holds a pixel centre.  Coordinates are 32-bit
+// (below 2^28), edge functions 64-bit.  A box of more than kWaveBox pixels is
+// walked by the whole wave.  Bound by the vector ALU (36.9M instructions) and the
 // atomics of every front and back fragment: 6.5M triangles of about half a
 // pixel in 8 views of 512x512 take 130 us; with a projection per triangle
 // corner 147 us, besides the pass that rounded the clip positions to float.
@@ -154,14 +154,6 @@ __global__ __launch_bounds__(kBlock) void project_kernel(const C* __restrict__ p
     snap[ci * d.V + v] = snap_vertex(make_float4((float)o.x, (float)o.y, (float)o.z, (float)o.w), d);
 }
 
-// Snapped vertices of given clip positions.
-__global__ __launch_bounds__(kBlock) void snap_kernel(const float* __restrict__ clip, Dims d, size_t n,
-                                                       Snap* __restrict__ snap)
-{
-    const size_t g = (size_t)blockIdx.x * kBlock + threadIdx.x;
-    if (g < n) snap[g] = snap_vertex(reinterpret_cast<const float4*>(clip)[g], d);
-}
-
 // A triangle ready to be walked over its box of pixels: edge functions at the
 // first centre minus the top-left bias (a centre is covered iff all are >= 0),
 // the depth plane from vertex 0.
@@ -174,15 +166,22 @@ struct TriWalk {
     uint32_t id;
     float size;         // area in pixels
 
-    // Visibility-buffer key of pixel (i, j) of the box; all ones where the
-    // centre is not covered.
+    // Edge function k at pixel (i, j) of the box.
+    __device__ __forceinline__ long long edge_at(int k, int i, int j) const
+    {
+        return e[k] + (((long long)j * ex[k] - (long long)i * ey[k]) << 8);
+    }
+    // Visibility-buffer key of pixel (i, j), covered or not; all ones where the
+    // depth is out of range.
+    __device__ __forceinline__ unsigned long long depth_key(int i, int j) const
+    {
+        const float z = z0 + (za * ((float)(ox + 256 * i) * 0.00390625f) + zb * ((float)(oy + 256 * j) * 0.00390625f));
+        return z >= 0.0f && z <= 1.0f ? make_key(z, id) : ~0ull;
+    }
+    // The same, all ones also where the centre is not covered.
     __device__ __forceinline__ unsigned long long key_at(int i, int j) const
     {
-        long long c = 0;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) c |= e[k] + (((long long)j * ex[k] - (long long)i * ey[k]) << 8);
-        const float z = z0 + (za * ((float)(ox + 256 * i) * 0.00390625f) + zb * ((float)(oy + 256 * j) * 0.00390625f));
-        return c >= 0 && z >= 0.0f && z <= 1.0f ? make_key(z, id) : ~0ull;
+        return (edge_at(0, i, j) | edge_at(1, i, j) | edge_at(2, i, j)) >= 0 ? depth_key(i, j) : ~0ull;
     }
 };
 
@@ -211,20 +210,27 @@ enum : uint8_t { kHidden = 0, kSeen = 1, kWide = 2 };
 
 // boxes (null with vis and wide, for a raster alone): the pixel box of each
 // triangle with a fragment.
-__global__ __launch_bounds__(kBlock) void raster_tris_kernel(const Snap* __restrict__ snap, const int* __restrict__ tris,
+// V: Snap, or float4 for clip positions, projected and snapped here for each
+// corner (three times the divisions, but no pass over the vertices before).
+__device__ __forceinline__ Snap snapped(const Snap& v, const Dims&) { return v; }
+__device__ __forceinline__ Snap snapped(const float4& v, const Dims& d) { return snap_vertex(v, d); }
+template <typename V>
+__global__ __launch_bounds__(kBlock) void raster_tris_kernel(const V* __restrict__ vtx, const int* __restrict__ tris,
                                                               Dims d, unsigned long long* __restrict__ keys,
                                                               unsigned long long* __restrict__ boxes,
                                                               uint8_t* __restrict__ vis, uint32_t* __restrict__ wide_flag,
-                                                              int cull_back)
+                                                              int per_wave, int cull_back)
 {
-    const int t = (int)(blockIdx.x * kBlock + threadIdx.x), lane = (int)(threadIdx.x & 63u);
+    const int lane = (int)(threadIdx.x & 63u), wave = (int)(blockIdx.x * (kBlock / 64u) + (threadIdx.x >> 6));
+    const int t = lane < per_wave ? wave * per_wave + lane : d.T;
     for (int ci = (int)blockIdx.y; ci < d.C * d.I; ci += (int)gridDim.y) {
-        const Snap* sv = snap + (size_t)ci * d.V;
+        const V* sv = vtx + (size_t)ci * d.V;
         unsigned long long* img = keys + (size_t)(ci / d.I) * d.H * d.W;
         TriWalk w;
         bool live = false;
         if (t < d.T) {
-            const Snap a = sv[tris[3 * t]], b = sv[tris[3 * t + 1]], c = sv[tris[3 * t + 2]];
+            const Snap a = snapped(sv[tris[3 * t]], d), b = snapped(sv[tris[3 * t + 1]], d),
+                       c = snapped(sv[tris[3 * t + 2]], d);
             w.px0 = max((min(a.x, min(b.x, c.x)) + 127) >> 8, 0);
             w.px1 = min((max(a.x, max(b.x, c.x)) - 128) >> 8, d.W - 1);
             w.py0 = max((min(a.y, min(b.y, c.y)) + 127) >> 8, 0);
@@ -279,7 +285,10 @@ __global__ __launch_bounds__(kBlock) void raster_tris_kernel(const Snap* __restr
                 }
             }
         }
-        // one wide triangle at a time, a pixel per lane
+        // one wide triangle at a time in blocks of 8x8 pixels, a pixel per lane,
+        // the edge functions stepped from block to block (with a division and six
+        // products a pixel instead, 10240 triangles with boxes around 60x60 took 360
+        // us, not 288)
         unsigned long long pending = __ballot(wide);
         while (pending != 0ull) {
             const int j = __ffsll((long long)pending) - 1;
@@ -291,14 +300,26 @@ __global__ __launch_bounds__(kBlock) void raster_tris_kernel(const Snap* __restr
             uint32_t* to = reinterpret_cast<uint32_t*>(&u);
 #pragma unroll
             for (int k = 0; k < kWords; ++k) to[k] = (uint32_t)__builtin_amdgcn_readlane((int)from[k], j);
-            const int bw = u.px1 - u.px0 + 1, n = bw * (u.py1 - u.py0 + 1);
+            const int lx = lane & 7, ly = lane >> 3, bw = u.px1 - u.px0 + 1, bh = u.py1 - u.py0 + 1;
+            unsigned long long* at = img + (size_t)u.py0 * d.W + u.px0;
+            long long row[3] = { u.edge_at(0, lx, ly), u.edge_at(1, lx, ly), u.edge_at(2, lx, ly) };
             bool any = false;
-            for (int q = lane; q < n; q += 64) {
-                const int j2 = q / bw, i2 = q - j2 * bw;
-                const unsigned long long key = u.key_at(i2, j2);
-                if (key == ~0ull) continue;
-                key_min(img + (size_t)(u.py0 + j2) * d.W + u.px0 + i2, key);
-                any = true;
+            for (int by = 0; by < bh; by += 8) {
+                long long v[3] = { row[0], row[1], row[2] };
+                for (int bx = 0; bx < bw; bx += 8) {
+                    const int i = bx + lx, jj = by + ly;
+                    if (i < bw && jj < bh && (v[0] | v[1] | v[2]) >= 0) {
+                        const unsigned long long key = u.depth_key(i, jj);
+                        if (key != ~0ull) {
+                            key_min(at + (size_t)jj * d.W + i, key);
+                            any = true;
+                        }
+                    }
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) v[k] -= (long long)u.ey[k] * 2048;
+                }
+#pragma unroll
+                for (int k = 0; k < 3; ++k) row[k] += (long long)u.ex[k] * 2048;
             }
             if (__ballot(any) != 0ull && lane == j) drawn = true;
         }
@@ -1860,18 +1881,35 @@ inline unsigned blocks(size_t n) { return (unsigned)((n + kBlock - 1) / kBlock);
 } // namespace
 
 // ---------------------------------------------------------------------------
-static dim3 raster_grid(const Dims& d) { return dim3(blocks((size_t)d.T), std::min(d.C * d.I, 65535)); }
+// Triangles a wave of the raster takes: 64, or fewer where 64 leave the chip
+// idle (below kRasterWaves / 2 waves), so that triangles with large boxes, which a
+// wave walks one after another, are spread over it: 10240 triangles with boxes
+// around 60x60 288 -> 67 us, 92160 around 20x20 130 -> 112, 2000 around a vertex
+// in each of 4 views of 512x512 2300 -> 128.  With fewer than kSpreadPixels pixels a
+// triangle hardly a box is large, and the smaller waves cost 2 us (1280 triangles
+// at 64x64 8 -> 10).
+constexpr size_t kRasterWaves = 4096, kSpreadPixels = 4;
+static int raster_per_wave(const Dims& d)
+{
+    int per = 64;
+    if ((size_t)d.H * d.W > kSpreadPixels * d.T)
+        while (per > 1 && (size_t)d.C * d.I * d.T / per < kRasterWaves / 2) per /= 2;
+    return per;
+}
+static dim3 raster_grid(const Dims& d)
+{
+    const size_t per_block = (size_t)raster_per_wave(d) * (kBlock / 64u);
+    return dim3((unsigned)(((size_t)d.T + per_block - 1) / per_block), std::min(d.C * d.I, 65535));
+}
 
-void raster_tris(const float* clip, const int* tris, int C, int I, int V, int T, int H, int W, int cull_back, void* snap,
+void raster_tris(const float* clip, const int* tris, int C, int I, int V, int T, int H, int W, int cull_back,
                  unsigned long long* keys, int* ids, float* depth, hipStream_t st)
 {
     const Dims d{ C, I, V, T, H, W };
-    const size_t npx = (size_t)C * H * W, nv = (size_t)C * I * V;
-    if (C * I && T && nv && npx) {
-        snap_kernel<<<blocks(nv), kBlock, 0, st>>>(clip, d, nv, static_cast<Snap*>(snap));
-        raster_tris_kernel<<<raster_grid(d), kBlock, 0, st>>>(static_cast<const Snap*>(snap), tris, d, keys, nullptr,
-                                                              nullptr, nullptr, cull_back);
-    }
+    const size_t npx = (size_t)C * H * W;
+    if (C * I && T && V && npx)
+        raster_tris_kernel<<<raster_grid(d), kBlock, 0, st>>>(reinterpret_cast<const float4*>(clip), tris, d, keys, nullptr,
+                                                              nullptr, nullptr, raster_per_wave(d), cull_back);
     if (npx) keys_to_ids_kernel<<<blocks(npx), kBlock, 0, st>>>(keys, npx, ids, depth);
 }
 
@@ -2057,7 +2095,7 @@ static void render_fwd_t(const C* pos, const C* M, const R* attr, const int* tri
         pos, M, d, clip, static_cast<Snap*>(snap), keys, npx, reinterpret_cast<uint32_t*>(vis), nvis);
     if (d.C * d.I && d.T && d.V)
         raster_tris_kernel<<<raster_grid(d), kBlock, 0, st>>>(static_cast<const Snap*>(snap), tris, d, keys, boxes, vis,
-                                                              flag, 0);
+                                                              flag, raster_per_wave(d), 0);
     aa_fwd_t<C, R, kFromKeys>(color, clip, attr, tris, ids, depth, keys, d, A, out, nullptr, nullptr, vis, flag, st);
 }
 

@@ -6,9 +6,8 @@
 
 namespace vkgv_diff {
 
-// keys: C*H*W u64 set to all ones by the caller; ids / depth: C*H*W; snap:
-// scratch of 16 bytes per clip position.
-void raster_tris(const float* clip, const int* tris, int C, int I, int V, int T, int H, int W, int cull_back, void* snap,
+// keys: C*H*W u64 set to all ones by the caller; ids / depth: C*H*W.
+void raster_tris(const float* clip, const int* tris, int C, int I, int V, int T, int H, int W, int cull_back,
                  unsigned long long* keys, int* ids, float* depth, hipStream_t st);
 // Vertex transform: clip [CI, V, 4] = A [CI, 4, 4] (pos [V, 3], 1), and its
 // backward: g_pos [V, 3] (written) and g_A [CI, 4, 4] (accumulated into,

@@ -374,9 +374,8 @@ std::vector<Tensor> rasterize(Tensor clip, Tensor tris, int64_t H, int64_t W, bo
     Tensor keys = torch::full({ C, H, W }, -1, opt.dtype(torch::kInt64));
     Tensor ids = torch::empty({ C, H, W }, opt.dtype(torch::kInt32));
     Tensor depth = torch::empty({ C, H, W }, opt);
-    Tensor snap = torch::empty_like(clip);   // 16 bytes per vertex, as the clip positions
     vkgv_diff::raster_tris(clip.data_ptr<float>(), tris.data_ptr<int>(), C, (int)clip.size(1), (int)clip.size(2),
-                           (int)tris.size(0), (int)H, (int)W, cull_back ? 1 : 0, snap.data_ptr<float>(),
+                           (int)tris.size(0), (int)H, (int)W, cull_back ? 1 : 0,
                            reinterpret_cast<unsigned long long*>(keys.data_ptr<int64_t>()), ids.data_ptr<int>(),
                            depth.data_ptr<float>(), stream());
     return { ids, depth };
