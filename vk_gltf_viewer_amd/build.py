@@ -21,7 +21,7 @@ INCLUDE = os.path.join(ROOT, "include")
 
 HIP_SOURCES = ["api.hip", "cull.hip", "raster.hip", "hiz.hip", "resolve.hip", "grad.hip", "anim.hip", "calib.hip",
                "readback.hip"]
-HIP_HEADERS = ["internal.hpp", "device_math.hpp"]
+HIP_HEADERS = ["internal.hpp", "device_math.hpp", "band.hpp"]
 
 # -ffp-contract=off: the kernels fix their floating-point evaluation order.
 # -packed-fp32-ops: no packed FP32 instructions are generated.

@@ -44,6 +44,7 @@
 //                 into keys held in registers, then merging them into the
 //                 visibility buffer.
 #include "internal.hpp"
+#include "band.hpp"
 
 namespace vkgv {
 namespace {
@@ -1290,17 +1291,15 @@ __device__ __forceinline__ void tile_item(const BigArgs& a, uint32_t tile, uint3
             in_band = by1 >= yb && by0 < yb + kBandRows;
             dx0 = (float)(xb * 256 + 128 - s.x0) * 0.00390625f;
             dy0 = (float)(yb * 256 + 128 - s.y0) * 0.00390625f;
-            int out = 0;   // negative: one edge is negative all over the band
+            bool out = false;   // one edge is negative all over the band
 #pragma unroll
             for (int q = 0; q < 3; ++q) {
-                const long long h = (s.e0[q] - (long long)(xb - bx0) * (long long)s.ey[q] * 256
-                                     + (long long)(yb - by0) * (long long)s.ex[q] * 256) >> 8;
-                const long long lim = 1ll << 29;
-                start[q] = (int)(h < -lim ? -lim : h > lim ? lim : h);
-                narrow = narrow && abs(s.ex[q]) < (1 << 22) && abs(s.ey[q]) < (1 << 22);
-                out |= start[q] + max(0, -(int)(kBinTile - 1u) * s.ey[q]) + max(0, (kBandRows - 1) * s.ex[q]);
+                const BandEdge be = band_edge(s.e0[q], s.ex[q], s.ey[q], xb - bx0, yb - by0, (int)kBinTile, kBandRows);
+                start[q] = be.start;
+                narrow = narrow && be.narrow;
+                out = out || be.out;
             }
-            if (narrow && out < 0) in_band = false;
+            if (narrow && out) in_band = false;
         }
         auto word = [](int v, int j) { return __builtin_amdgcn_readlane(v, j); };
         auto wordf = [](float v, int j) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j)); };
