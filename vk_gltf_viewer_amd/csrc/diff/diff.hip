@@ -52,7 +52,9 @@ __device__ __forceinline__ unsigned long long make_key(float z, uint32_t id)
 template <typename T> struct V2 {
     T x, y;
 };
-template <typename T> struct alignas(4 * sizeof(T) > 16 ? 16 : 4 * sizeof(T)) V4 {
+// A caller's clip position: aligned as its elements are (a contiguous tensor may
+// start anywhere in its storage); loaded 16 bytes at a time all the same.
+template <typename T> struct V4 {
     T x, y, z, w;
 };
 // A pair moved by one load or store.
@@ -117,7 +119,7 @@ struct alignas(16) Snap {
 };
 constexpr int kWaveBox = 64;
 
-__device__ __forceinline__ Snap snap_vertex(float4 p, const Dims& d)
+__device__ __forceinline__ Snap snap_vertex(const V4<float>& p, const Dims& d)
 {
     const float hw = (float)d.W * 0.5f, hh = (float)d.H * 0.5f;
     Snap s{ 0, 0, 0.0f, 0 };
@@ -151,7 +153,7 @@ __global__ __launch_bounds__(kBlock) void project_kernel(const C* __restrict__ p
     V4<C> o;
     transform_vertex(M + ci * 16, pos + 3 * (size_t)v, o);
     reinterpret_cast<V4<C>*>(clip)[ci * d.V + v] = o;
-    snap[ci * d.V + v] = snap_vertex(make_float4((float)o.x, (float)o.y, (float)o.z, (float)o.w), d);
+    snap[ci * d.V + v] = snap_vertex(V4<float>{ (float)o.x, (float)o.y, (float)o.z, (float)o.w }, d);
 }
 
 // A triangle ready to be walked over its box of pixels: edge functions at the
@@ -210,10 +212,10 @@ enum : uint8_t { kHidden = 0, kSeen = 1, kWide = 2 };
 
 // boxes (null with vis and wide, for a raster alone): the pixel box of each
 // triangle with a fragment.
-// V: Snap, or float4 for clip positions, projected and snapped here for each
+// V: Snap, or V4<float> for clip positions, projected and snapped here for each
 // corner (three times the divisions, but no pass over the vertices before).
 __device__ __forceinline__ Snap snapped(const Snap& v, const Dims&) { return v; }
-__device__ __forceinline__ Snap snapped(const float4& v, const Dims& d) { return snap_vertex(v, d); }
+__device__ __forceinline__ Snap snapped(const V4<float>& v, const Dims& d) { return snap_vertex(v, d); }
 template <typename V>
 __global__ __launch_bounds__(kBlock) void raster_tris_kernel(const V* __restrict__ vtx, const int* __restrict__ tris,
                                                               Dims d, unsigned long long* __restrict__ keys,
@@ -1908,7 +1910,7 @@ void raster_tris(const float* clip, const int* tris, int C, int I, int V, int T,
     const Dims d{ C, I, V, T, H, W };
     const size_t npx = (size_t)C * H * W;
     if (C * I && T && V && npx)
-        raster_tris_kernel<<<raster_grid(d), kBlock, 0, st>>>(reinterpret_cast<const float4*>(clip), tris, d, keys, nullptr,
+        raster_tris_kernel<<<raster_grid(d), kBlock, 0, st>>>(reinterpret_cast<const V4<float>*>(clip), tris, d, keys, nullptr,
                                                               nullptr, nullptr, raster_per_wave(d), cull_back);
     if (npx) keys_to_ids_kernel<<<blocks(npx), kBlock, 0, st>>>(keys, npx, ids, depth);
 }
