@@ -505,7 +505,8 @@ int vkgv_view_aa_image(vkgv_ctx* ctx, vkgv_view* view, const vkgv_camera* camera
  * more than 3840 x 2160 pixels fail with VKGV_ERROR_LIMIT. */
 int vkgv_view_aa_image_noalloc(vkgv_ctx* ctx, vkgv_view* view, const vkgv_camera* camera, float* image, void* stream);
 /* g_transforms (double [transform_count][16], column-major like
- * vkgv_set_transforms) += d(sum g_image . image) / d transforms, for
+ * vkgv_set_transforms; memory of the context's device, added to with atomics of
+ * device scope) += d(sum g_image . image) / d transforms, for
  * g_image float [H][W][3].  transform_count must be at least the count last
  * given to vkgv_set_transforms.  The rasterization has no gradient. */
 int vkgv_view_aa_backward(vkgv_ctx* ctx, vkgv_view* view, const vkgv_camera* camera, const float* g_image,

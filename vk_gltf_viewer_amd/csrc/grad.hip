@@ -390,14 +390,14 @@ __global__ __launch_bounds__(kGradBlock) void aa_backward_kernel(GradArgs a, con
                 const int tr = s_tr[i];
                 if (tr < 0) continue;
                 if (tr != cur) {
-                    if (cur >= 0) unsafeAtomicAdd(&g_transforms[16ull * (uint32_t)cur + j], acc);
+                    if (cur >= 0) atomicAdd(&g_transforms[16ull * (uint32_t)cur + j], acc);
                     cur = tr;
                     acc = 0.0;
                 }
                 const double p0 = col < 3 ? s_v[4 + col][i] : 1.0, p1 = col < 3 ? s_v[11 + col][i] : 1.0;
                 acc += s_v[r][i] * p0 + s_v[7 + r][i] * p1;
             }
-            if (cur >= 0) unsafeAtomicAdd(&g_transforms[16ull * (uint32_t)cur + j], acc);
+            if (cur >= 0) atomicAdd(&g_transforms[16ull * (uint32_t)cur + j], acc);
         }
         __syncthreads();   // the records are overwritten by the next round
     }
