@@ -499,10 +499,10 @@ int  vkgv_autotune_batch(vkgv_ctx* ctx, vkgv_batch* batch, const vkgv_frame_desc
  * pixels of different colour blended along the front triangle's crossed
  * edge (see csrc/grad.hip). */
 int vkgv_view_aa_image(vkgv_ctx* ctx, vkgv_view* view, const vkgv_camera* camera, float* image, void* stream);
-/* vkgv_view_aa_image without any device allocation: no counterpart in the
- * reference; for callers that cannot allocate (code under graph capture,
- * serving loops).  The same kernel and the same image, bit for bit.  Views of
- * more than 3840 x 2160 pixels fail with VKGV_ERROR_LIMIT. */
+/* vkgv_view_aa_image for callers that cannot allocate (code under graph
+ * capture, serving loops): no counterpart in the reference.  The same call
+ * (vkgv_view_aa_image allocates nothing either); views of more than 3840 x 2160
+ * pixels fail with VKGV_ERROR_LIMIT, as they always have here. */
 int vkgv_view_aa_image_noalloc(vkgv_ctx* ctx, vkgv_view* view, const vkgv_camera* camera, float* image, void* stream);
 /* g_transforms (double [transform_count][16], column-major like
  * vkgv_set_transforms; memory of the context's device, added to with atomics of

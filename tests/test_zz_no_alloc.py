@@ -1,8 +1,7 @@
-"""vkgv_view_aa_image_noalloc against vkgv_view_aa_image through the C ABI:
-the same antialiased image, bit for bit, on two calls in a row (the second on
-a smaller view, so the fixed scratch keeps the larger call's contents beyond
-the smaller view's pixels), and views above the scratch's 3840 x 2160 pixels
-refused with VKGV_ERROR_LIMIT."""
+"""vkgv_view_aa_image_noalloc against vkgv_view_aa_image through the C ABI: the
+same antialiased image, bit for bit, on two calls in a row (one launch serves
+both entry points; test_gpu_noalloc.py compares it with the FP64 reference),
+and views of more than 3840 x 2160 pixels refused with VKGV_ERROR_LIMIT."""
 import numpy as np
 import pytest
 

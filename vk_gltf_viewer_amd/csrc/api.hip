@@ -27,7 +27,8 @@ namespace vkgv {
 uint32_t hiz_tile_levels(const PyramidDesc& pd);
 }
 
-// Largest view of vkgv_view_aa_image_noalloc (4K UHD).
+// Largest view of vkgv_view_aa_image_noalloc (4K UHD): a limit of its interface,
+// nothing here needs it.
 constexpr size_t kNoAllocPixels = 3840u * 2160u;
 
 namespace {
@@ -1408,6 +1409,7 @@ int vkgv_view_aa_image(vkgv_ctx* c, vkgv_view* v, const vkgv_camera* cam, float*
 {
     int rc = check_grad(c, v, cam, image, image);
     if (rc) return rc;
+    HIP_TRY(c, hipSetDevice(c->device));
     hipStream_t st = stream ? static_cast<hipStream_t>(stream) : c->stream;
     if (v->last_stream && v->last_stream != st) HIP_TRY(c, hipStreamSynchronize(v->last_stream));
     launch_aa_image(scene_dev(c), v->dev.keys, v->dev.width, v->dev.height, cam->view_projection, image, st);
@@ -1423,12 +1425,7 @@ int vkgv_view_aa_image_noalloc(vkgv_ctx* c, vkgv_view* v, const vkgv_camera* cam
     if (npx > kNoAllocPixels)
         return fail(c, VKGV_ERROR_LIMIT, "aa_image_noalloc: the view has " + std::to_string(npx)
                                              + " pixels, more than the limit of " + std::to_string(kNoAllocPixels));
-    HIP_TRY(c, hipSetDevice(c->device));
-    hipStream_t st = stream ? static_cast<hipStream_t>(stream) : c->stream;
-    if (v->last_stream && v->last_stream != st) HIP_TRY(c, hipStreamSynchronize(v->last_stream));
-    launch_aa_image(scene_dev(c), v->dev.keys, v->dev.width, v->dev.height, cam->view_projection, image, st);
-    HIP_TRY(c, hipGetLastError());
-    return VKGV_OK;
+    return vkgv_view_aa_image(c, v, cam, image, stream);
 }
 
 int vkgv_view_aa_backward(vkgv_ctx* c, vkgv_view* v, const vkgv_camera* cam, const float* g_image,
