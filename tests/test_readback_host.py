@@ -17,14 +17,14 @@ FAKE = r"""
 #include <string.h>
 typedef struct { uint32_t x, y, z; } dim3;
 unsigned host_flags = 0;
-int allocs = 0, frees = 0, copies = 0, launches = 0, busy = 0, news = 0;
+int allocs = 0, frees = 0, copies = 0, launches = 0, busy = 0, news = 0, late = 0;
 void* _Znwm(size_t n) { ++news; return malloc(n ? n : 1); }   /* operator new */
 int hipHostMalloc(void** p, size_t n, unsigned flags) { ++allocs; host_flags = flags; return posix_memalign(p, 4096, n) ? 2 : 0; }
 int hipHostFree(void* p) { ++frees; free(p); return 0; }
 int hipPointerGetAttributes(void* a, const void* p) { (void)a; (void)p; return 1; }
 int hipGetLastError(void) { return 0; }
-int hipMemcpyAsync(void* d, const void* s, size_t n, int kind, void* st) { (void)kind; (void)st; ++copies; memcpy(d, s, n); return 0; }
-int hipStreamSynchronize(void* st) { (void)st; return 0; }
+int hipMemcpyAsync(void* d, const void* s, size_t n, int kind, void* st) { (void)kind; (void)st; ++copies; late += busy; memcpy(d, s, n); return 0; }
+int hipStreamSynchronize(void* st) { (void)st; busy = 0; return 0; }
 int hipStreamQuery(void* st) { (void)st; return busy ? 600 : 0; }
 int __hipPushCallConfiguration(dim3 g, dim3 b, size_t sh, void* st) { (void)g; (void)b; (void)sh; (void)st; return 0; }
 int __hipPopCallConfiguration(dim3* g, dim3* b, size_t* sh, void** st)
@@ -100,11 +100,23 @@ def test_small_reads_are_staged_only_behind_work(fake):
     """On an idle stream a plain copy is faster below 896 KB."""
     child(fake, """
         user(True)
-        for n, busy, launches in ((65536, 0, 0), (917500, 0, 0), (917504, 0, 1), (65536, 1, 1), (65532, 1, 0)):
+        for n, busy, launches in ((262144, 0, 0), (917500, 0, 0), (917504, 0, 1), (262144, 1, 1), (262140, 1, 0)):
             setv("busy", busy)
             before = count("launches")
             read(n)
             assert count("launches") - before == launches, (n, busy)
+        user(False)
+    """)
+
+
+def test_a_plain_copy_is_not_queued_behind_work(fake):
+    """The runtime is slow at that; the stream is waited for first."""
+    child(fake, """
+        user(True)
+        for n in (4, 4096, 65536, 262140):
+            setv("busy", 1)
+            read(n)
+        assert count("copies") == 4 and count("late") == 0
         user(False)
     """)
 
@@ -124,8 +136,8 @@ def test_a_read_allocates_nothing_that_could_throw(fake):
 def test_any_size_arrives_whole(fake):
     child(fake, """
         user(True)
-        setv("busy", 1)
-        for n in (1, 4, 65532, 65536, 65540, 2**20 - 4, 2**20, 2**21, 2**21 + 4, 2**22 + 16388, 9 * 2**20):
+        for n in (1, 4, 65540, 262140, 262144, 262148, 2**20 - 4, 2**20, 2**21, 2**21 + 4, 2**22 + 16388, 9 * 2**20):
+            setv("busy", 1)
             read(n)
         before = count("launches")
         read(2**21 + 2)          # not whole words: the plain copy

@@ -413,7 +413,7 @@ hipError_t launch_check_meshes(const MeshCheck* meshes, uint32_t mesh_count, uin
 // (readback.hip); reads of kReadStaged bytes behind unfinished work, and of
 // kReadStagedIdle always, go through a pinned stage.  read_back_user(true /
 // false): a context that may read joins / leaves.
-constexpr size_t kReadStaged = 64u << 10;
+constexpr size_t kReadStaged = 256u << 10;
 constexpr size_t kReadStagedIdle = 896u << 10;
 hipError_t read_back(void* dst, const void* src, size_t bytes, hipStream_t st);
 void read_back_user(bool joins);

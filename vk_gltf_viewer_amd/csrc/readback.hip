@@ -15,10 +15,11 @@
 // The kernel's launch and its pieces cost some 7 us more than a small plain copy
 // does on an idle stream: 64 KB 20 us against 12, 512 KB 36 against 30, equal at
 // 896 KB (47), 1 MB 50 against 61.  Behind a frame that is still running the
-// launch is hidden and the plain copy starts late: a 160x120 frame with its
-// 75 KB of colour 88 us against 97, 480x270 with 506 KB 104 against 116.  So a
-// read of kReadStaged bytes is staged while the stream is busy, one of
-// kReadStagedIdle always.
+// launch is hidden: a 480x270 frame with its 506 KB of colour 94 us against 96,
+// 560x400 with 875 KB 104 against 110, equal up to 300 KB.  So a read of
+// kReadStaged bytes is staged while the stream is busy, one of kReadStagedIdle
+// always.  A plain copy waits for the stream first: queued behind a frame it takes
+// the runtime 15 us more (a 96x64 frame with its colour 95 us, not 80).
 #include <algorithm>
 #include <array>
 #include <atomic>
@@ -167,7 +168,8 @@ hipError_t read_back(void* dst, const void* src, size_t bytes, hipStream_t st)
     const bool words = bytes % 4 == 0 && reinterpret_cast<uintptr_t>(src) % 16 == 0;
     const bool large = bytes >= kReadStagedIdle || (bytes >= kReadStaged && busy(st));
     if (!large || !words || !pageable(dst) || !take_stage(s)) {
-        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
+        hipError_t e = hipStreamSynchronize(st);
+        if (e == hipSuccess) e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
         return e == hipSuccess ? hipStreamSynchronize(st) : e;
     }
     const size_t n = (bytes + kHalfBytes - 1) / kHalfBytes;   // halves to go through
