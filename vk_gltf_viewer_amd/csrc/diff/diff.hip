@@ -1887,16 +1887,17 @@ inline unsigned blocks(size_t n) { return (unsigned)((n + kBlock - 1) / kBlock);
 // idle (below kRasterWaves / 2 waves), so that triangles with large boxes, which a
 // wave walks one after another, are spread over it: 10240 triangles with boxes
 // around 60x60 288 -> 67 us, 92160 around 20x20 130 -> 112, 2000 around a vertex
-// in each of 4 views of 512x512 2300 -> 128.  With fewer than kSpreadPixels pixels a
-// triangle hardly a box is large, and the smaller waves cost 2 us (1280 triangles
-// at 64x64 8 -> 10).
-constexpr size_t kRasterWaves = 4096, kSpreadPixels = 4;
+// in each of 4 views of 512x512 2300 -> 128.  Below kSpreadPixels pixels a triangle
+// hardly a box is large, and the smaller waves cost 2 to 4 us (1280 triangles at
+// 100x70); a quarter of it still halves them, for the slivers of a fan (2000
+// around a vertex in each of 4 views of 96x96 161 -> 98 us).
+constexpr size_t kRasterWaves = 4096, kSpreadPixels = 16;
 static int raster_per_wave(const Dims& d)
 {
-    int per = 64;
-    if ((size_t)d.H * d.W > kSpreadPixels * d.T)
-        while (per > 1 && (size_t)d.C * d.I * d.T / per < kRasterWaves / 2) per /= 2;
-    return per;
+    const size_t px = (size_t)d.H * d.W, least = px > kSpreadPixels * d.T ? 1 : px > kSpreadPixels / 4 * d.T ? 32 : 64;
+    size_t per = 64;
+    while (per > least && (size_t)d.C * d.I * d.T / per < kRasterWaves / 2) per /= 2;
+    return (int)per;
 }
 static dim3 raster_grid(const Dims& d)
 {
