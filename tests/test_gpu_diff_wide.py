@@ -84,3 +84,21 @@ def test_time_of_a_fan():
     one, apart = best(_render), best(_separate)
     print(f"render {1e3 * one:.2f} ms, the separate functions {1e3 * apart:.2f} ms", flush=True)
     assert one <= apart
+
+
+@pytest.mark.parametrize("vertices,channels,dtype", [(0, 3, torch.float64), (1, 1, torch.float32), (3, 3, torch.float64),
+                                                     (257, 8, torch.float32)])
+def test_gradients_hold_their_own_storage(vertices, channels, dtype):
+    """A gradient that is kept or saved is its own elements and no scratch, and
+    starts from zero whatever the allocator's memory held before."""
+    pos = torch.rand(vertices, 3, device="cuda", dtype=dtype)
+    A = torch.eye(4, device="cuda", dtype=dtype).reshape(1, 1, 4, 4).repeat(2, 3, 1, 1)
+    attr = torch.rand(vertices, channels, device="cuda", dtype=torch.float32 if vertices == 3 else dtype)
+    tris = torch.zeros(0, 3, device="cuda", dtype=torch.int32)
+    junk = [torch.full((n,), float("nan"), device="cuda") for n in (64, 192, 512, 4096, 65536)]
+    del junk
+    params = [x.requires_grad_() for x in (pos, A, attr)]
+    img = D.ext().render(*params, tris, 8, 8)[0]
+    for x, g in zip(params, torch.autograd.grad(img, params, torch.ones_like(img))):
+        assert g.shape == x.shape and g.dtype == x.dtype and not g.any()
+        assert g.untyped_storage().nbytes() == g.numel() * g.element_size()

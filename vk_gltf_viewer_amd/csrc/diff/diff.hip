@@ -2104,15 +2104,33 @@ static void render_fwd_t(const C* pos, const C* M, const R* attr, const int* tri
 
 int render_parts(int nc, int I) { return std::max(1, (nc * I + kPairs - 1) / kPairs); }
 
+static size_t pad16(size_t bytes) { return (bytes + 15) / 16 * 16; }
+size_t render_wide_bytes(int V, int A, size_t c, size_t r) { return pad16((size_t)V * 3 * c) + pad16((size_t)V * A * r); }
+
+// Clears what render's backward adds to, in one launch: g_M and, behind it, the
+// sums of the kWide triangles.
+static __global__ __launch_bounds__(kBlock) void clear_sums_kernel(uint4* __restrict__ a, size_t na,
+                                                                    uint4* __restrict__ b, size_t nb)
+{
+    const size_t j = (size_t)blockIdx.x * kBlock + threadIdx.x;
+    if (j < na) a[j] = uint4{ 0u, 0u, 0u, 0u };
+    else if (j < na + nb) b[j - na] = uint4{ 0u, 0u, 0u, 0u };
+}
+
 // part_pos and part_attr: render_parts(nc, I) gradients, reduced into g_pos and
-// g_attr (with one part they are those themselves).  g_M, wide_pos and wide_attr
-// are zero.
+// g_attr (with one part they are those themselves).
 template <typename C, typename R>
 static void render_bwd_t(const C* pos, const C* M, const R* attr, const int* tris, const Dims& d, int A, const C* clip,
                          const unsigned long long* boxes, const uint8_t* vis, const int* ids, const float* depth,
                          const R* color, const int* adj_off, const int* adj, const R* g_out, R* contrib, C* part_pos,
-                         R* part_attr, C* wide_pos, R* wide_attr, C* g_pos, C* g_M, R* g_attr, hipStream_t st)
+                         R* part_attr, void* wide, C* g_pos, C* g_M, R* g_attr, hipStream_t st)
 {
+    C* wide_pos = static_cast<C*>(wide);
+    R* wide_attr = reinterpret_cast<R*>(static_cast<char*>(wide) + pad16((size_t)d.V * 3 * sizeof(C)));
+    const size_t m4 = (size_t)d.C * d.I * 16 * sizeof(C) / 16, w4 = render_wide_bytes(d.V, A, sizeof(C), sizeof(R)) / 16;
+    if (m4 + w4)
+        clear_sums_kernel<<<blocks(m4 + w4), kBlock, 0, st>>>(reinterpret_cast<uint4*>(g_M), m4,
+                                                              static_cast<uint4*>(wide), w4);
     if (d.V == 0) return;
     const int parts = render_parts(d.C, d.I);
     const uint32_t* flag = reinterpret_cast<const uint32_t*>(vis) + wide_word(d);
@@ -2207,12 +2225,11 @@ void transform_bwd(const double* g_clip, const double* pos, const double* A, int
     void render_bwd(const C* pos, const C* M, const R* attr, const int* tris, int nc, int I, int V, int T, int H,      \
                     int W, int A, const C* clip, const unsigned long long* boxes, const uint8_t* vis, const int* ids,  \
                     const float* depth, const R* color, const int* adj_off, const int* adj, const R* g_out,            \
-                    R* contrib, C* part_pos, R* part_attr, C* wide_pos, R* wide_attr, C* g_pos, C* g_M, R* g_attr,     \
-                    hipStream_t st)                                                                                    \
+                    R* contrib, C* part_pos, R* part_attr, void* wide, C* g_pos, C* g_M, R* g_attr, hipStream_t st)        \
     {                                                                                                                  \
         const Dims d{ nc, I, V, T, H, W };                                                                             \
         render_bwd_t<C, R>(pos, M, attr, tris, d, A, clip, boxes, vis, ids, depth, color, adj_off, adj, g_out,         \
-                           contrib, part_pos, part_attr, wide_pos, wide_attr, g_pos, g_M, g_attr, st);                 \
+                           contrib, part_pos, part_attr, wide, g_pos, g_M, g_attr, st);                                \
     }                                                                                                                  \
     void aa_bwd(const R* color, const C* clip, const int* tris, const int* ids, const float* depth, int nc, int I,     \
                 int V, int T, int H, int W, int A, const unsigned long long* boxes, const unsigned* stray_blocks,      \

@@ -54,10 +54,10 @@ size_t stray_flag_count(int nc, int H, int W);
 // entries; contrib as for shade_bwd; part_pos [render_parts][V][3] and
 // part_attr [render_parts][V][A].  Kept for the backward: clip, boxes (one
 // entry per camera, instance and triangle, written for those with a fragment),
-// vis (as many bytes, rounded up to 4, and a word), ids, depth, color.  g_M,
-// wide_pos [V][3] and wide_attr [V][A] are accumulated into, zeroed by the
-// caller; the last two are scratch.
+// vis (as many bytes, rounded up to 4, and a word), ids, depth, color.  wide is
+// scratch of render_wide_bytes, 16-byte aligned like g_M.
 int render_parts(int nc, int I);
+size_t render_wide_bytes(int V, int A, size_t c, size_t r);   // c, r: bytes of a C and an R
 #define VKGV_DIFF_DECLARE(C, R)                                                                                       \
     void interp_fwd(const C* clip, const R* attr, const int* tris, const int* ids, int nc, int I, int V, int T, int H, \
                     int W, int A, R* out, unsigned long long* boxes, unsigned* stray_blocks, hipStream_t st);          \
@@ -76,8 +76,7 @@ int render_parts(int nc, int I);
     void render_bwd(const C* pos, const C* M, const R* attr, const int* tris, int nc, int I, int V, int T, int H,      \
                     int W, int A, const C* clip, const unsigned long long* boxes, const uint8_t* vis, const int* ids,  \
                     const float* depth, const R* color, const int* adj_off, const int* adj, const R* g_out,            \
-                    R* contrib, C* part_pos, R* part_attr, C* wide_pos, R* wide_attr, C* g_pos, C* g_M, R* g_attr,     \
-                    hipStream_t st);                                                                                   \
+                    R* contrib, C* part_pos, R* part_attr, void* wide, C* g_pos, C* g_M, R* g_attr, hipStream_t st);       \
     void aa_bwd(const R* color, const C* clip, const int* tris, const int* ids, const float* depth, int nc, int I,     \
                 int V, int T, int H, int W, int A, const unsigned long long* boxes, const unsigned* stray_blocks,      \
                 const int* adj_off, const int* adj, const R* g_out, R* contrib, R* g_color, C* g_clip,                 \

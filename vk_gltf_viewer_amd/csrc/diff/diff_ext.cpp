@@ -436,13 +436,9 @@ struct RenderFn : public torch::autograd::Function<RenderFn> {
                        (int)ids.size(2), (int)attr.size(1) };
         Tensor g_out = grads[0].to(attr.scalar_type()).contiguous();
         Tensor g_pos = torch::empty_like(pos), g_attr = torch::empty_like(attr);
-        // The gradients that are added to, cleared by one launch: g_M, then those of
-        // wide triangles, which are scratch.  g_M is the storage's first part (a view
-        // would cost a small step's host 1.5 us).
-        const int64_t nm = M.numel(), np3 = pos.numel();
-        const int64_t na = (attr.numel() * attr.element_size() + pos.element_size() - 1) / pos.element_size();
-        Tensor g_M = torch::zeros({ nm + np3 + na }, M.options());
-        g_M.unsafeGetTensorImpl()->set_sizes_contiguous(M.sizes());
+        Tensor g_M = torch::empty(M.sizes(), M.options());
+        const size_t nwide = vkgv_diff::render_wide_bytes(s.V, s.A, pos.element_size(), attr.element_size());
+        Tensor wide = torch::empty({ (int64_t)nwide }, pos.options().dtype(torch::kUInt8));
         const int64_t npx = (int64_t)s.C * s.H * s.W, parts = vkgv_diff::render_parts(s.C, s.I);
         Tensor contrib = torch::empty({ std::max<int64_t>(npx * 3 * (3 + s.A), 1) }, attr.options());
         const int64_t scratch = parts > 1 ? parts * s.V : 0;
@@ -457,9 +453,8 @@ struct RenderFn : public torch::autograd::Function<RenderFn> {
                                   ids.data_ptr<int>(), depth.data_ptr<float>(), color.data_ptr<R>(),
                                   adj.first.data_ptr<int>(), adj.second.data_ptr<int>(), g_out.data_ptr<R>(),
                                   contrib.data_ptr<R>(), part_pos.data_ptr<C>(), part_attr.data_ptr<R>(),
-                                  g_M.data_ptr<C>() + nm, reinterpret_cast<R*>(g_M.data_ptr<C>() + nm + np3),
-                                  g_pos.data_ptr<C>(),
-                                  g_M.data_ptr<C>(), g_attr.data_ptr<R>(), stream());
+                                  wide.data_ptr<uint8_t>(), g_pos.data_ptr<C>(), g_M.data_ptr<C>(),
+                                  g_attr.data_ptr<R>(), stream());
         });
         return { g_pos, g_M, g_attr, Tensor(), Tensor(), Tensor() };
     }
