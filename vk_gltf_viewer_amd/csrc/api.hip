@@ -1054,7 +1054,7 @@ int vkgv_set_hierarchy(vkgv_ctx* c, const vkgv_node* nodes, uint32_t node_count,
     uint32_t kept = 0;
     for (uint32_t g = 0; g < 6; ++g) {
         const uint32_t n = group_end[g] - group_first[g];
-        std::copy(chans.get() + group_first[g], chans.get() + group_end[g], chans.get() + kept);
+        if (n) std::memmove(chans.get() + kept, chans.get() + group_first[g], n * sizeof(AnimChan));   // may be in place
         kept += n;
     }
     // depth-first walk of the roots (World::iterateNode order, as vkgv_world_build):
